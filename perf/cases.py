@@ -105,7 +105,7 @@ def draw(rng: random.Random):
                 "backfill": rng.random() < 0.4}
     if op == "build":
         dim = rng.choice(dims)
-        return {"op": op, "rows": _log(rng, 5000, min(1e6, 3e8 / dim)), "dim": dim,
+        return {"op": op, "rows": _log(rng, 5000, min(250_000, 2e8 / dim)), "dim": dim,
                 "c_max": rng.choice([512, 1024, 2048]), "fanout": 2, "k": rng.choice([10, 32]),
                 "l_max": rng.choice([32, 64]), "unit": rng.random() < 0.5, "backfill": rng.random() < 0.5,
                 "prune": rng.random() < 0.2}

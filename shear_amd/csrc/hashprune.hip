@@ -16,17 +16,12 @@
 // reduction.  Record batches:
 //   1. count records per source (atomics), exclusive scan, scatter the records
 //      grouped by source (the per-source counters return to zero);
-//   2. one wave per source with new records merges its current slots with them
-//      (in registers up to 256 candidates, else in LDS up to kHpMergeCap at a
-//      time): a bitonic sort by (hash, total order: dist key, target) puts
-//      each hash's best first; when more than l_max hashes remain, a sort of
-//      those by the total order gives the l_max-th as a threshold; the
-//      survivors are the new slots.
+//   2. one wave per source with new records merges its slots with them
+//      (hp_merge_kernel).
 // Segment batches (records left where the emitter wrote them, described by
-// per-source runs) are merged by streaming each source's records through its
-// reservoir held in registers (hp_merge_stream_kernel).  Between merges the
-// slots are kept in no particular order; the export sorts each reservoir by
-// hash, the reference's emit order.
+// per-source runs) are merged in place by the same kernel.  Between merges
+// the slots are kept in no particular order; the export sorts each reservoir
+// by hash, the reference's emit order.
 #include <hipcub/hipcub.hpp>
 
 #include "hashprune_kernels.h"
@@ -36,7 +31,7 @@ namespace tessa {
 namespace {
 
 constexpr int kHpWaves = 4;                 // waves per workgroup of the merge kernels
-constexpr uint32_t kHpRegMax = 256;         // largest merge done in registers (4 candidates per lane)
+constexpr uint32_t kHpMergeGrid = 4096;     // workgroups of a merge, each walking its share of the sources
 constexpr int kHpThreads = kHpWaves * 64;
 constexpr int kScanThreads = 1024;
 constexpr int kScanPerThread = 4;
@@ -195,63 +190,12 @@ __global__ void hp_scatter_kernel(const uint4 *rec, uint64_t count, uint32_t num
     }
 }
 
-// Ascending bitonic sort of (key, payload) pairs, lexicographic, over
-// [0, P) (P a power of two >= 64), by one wave on its LDS region.  LDS
-// operations of one wave complete in order, so stages need no barrier.
-template <typename K>
-__device__ void wave_bitonic(K *key, uint32_t *val, uint32_t P, uint32_t lane) {
-    for (uint32_t k = 2; k <= P; k <<= 1) {
-        for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-            for (uint32_t c = lane; c < P / 2; c += 64) {
-                const uint32_t i = ((c & ~(j - 1u)) << 1) | (c & (j - 1u));
-                const uint32_t l = i + j;
-                const bool up = (i & k) == 0;
-                const K a = key[i], b = key[l];
-                const uint32_t va = val[i], vb = val[l];
-                const bool b_less = b < a || (b == a && vb < va);
-                const bool a_less = a < b || (a == b && va < vb);
-                if (up ? b_less : a_less) {
-                    key[i] = b;
-                    key[l] = a;
-                    val[i] = vb;
-                    val[l] = va;
-                }
-            }
-            __builtin_amdgcn_wave_barrier();
-        }
-    }
-}
-
-// Ascending bitonic sort of (hash, key) pairs, hash first, over [0, P).
-__device__ void wave_bitonic_hk(uint32_t *hash, uint64_t *key, uint32_t P, uint32_t lane) {
-    for (uint32_t k = 2; k <= P; k <<= 1) {
-        for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-            for (uint32_t c = lane; c < P / 2; c += 64) {
-                const uint32_t i = ((c & ~(j - 1u)) << 1) | (c & (j - 1u));
-                const uint32_t l = i + j;
-                const bool up = (i & k) == 0;
-                const uint32_t ha = hash[i], hb = hash[l];
-                const uint64_t a = key[i], b = key[l];
-                const bool b_less = hb < ha || (hb == ha && b < a);
-                const bool a_less = ha < hb || (ha == hb && a < b);
-                if (up ? b_less : a_less) {
-                    hash[i] = hb;
-                    hash[l] = ha;
-                    key[i] = b;
-                    key[l] = a;
-                }
-            }
-            __builtin_amdgcn_wave_barrier();
-        }
-    }
-}
-
 // Register bitonic sort of P = 64*E elements, element q*64 + lane in lane
-// `lane`'s slot q, by (hash, key) when kHashFirst, else by (key, hash).
-template <int E, bool kHashFirst>
+// `lane`'s slot q, by (hash, key).
+template <int E>
 __device__ __forceinline__ void reg_bitonic(uint32_t (&h)[E], uint64_t (&k)[E], uint32_t lane) {
     auto less = [](uint32_t ha, uint64_t ka, uint32_t hb, uint64_t kb) {
-        return kHashFirst ? (ha < hb || (ha == hb && ka < kb)) : (ka < kb || (ka == kb && ha < hb));
+        return ha < hb || (ha == hb && ka < kb);
     };
 #pragma unroll
     for (uint32_t kk = 2; kk <= 64u * E; kk <<= 1) {
@@ -290,240 +234,6 @@ __device__ __forceinline__ void reg_bitonic(uint32_t (&h)[E], uint64_t (&k)[E], 
     }
 }
 
-// Of the candidates in h/k (E register slots per lane; an empty entry is
-// h = 0xffffffff, k = ~0, after every real hash <= 0xffff), keeps each hash's
-// best and, of those, the l_max best in total order; leaves them in h/k at
-// positions [0, n) (position q*64 + lane in slot q of lane), ascending in
-// total order, empty entries after them, and returns n.
-template <int E>
-__device__ __forceinline__ uint32_t select_sorted(uint32_t (&h)[E], uint64_t (&k)[E], uint32_t l_max, uint32_t lane) {
-    reg_bitonic<E, true>(h, k, lane);
-    // kept = first of its hash (the predecessor of element 64*q is lane 63 of slot q-1)
-    uint32_t n_kept = 0;
-    bool kept[E];
-#pragma unroll
-    for (int q = 0; q < E; ++q) {
-        uint32_t prev = __shfl_up(h[q], 1);
-        if (q > 0) {
-            const uint32_t last = __shfl(h[q - 1], 63);
-            prev = lane == 0 ? last : prev;
-        }
-        const uint32_t e = (uint32_t)q * 64u + lane;
-        kept[q] = h[q] != 0xffffffffu && (e == 0 || prev != h[q]);
-        n_kept += (uint32_t)__popcll(__ballot(kept[q]));
-    }
-#pragma unroll
-    for (int q = 0; q < E; ++q) {
-        h[q] = kept[q] ? h[q] : 0xffffffffu;
-        k[q] = kept[q] ? k[q] : ~0ull;
-    }
-    reg_bitonic<E, false>(h, k, lane);
-    const uint32_t n = n_kept < l_max ? n_kept : l_max;
-#pragma unroll
-    for (int q = 0; q < E; ++q) {
-        const bool live = (uint32_t)q * 64u + lane < n;
-        h[q] = live ? h[q] : 0xffffffffu;
-        k[q] = live ? k[q] : ~0ull;
-    }
-    return n;
-}
-
-// One merge of a source's n_old slots and n_new records (n_old + n_new <= 64*E)
-// entirely in registers; writes the new slots and returns their count.
-// fetch(q, t) returns new record t (t < n_new) for register slot q.
-template <int E, typename Fetch>
-__device__ uint32_t reg_merge_f(const uint64_t *slot_keys_in, const uint16_t *slot_hash_in, uint32_t n_old,
-                                uint32_t n_new, Fetch &&fetch, uint32_t l_max, uint32_t lane,
-                                uint64_t *slot_keys_out, uint16_t *slot_hash_out) {
-    const uint32_t N = n_old + n_new;
-    uint32_t h[E];
-    uint64_t k[E];
-#pragma unroll
-    for (int q = 0; q < E; ++q) {
-        const uint32_t e = (uint32_t)q * 64u + lane;
-        h[q] = 0xffffffffu;
-        k[q] = ~0ull;
-        if (e < n_old) {
-            k[q] = slot_keys_in[e];
-            h[q] = slot_hash_in[e];
-        } else if (e < N) {
-            const uint4 r = fetch(q, e - n_old);
-            k[q] = ((uint64_t)total_key(__uint_as_float(r.w)) << 32) | r.y;
-            h[q] = r.z & 0xffffu;
-        }
-    }
-    const uint32_t n = select_sorted<E>(h, k, l_max, lane);
-#pragma unroll
-    for (int q = 0; q < E; ++q) {
-        const uint32_t e = (uint32_t)q * 64u + lane;
-        if (e < n) {
-            slot_keys_out[e] = k[q];
-            slot_hash_out[e] = (uint16_t)h[q];
-        }
-    }
-    return n;
-}
-
-// Records contiguous at recs; the first 64 were prefetched into r0 (they line
-// up with register slot q when n_old == 64*q).
-template <int E>
-__device__ uint32_t reg_merge(const uint64_t *slot_keys_in, const uint16_t *slot_hash_in, uint32_t n_old,
-                              const uint4 *recs, uint32_t n_new, const uint4 &r0, uint32_t l_max, uint32_t lane,
-                              uint64_t *slot_keys_out, uint16_t *slot_hash_out) {
-    auto fetch = [&](int q, uint32_t t) -> uint4 { return (n_old == (uint32_t)q * 64u) ? r0 : recs[t]; };
-    return reg_merge_f<E>(slot_keys_in, slot_hash_in, n_old, n_new, fetch, l_max, lane, slot_keys_out,
-                          slot_hash_out);
-}
-
-struct HpWaveLds {
-    uint64_t key[kHpMergeCap];      // candidates: total-order key (dist key << 32 | target)
-    uint32_t val[kHpMergeCap];      // their hashes
-    uint64_t tkey[kHpMergeCap];     // each hash's best, sorted by total order: the merged
-    uint32_t thash[kHpMergeCap];    // reservoir is their first min(count, l_max)
-};
-
-// Sources with at most kHpRegMax candidates (slots + new records): register
-// merges, no LDS, so occupancy is set by registers alone.
-__global__ __launch_bounds__(kHpThreads) void hp_merge_small_kernel(const uint4 *grouped, const uint32_t *offsets,
-                                                                    uint32_t num_points, uint32_t l_max,
-                                                                    uint64_t *slot_keys, uint16_t *slot_hash,
-                                                                    uint32_t *slot_count) {
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t waves = gridDim.x * kHpWaves;
-    // the next source's offsets and first 64 records are loaded one iteration
-    // ahead, so their latency overlaps the current merge
-    uint32_t src = blockIdx.x * kHpWaves + (threadIdx.x >> 6);
-    uint32_t p_off = 0, p_n = 0;
-    uint4 p_rec = make_uint4(0u, 0u, 0u, 0u);
-    if (src < num_points) {
-        p_off = offsets[src];
-        p_n = offsets[src + 1] - p_off;
-        if (lane < p_n) p_rec = grouped[p_off + lane];
-    }
-    for (; src < num_points; src += waves) {
-        const uint32_t off = p_off;
-        const uint32_t n_new = p_n;
-        const uint4 r0 = p_rec;
-        const uint32_t nsrc = src + waves;
-        if (nsrc < num_points) {
-            p_off = offsets[nsrc];
-            p_n = offsets[nsrc + 1] - p_off;
-            if (lane < p_n) p_rec = grouped[p_off + lane];
-        }
-        if (n_new == 0) continue;
-        const uint32_t n_old = slot_count[src];
-        const uint64_t sbase = (uint64_t)src * l_max;
-        uint32_t c;
-        if (n_old + n_new <= 64u)
-            c = reg_merge<1>(slot_keys + sbase, slot_hash + sbase, n_old, grouped + off, n_new, r0, l_max, lane,
-                             slot_keys + sbase, slot_hash + sbase);
-        else if (n_old + n_new <= 128u)
-            c = reg_merge<2>(slot_keys + sbase, slot_hash + sbase, n_old, grouped + off, n_new, r0, l_max, lane,
-                             slot_keys + sbase, slot_hash + sbase);
-        else if (n_old + n_new <= kHpRegMax)
-            c = reg_merge<4>(slot_keys + sbase, slot_hash + sbase, n_old, grouped + off, n_new, r0, l_max, lane,
-                             slot_keys + sbase, slot_hash + sbase);
-        else
-            continue;  // hp_merge_large_kernel
-        if (lane == 0) slot_count[src] = c;
-    }
-}
-
-// Sources with more than kHpRegMax candidates: merged in LDS, kHpMergeCap at a
-// time.
-// One LDS merge round: the wave's reservoir w.key/w.val[0, n_old) and new
-// candidates w.key/w.val[n_old, N) become the merged reservoir in
-// w.tkey/w.thash[0, result), ascending in total order; returns its size.
-__device__ uint32_t lds_merge_round(HpWaveLds &w, uint32_t n_old, uint32_t N, uint32_t l_max, uint32_t lane) {
-    uint32_t P = 64;
-    while (P < N) P <<= 1;
-    for (uint32_t e = N + lane; e < P; e += 64) {
-        w.key[e] = ~0ull;
-        w.val[e] = 0xffffffffu;  // after every real hash (<= 0xffff)
-    }
-    __builtin_amdgcn_wave_barrier();
-    // each hash's best first: sort by (hash, total-order key)
-    wave_bitonic_hk(w.val, w.key, P, lane);
-    const uint32_t E = P / 64;
-    const uint32_t eb = lane * E;
-    // kept = first of its hash, compacted into tkey / thash
-    uint32_t kcount = 0;
-    for (uint32_t q = 0; q < E; ++q) {
-        const uint32_t e = eb + q;
-        kcount += (e < N && (e == 0 || w.val[e - 1] != w.val[e])) ? 1u : 0u;
-    }
-    uint32_t n_kept;
-    uint32_t run = wave_excl_scan(kcount, lane, n_kept);
-    for (uint32_t q = 0; q < E; ++q) {
-        const uint32_t e = eb + q;
-        if (e < N && (e == 0 || w.val[e - 1] != w.val[e])) {
-            w.tkey[run] = w.key[e];
-            w.thash[run] = w.val[e];
-            ++run;
-        }
-    }
-    // the kept by total order; the first l_max of them remain
-    uint32_t P2 = 64;
-    while (P2 < n_kept) P2 <<= 1;
-    for (uint32_t e = n_kept + lane; e < P2; e += 64) {
-        w.tkey[e] = ~0ull;
-        w.thash[e] = 0xffffffffu;
-    }
-    __builtin_amdgcn_wave_barrier();
-    wave_bitonic<uint64_t>(w.tkey, w.thash, P2, lane);
-    __builtin_amdgcn_wave_barrier();
-    return n_kept < l_max ? n_kept : l_max;
-}
-
-// Sources with more than kHpRegMax candidates: merged in LDS, kHpMergeCap at a
-// time.
-__global__ __launch_bounds__(kHpThreads) void hp_merge_large_kernel(const uint4 *grouped, const uint32_t *offsets,
-                                                                    uint32_t num_points, uint32_t l_max,
-                                                                    uint64_t *slot_keys, uint16_t *slot_hash,
-                                                                    uint32_t *slot_count) {
-    __shared__ HpWaveLds lds[kHpWaves];
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t wave = threadIdx.x >> 6;
-    HpWaveLds &w = lds[wave];
-    const uint32_t waves = gridDim.x * kHpWaves;
-    for (uint32_t src = blockIdx.x * kHpWaves + wave; src < num_points; src += waves) {
-        const uint32_t off = offsets[src];
-        const uint32_t n_new = offsets[src + 1] - off;
-        if (n_new == 0) continue;
-        uint32_t n_old = slot_count[src];
-        if (n_old + n_new <= kHpRegMax) continue;  // merged by hp_merge_small_kernel
-        const uint64_t sbase = (uint64_t)src * l_max;
-        for (uint32_t e = lane; e < n_old; e += 64) {
-            w.key[e] = slot_keys[sbase + e];
-            w.val[e] = slot_hash[sbase + e];
-        }
-        uint32_t used = 0;
-        while (used < n_new) {
-            const uint32_t take = (n_new - used < kHpMergeCap - n_old) ? n_new - used : kHpMergeCap - n_old;
-            for (uint32_t e = lane; e < take; e += 64) {
-                const uint4 r = grouped[off + used + e];
-                w.key[n_old + e] = ((uint64_t)total_key(__uint_as_float(r.w)) << 32) | r.y;
-                w.val[n_old + e] = r.z & 0xffffu;
-            }
-            n_old = lds_merge_round(w, n_old, n_old + take, l_max, lane);
-            used += take;
-            if (used < n_new) {
-                for (uint32_t e = lane; e < n_old; e += 64) {
-                    w.key[e] = w.tkey[e];
-                    w.val[e] = w.thash[e];
-                }
-                __builtin_amdgcn_wave_barrier();
-            }
-        }
-        for (uint32_t e = lane; e < n_old; e += 64) {
-            slot_keys[sbase + e] = w.tkey[e];
-            slot_hash[sbase + e] = (uint16_t)w.thash[e];
-        }
-        if (lane == 0) slot_count[src] = n_old;
-        __builtin_amdgcn_wave_barrier();
-    }
-}
-
 // ---- segment mode: records left where the emitter put them ------------------
 // A segment {src, first record lo/hi, count} names a run of records of one
 // source.  The batch's segments are sorted by source (radix sort of the
@@ -551,24 +261,35 @@ __global__ void hp_seg_gather_kernel(const uint4 *segs, const uint32_t *order, u
         sorted[i] = segs[order[i]];
 }
 
-// ---- streaming merge of a source's segments ----------------------------------
-// Every merge leaves a reservoir's slots ascending in total order (the export
-// sorts them by hash, the reference's emit order).  One wave per active source
-// holds the reservoir in registers (slot position q*64 + lane in register q,
-// ER = ceil(l_max / 64) registers) and streams the source's records through
-// it 64 at a time.  A full reservoir's last slot bounds what can still enter:
-// a candidate no better than it either repeats a slot's hash with a worse (or
-// equal) key or is worse than l_max slots of distinct hashes, so it is
-// dropped by one compare.  The candidates that pass are inserted one at a time
-// (the reference's insert: a hash hit keeps the better, a new hash fills a
-// free slot or replaces the worst) by a rank ballot and a one-position shift;
-// a first chunk into an empty reservoir is sorted instead.
+// ---- merge ---------------------------------------------------------------------
+// One wave per source with new records.  A batch of the source's records (64 *
+// kHpNew of them, in registers beside its slots) is reduced at once instead of
+// record by record:
+//   1. a full reservoir drops the candidates past its worst distance;
+//   2. each hash's best is found through a small table in LDS (best_of_hash):
+//      every candidate takes the minimum of its bucket, the one that finds its
+//      own key there claims the bucket and leaves its hash as a tag, and the
+//      others see from the tag whether they lost to their own hash or only
+//      share the bucket with another one (those try again);
+//   3. when more than l_max hashes remain, the l_max best are the ones up to a
+//      distance found by bisection, counting with ballots (keep_best); equal
+//      distances at the border are settled by target, then hash;
+//   4. the survivors are packed through LDS into the slots.
+// What bounds it is latency (the memory pipeline below, then the dependent LDS
+// steps at four waves per SIMD): about 300 vector and 470 scalar instructions
+// and 40 LDS operations for a source with 128 records.  Inserting the
+// candidates one by one (a rank ballot, a hash ballot and a shift each) took
+// 88 SIMD cycles a record: 67 M records of 524,288 points, 2.45 ms then and
+// 0.73 ms now; with the groups of a backfill policy, 29 batches of a 1 M x 768
+// build, 13.8 ms then and 4.9 ms now.  Larger tables (fewer candidates try
+// again) or five waves per SIMD (registers spill: 0.89 ms) cost more.
+constexpr int kHpNew = 4;              // new records per lane in one batch
+constexpr uint32_t kHpBuckets = 1024;  // per wave; >= kHpMaxLMax (staging of the slots), a power of two
 
-constexpr uint32_t kBatchMin = 24;  // passing candidates of a chunk into an empty reservoir that are sorted
+struct HpWaveLds {
+    uint64_t key[kHpBuckets];  // ~0 between uses
+};
 
-__device__ __forceinline__ bool ent_less(uint64_t ka, uint32_t ha, uint64_t kb, uint32_t hb) {
-    return ka < kb || (ka == kb && ha < hb);
-}
 __device__ __forceinline__ uint64_t readlane64(uint64_t v, uint32_t l) {
     return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), (int)l) << 32) |
            (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, (int)l);
@@ -577,267 +298,540 @@ __device__ __forceinline__ uint32_t readlane32(uint32_t v, uint32_t l) {
     return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)l);
 }
 __device__ __forceinline__ uint64_t ballot64(bool pred) { return __builtin_amdgcn_ballot_w64(pred); }
-
-template <int ER>
-struct Reservoir {
-    uint64_t k[ER];  // live positions [0, c) ascending by (k, h); the rest k = ~0, h = 0xffffffff
-    uint32_t h[ER];
-    uint32_t c;
-};
-
-// Key / hash at position pos (the same in every lane).
-template <int ER>
-__device__ __forceinline__ void res_at(const Reservoir<ER> &r, uint32_t pos, uint64_t &k, uint32_t &h) {
-    uint64_t kk = r.k[0];
-    uint32_t hh = r.h[0];
-#pragma unroll
-    for (int q = 1; q < ER; ++q) {
-        kk = pos / 64u == (uint32_t)q ? r.k[q] : kk;
-        hh = pos / 64u == (uint32_t)q ? r.h[q] : hh;
-    }
-    k = readlane64(kk, pos & 63u);
-    h = readlane32(hh, pos & 63u);
+__device__ __forceinline__ bool lane_in(uint64_t mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
+__device__ __forceinline__ uint32_t below(uint64_t mask) {  // set bits of mask under this lane
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+// The lanes of positions [q * 64, q * 64 + 64) below n.
+__device__ __forceinline__ uint64_t lanes_below(uint32_t n, uint32_t q) {
+    const uint32_t m = n > q * 64u ? n - q * 64u : 0u;
+    return m >= 64u ? ~0ull : (1ull << m) - 1ull;
 }
 
-// Positions (p, end] take the entry before them; position p takes (bk, bh).
-template <int ER>
-__device__ __forceinline__ void res_shift_in(Reservoir<ER> &r, uint32_t p, uint32_t end, uint64_t bk, uint32_t bh,
+// The wave's LDS operations complete in order; this keeps the compiler to it.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+template <int kCtrl>
+__device__ __forceinline__ uint32_t dpp_or_zero(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, 0xf, 0xf, true);
+}
+// Largest value of the wave (row shifts by 1, 2, 4, 8, then the row ends carried over).
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+    uint32_t o;
+    o = dpp_or_zero<0x111>(v), v = v > o ? v : o;
+    o = dpp_or_zero<0x112>(v), v = v > o ? v : o;
+    o = dpp_or_zero<0x114>(v), v = v > o ? v : o;
+    o = dpp_or_zero<0x118>(v), v = v > o ? v : o;
+    o = dpp_or_zero<0x142>(v), v = v > o ? v : o;
+    o = dpp_or_zero<0x143>(v), v = v > o ? v : o;
+    return readlane32(v, 63u);
+}
+
+// Sets of candidates are lane masks, one per register (scalar registers, and a
+// register without a candidate of the set costs one scalar branch).
+//
+// Among the candidates `in` (no key of ~0), win = the best key of each hash
+// (one of several equal ones) and, when asked, rest = those of a winner's hash
+// with another target than the winner's.
+template <int R, bool kRest>
+__device__ __forceinline__ void best_of_hash(HpWaveLds &t, const uint64_t (&k)[R], const uint32_t (&h)[R],
+                                             const uint64_t (&in)[R], uint64_t (&win)[R], uint64_t (&rest)[R],
                                              uint32_t lane) {
+    uint64_t pend[R], any = 0;
 #pragma unroll
-    for (int q = ER - 1; q >= 0; --q) {
-        if ((uint32_t)q * 64u > end || (uint32_t)q * 64u + 63u < p) continue;  // register untouched
-        const uint32_t lo = __shfl_up((uint32_t)r.k[q], 1);
-        const uint32_t hi = __shfl_up((uint32_t)(r.k[q] >> 32), 1);
-        uint64_t uk = ((uint64_t)hi << 32) | lo;
-        uint32_t uh = __shfl_up(r.h[q], 1);
-        if (q > 0) {
-            const uint64_t ck = readlane64(r.k[q - 1], 63);
-            const uint32_t ch = readlane32(r.h[q - 1], 63);
-            uk = lane == 0 ? ck : uk;
-            uh = lane == 0 ? ch : uh;
+    for (int q = 0; q < R; ++q) {
+        pend[q] = in[q];
+        win[q] = 0;
+        if (kRest) rest[q] = 0;
+        any |= pend[q];
+    }
+    while (any) {
+        uint64_t best[R], mark[R];
+        // the bucket's best key
+#pragma unroll
+        for (int q = 0; q < R; ++q)
+            if (pend[q] && lane_in(pend[q]))
+                __hip_atomic_fetch_min(&t.key[h[q] & (kHpBuckets - 1u)], k[q], __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_WAVEFRONT);
+        wave_lds_order();
+#pragma unroll
+        for (int q = 0; q < R; ++q)
+            if (pend[q]) best[q] = t.key[h[q] & (kHpBuckets - 1u)];
+        wave_lds_order();
+        // its owner (the last to write, when keys are equal) leaves its hash and position
+#pragma unroll
+        for (int q = 0; q < R; ++q)
+            if (pend[q] && lane_in(pend[q] & ballot64(best[q] == k[q])))
+                t.key[h[q] & (kHpBuckets - 1u)] = ((uint64_t)h[q] << 32) | ((uint32_t)q * 64u + lane);
+        wave_lds_order();
+#pragma unroll
+        for (int q = 0; q < R; ++q)
+            if (pend[q]) mark[q] = t.key[h[q] & (kHpBuckets - 1u)];
+        wave_lds_order();
+        any = 0;
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            if (!pend[q]) continue;
+            const uint64_t own = pend[q] & ballot64((uint32_t)mark[q] == (uint32_t)q * 64u + lane);
+            const uint64_t same = pend[q] & ballot64((uint32_t)(mark[q] >> 32) == h[q]);
+            if (lane_in(own)) t.key[h[q] & (kHpBuckets - 1u)] = ~0ull;
+            win[q] |= own;
+            if (kRest) rest[q] |= same & ~own & ballot64((uint32_t)best[q] != (uint32_t)k[q]);
+            pend[q] &= ~same;
+            any |= pend[q];
         }
-        const uint32_t e = (uint32_t)q * 64u + lane;
-        const bool mv = e > p && e <= end;
-        r.k[q] = e == p ? bk : (mv ? uk : r.k[q]);
-        r.h[q] = e == p ? bh : (mv ? uh : r.h[q]);
+        wave_lds_order();
     }
 }
 
-// Inserts candidate (bk, bh), the same in every lane (r.c, p, hit and the
-// decision are wave-uniform, so they stay scalar).
-template <int ER>
-__device__ __forceinline__ void res_insert(Reservoir<ER> &r, uint64_t bk, uint32_t bh, uint32_t l_max,
-                                           uint32_t lane) {
-    uint32_t p = 0;                // slots before the candidate in total order
-    uint32_t hit = 0xffffffffu;    // the slot of its hash
+// Over the values v of the set m (more than `need` of them): a t with
+// count(v <= t) == need if there is one, else the smallest t with more; cle =
+// count(v <= t).  Each other step interpolates between the counts at the
+// ends (the distances of a reservoir's candidates spread evenly enough for
+// about 4 steps where bisection alone takes 10), the ones between halve.
+template <int R>
+__device__ __forceinline__ uint32_t kth_value(const uint32_t (&v)[R], const uint64_t (&m)[R], uint32_t need,
+                                              uint32_t &cle) {
+    uint32_t mx = 0, mn = 0, n = 0;
 #pragma unroll
-    for (int q = 0; q < ER; ++q) {
-        const bool live = (uint32_t)q * 64u + lane < r.c;
-        p += (uint32_t)__popcll(ballot64(live && ent_less(r.k[q], r.h[q], bk, bh)));
-        const uint64_t m = ballot64(live && r.h[q] == bh);
-        hit = m ? (uint32_t)q * 64u + (uint32_t)__builtin_ctzll(m) : hit;
+    for (int q = 0; q < R; ++q) {
+        const uint32_t a = lane_in(m[q]) ? v[q] : 0u, b = lane_in(m[q]) ? ~v[q] : 0u;
+        mx = mx > a ? mx : a;
+        mn = mn > b ? mn : b;
+        n += (uint32_t)__popcll(m[q]);
     }
-    bool go;
-    uint32_t end;
-    if (hit != 0xffffffffu) {
-        // a hash hit: the candidate replaces the slot when it is better (a
-        // better or equal slot sorts before it, hit < p, or is the same key)
-        uint64_t ek;
-        uint32_t eh;
-        res_at(r, hit, ek, eh);
-        go = hit >= p && ek != bk;
-        end = hit;
-    } else if (r.c < l_max) {
-        go = true;  // a free slot
-        end = r.c;
-        r.c = r.c + 1u;
-    } else {
-        go = p < l_max;  // the worst slot goes unless the candidate is worse than every slot
-        end = l_max - 1u;
+    // count(v <= hi) = c_hi >= need, count(v < lo) = c_lo < need
+    uint32_t hi = wave_max_u32(mx), lo = ~wave_max_u32(mn), c_hi = n, c_lo = 0;
+    bool halve = false;
+    while (lo < hi) {
+        const uint32_t span = hi - lo;
+        uint32_t step = span / 2u;
+        if (!halve) {
+            const float f = (float)(need - c_lo) * __builtin_amdgcn_rcpf((float)(c_hi - c_lo));
+            const uint32_t s = (uint32_t)(f * (float)span);
+            step = (uint32_t)__builtin_amdgcn_readfirstlane((int)(s < span ? s : span - 1u));
+        }
+        halve = !halve;
+        const uint32_t mid = lo + step;
+        uint32_t c = 0;
+#pragma unroll
+        for (int q = 0; q < R; ++q)
+            if (m[q]) c += (uint32_t)__popcll(ballot64(v[q] <= mid) & m[q]);
+        if (c == need) {
+            cle = c;
+            return mid;
+        }
+        if (c > need) {
+            hi = mid;
+            c_hi = c;
+        } else {
+            lo = mid + 1u;
+            c_lo = c;
+        }
     }
-    if (go) res_shift_in(r, p, end, bk, bh, lane);
+    cle = c_hi;
+    return lo;
 }
 
-// Merges one chunk (candidate (ck, ch) in each lane where v) into the reservoir.
-template <int ER>
-__device__ __forceinline__ void res_chunk(Reservoir<ER> &r, uint64_t ck, uint32_t ch, bool v, uint32_t l_max, uint32_t lane) {
-    bool pass = v;
-    if (r.c == l_max) {
-        uint64_t wk;
-        uint32_t wh;
-        res_at(r, l_max - 1u, wk, wh);
-        pass = v && ent_less(ck, ch, wk, wh);
-    }
-    uint64_t pm = ballot64(pass);
-    if (pm == 0) return;
-    if (r.c == 0 && (uint32_t)__popcll(pm) >= kBatchMin) {
-        uint32_t h[1] = {pass ? ch : 0xffffffffu};
-        uint64_t k[1] = {pass ? ck : ~0ull};
-        r.c = (uint32_t)__builtin_amdgcn_readfirstlane((int)select_sorted<1>(h, k, l_max, lane));
-        r.k[0] = k[0];
-        r.h[0] = h[0];
+// Leaves the l_max best of the candidates win (more than l_max of them,
+// distinct hashes) by (distance key, target, hash).
+template <int R>
+__device__ __forceinline__ void keep_best(const uint64_t (&k)[R], const uint32_t (&h)[R], uint64_t (&win)[R],
+                                          uint32_t l_max) {
+    uint32_t d[R], cle;
+#pragma unroll
+    for (int q = 0; q < R; ++q) d[q] = (uint32_t)(k[q] >> 32);
+    const uint32_t td = kth_value<R>(d, win, l_max, cle);
+    if (cle == l_max) {
+#pragma unroll
+        for (int q = 0; q < R; ++q) win[q] &= ballot64(d[q] <= td);
         return;
     }
-    while (pm) {
-        const uint32_t j = (uint32_t)__builtin_ctzll(pm);
-        pm &= pm - 1ull;
-        res_insert(r, readlane64(ck, j), readlane32(ch, j), l_max, lane);
+    // candidates of the distance at the border: by target, then by hash
+    uint64_t sure[R], eq[R];
+    uint32_t need = l_max, tg[R];
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+        sure[q] = win[q] & ballot64(d[q] < td);
+        eq[q] = win[q] & ballot64(d[q] == td);
+        tg[q] = (uint32_t)k[q];
+        need -= (uint32_t)__popcll(sure[q]);
     }
+    const uint32_t tt = kth_value<R>(tg, eq, need, cle);
+    if (cle == need) {
+#pragma unroll
+        for (int q = 0; q < R; ++q) win[q] = sure[q] | (eq[q] & ballot64(tg[q] <= tt));
+        return;
+    }
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+        const uint64_t lt = eq[q] & ballot64(tg[q] < tt);
+        sure[q] |= lt;
+        eq[q] &= ballot64(tg[q] == tt);
+        need -= (uint32_t)__popcll(lt);
+    }
+    const uint32_t th = kth_value<R>(h, eq, need, cle);  // distinct hashes: exact
+#pragma unroll
+    for (int q = 0; q < R; ++q) win[q] = sure[q] | (eq[q] & ballot64(h[q] <= th));
 }
 
-// What a wave loads for one active source before merging it: its segment
-// descriptors (lane s: the run's segment s, for s < 64) and its slots.
-template <int ER>
-struct SourceLoad {
-    uint32_t src, start, len;  // run: sorted segments [start, start + len)
-    uint32_t cnt;              // lane's segment: record count and first record
+// A wave's sources in the stages of its pipeline: the run (source, its sorted
+// segments [start, start + len); num_points: nothing to merge), the segments
+// (lane s: segment s, cnt records from first), then the slots and the first
+// batch of records (the lane's record q * 64 + lane of it, q < kHpNew).  Every
+// load is unconditional, from a clamped address: a branch around a load
+// costs a wait for it at the branch's end.
+struct HpRun {
+    uint32_t src, start, len;
+};
+struct HpSegs {
+    uint32_t ng, cnt;
     uint64_t first;
-    uint32_t c;
+};
+template <int ER>
+struct HpSlots {
     uint64_t k[ER];
-    uint32_t h[ER];
+    uint32_t h[ER], c;
+};
+struct HpBatch {
+    uint32_t dst[kHpNew], hash[kHpNew], dist[kHpNew], total;  // hash: with the record's flags above 16 bits
 };
 
+struct HpMergeArgs {
+    const uint4 *records;   // record batches: grouped by source
+    const uint4 *sorted;    // segments by source; the runs of equal sources
+    const uint32_t *run_src, *run_start, *run_len, *num_runs;
+    const uint32_t *offsets;  // record batches: records [offsets[src], offsets[src + 1])
+    uint32_t num_points, l_max, quota;
+    uint64_t *slot_keys;
+    uint16_t *slot_hash;
+    uint32_t *slot_count;
+    uint64_t *grp_keys;
+};
+
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+
+// Run a of na; raw loads, made a run by hp_run_ready once they have arrived.
+template <bool kGrouped>
+__device__ __forceinline__ HpRun hp_run_load(const HpMergeArgs &A, uint32_t a, uint32_t na) {
+    const uint32_t i = a < na ? a : na - 1u;
+    if (kGrouped) return HpRun{i, A.offsets[i], A.offsets[i + 1u]};
+    return HpRun{A.run_src[i], A.run_start[i], A.run_len[i]};
+}
+template <bool kGrouped>
+__device__ __forceinline__ HpRun hp_run_ready(const HpMergeArgs &A, const HpRun &l, uint32_t a, uint32_t na) {
+    HpRun r{uniform(l.src), uniform(l.start), uniform(l.len)};
+    // past the end, a point without records, the run of empty / bad segments
+    const bool none = a >= na || r.src >= A.num_points || (kGrouped && r.len == r.start);
+    if (none) r = HpRun{A.num_points, 0u, 0u};
+    return r;
+}
+
+// Segments [g0, g0 + 64) of a run; the same two steps.
+template <bool kGrouped>
+__device__ __forceinline__ uint4 hp_segs_load(const HpMergeArgs &A, const HpRun &r, uint32_t g0, uint32_t lane) {
+    if (kGrouped) return make_uint4(r.src, r.start, 0u, r.len - r.start);
+    const uint32_t s = g0 + lane;
+    return A.sorted[(uint64_t)r.start + (s < r.len ? s : 0u)];
+}
+template <bool kGrouped>
+__device__ __forceinline__ HpSegs hp_segs_ready(const HpRun &r, const uint4 &g, uint32_t g0, uint32_t lane) {
+    const uint32_t left = kGrouped ? (r.len ? 1u : 0u) : r.len - g0;
+    HpSegs s;
+    s.ng = left < 64u ? left : 64u;
+    s.cnt = lane < s.ng ? g.w : 0u;
+    s.first = ((uint64_t)g.z << 32) | g.y;
+    return s;
+}
+
 template <int ER>
-__device__ __forceinline__ void load_source(SourceLoad<ER> &L, uint32_t src, uint32_t start, uint32_t len,
-                                            const uint4 *sorted, uint32_t num_points, uint32_t l_max,
-                                            const uint64_t *slot_keys, const uint16_t *slot_hash,
-                                            const uint32_t *slot_count, uint32_t lane) {
-    L.src = src;
-    L.start = start;
-    L.len = len;
-    L.cnt = 0;
-    L.first = 0;
-    L.c = 0;
-    const bool real = src < num_points;  // the run of empty / bad segments sorts last
-    if (real && lane < len) {
-        const uint4 g = sorted[(uint64_t)start + lane];
-        L.cnt = g.w;
-        L.first = ((uint64_t)g.z << 32) | g.y;
-    }
-    const uint64_t sbase = (uint64_t)(real ? src : 0u) * l_max;
-    if (real) L.c = slot_count[src];
+__device__ __forceinline__ HpSlots<ER> hp_slots(const HpMergeArgs &A, uint32_t src, uint32_t lane) {
+    HpSlots<ER> s;
+    const uint32_t p = src < A.num_points ? src : 0u;
+    const uint64_t base = (uint64_t)p * A.l_max;
+    s.c = A.slot_count[p];
 #pragma unroll
     for (int q = 0; q < ER; ++q) {
-        // every slot position is read (not only the live ones), so these loads
-        // do not wait for the count
+        // every slot position is read, not only the live ones: these loads do
+        // not wait for the count
         const uint32_t e = (uint32_t)q * 64u + lane;
-        const bool in = real && e < l_max;
-        L.k[q] = in ? slot_keys[sbase + e] : ~0ull;
-        L.h[q] = in ? (uint32_t)slot_hash[sbase + e] : 0xffffffffu;
+        s.k[q] = A.slot_keys[base + (e < A.l_max ? e : 0u)];
+        s.h[q] = A.slot_hash[base + (e < A.l_max ? e : 0u)];
+    }
+    return s;
+}
+
+// Records [c0, c0 + 64 * kHpNew) of a group of segments, across their
+// boundaries; lanes past the group's records read `safe`.
+__device__ __forceinline__ void hp_batch(HpBatch &b, const uint4 *records, const uint4 *safe, const HpSegs &g,
+                                         uint32_t c0, uint32_t lane) {
+    uint32_t ps = 0;
+    uint64_t at[kHpNew] = {};
+    for (uint32_t s = 0; s < g.ng; ++s) {
+        const uint64_t d = readlane64(g.first, s) - ps;
+#pragma unroll
+        for (int q = 0; q < kHpNew; ++q) at[q] = c0 + (uint32_t)q * 64u + lane >= ps ? d : at[q];
+        ps += readlane32(g.cnt, s);
+    }
+    b.total = ps;
+#pragma unroll
+    for (int q = 0; q < kHpNew; ++q) {
+        const uint32_t p = c0 + (uint32_t)q * 64u + lane;
+        const uint4 *r = p < ps ? records + (at[q] + p) : safe;
+        b.dst[q] = r->y;
+        b.hash[q] = r->z;
+        b.dist[q] = r->w;
     }
 }
 
-// Streams the records of a group of up to 64 segments (lane s: segment s, cnt
-// records from first) 64 at a time across segment boundaries into
-// chunk(key, hash, valid).
-template <typename Chunk>
-__device__ __forceinline__ void stream_group(const uint4 *records, uint32_t ng, uint32_t cnt, uint64_t first,
-                                             uint32_t lane, Chunk &&chunk) {
-    uint32_t total;
-    const uint32_t pre = wave_excl_scan(cnt, lane, total);
-    uint32_t sg = 0;  // first segment not yet wholly read
-    for (uint32_t c0 = 0; c0 < total; c0 += 64) {
-        const uint32_t p = c0 + lane;
-        uint64_t addr = 0;
-        for (uint32_t s = sg; s < ng; ++s) {
-            const uint32_t ps = readlane32(pre, s);
-            if (ps >= c0 + 64u) break;
-            const uint32_t cs = readlane32(cnt, s);
-            const uint64_t fs = readlane64(first, s);
-            addr = (p >= ps && p < ps + cs) ? fs + (p - ps) : addr;
-            if (ps + cs <= c0 + 64u) sg = s + 1;
+// Merges one batch of records into the reservoir (slots rk / rh at positions
+// [0, c), in no particular order; with kRhalf and a free slot, each slot's
+// group g).
+template <int ER, bool kRhalf>
+__device__ __forceinline__ void hp_absorb(HpWaveLds &t, const HpBatch &b, uint32_t c0, uint64_t (&rk)[ER],
+                                          uint32_t (&rh)[ER], uint32_t &c, uint64_t (&g)[ER][kRhalfGroup],
+                                          uint32_t l_max, uint32_t quota, uint32_t lane) {
+    constexpr int S = ER + kHpNew;                               // slots, then new records
+    constexpr int R = S + (kRhalf ? ER * (int)kRhalfGroup : 0);  // then group keys
+    uint64_t k[R], in[R], win[R], rest[R];
+    uint32_t h[R];
+    uint32_t worst = 0xffffffffu;
+    if (c == l_max) {
+        uint32_t m = 0;
+#pragma unroll
+        for (int q = 0; q < ER; ++q) {
+            const uint32_t d = lane_in(lanes_below(c, q)) ? (uint32_t)(rk[q] >> 32) : 0u;
+            m = m > d ? m : d;
         }
-        const bool v = p < total;
-        uint64_t ck = ~0ull;
-        uint32_t ch = 0xffffffffu;
-        if (v) {
-            const uint4 rec = records[addr];
-            ck = ((uint64_t)total_key(__uint_as_float(rec.w)) << 32) | rec.y;
-            ch = rec.z & 0xffffu;
+        worst = wave_max_u32(m);
+    }
+    uint64_t fresh = 0, odd = 0;
+#pragma unroll
+    for (int q = 0; q < kHpNew; ++q) {
+        const uint32_t dk = total_key(__uint_as_float(b.dist[q]));
+        k[ER + q] = ((uint64_t)dk << 32) | b.dst[q];
+        h[ER + q] = b.hash[q] & 0xffffu;
+        in[ER + q] = lanes_below(b.total - c0, q) & ballot64(dk <= worst);
+        fresh |= in[ER + q];
+    }
+    if (!fresh) return;
+#pragma unroll
+    for (int q = 0; q < ER; ++q) {
+        k[q] = rk[q];
+        h[q] = rh[q];
+        in[q] = lanes_below(c, q);
+    }
+    // a key of ~0 (a NaN of all ones) takes no part in the buckets
+#pragma unroll
+    for (int q = 0; q < S; ++q) {
+        const uint64_t o = in[q] & ballot64(k[q] == ~0ull);
+        odd |= o;
+        in[q] &= ~o;
+    }
+    if constexpr (kRhalf) {
+#pragma unroll
+        for (int q = 0; q < ER; ++q)
+#pragma unroll
+            for (uint32_t j = 0; j < kRhalfGroup; ++j) {
+                const int i = S + q * (int)kRhalfGroup + (int)j;
+                k[i] = g[q][j];
+                h[i] = rh[q];
+                in[i] = c < l_max ? lanes_below(c, q) & ballot64(g[q][j] != ~0ull) : 0ull;
+            }
+    }
+    best_of_hash<R, kRhalf>(t, k, h, in, win, rest, lane);
+    if (odd) {
+        // it is the worst of any hash: kept if nothing else of its hash is
+#pragma unroll
+        for (int q = 0; q < S; ++q) {
+            uint64_t m = ballot64(k[q] == ~0ull) &
+                         (q < ER ? lanes_below(c, q) : lanes_below(b.total - c0, q - ER));
+            while (m) {
+                const uint32_t j = (uint32_t)__builtin_ctzll(m);
+                const uint64_t bit = m & (0ull - m);
+                m ^= bit;
+                const uint32_t bh = readlane32(h[q], j);
+                uint64_t held = 0;
+#pragma unroll
+                for (int p = 0; p < S; ++p) held |= win[p] & ballot64(h[p] == bh);
+                if (!held) win[q] |= bit;
+            }
         }
-        chunk(ck, ch, v);
+    }
+    uint32_t n = 0;
+#pragma unroll
+    for (int q = 0; q < S; ++q) n += (uint32_t)__popcll(win[q]);
+    if (n > l_max) {
+        uint64_t ks[S], ws[S];
+        uint32_t hs[S];
+#pragma unroll
+        for (int q = 0; q < S; ++q) ks[q] = k[q], hs[q] = h[q], ws[q] = win[q];
+        keep_best<S>(ks, hs, ws, l_max);
+#pragma unroll
+        for (int q = 0; q < S; ++q) win[q] = ws[q];
+        n = l_max;
+    }
+    // the survivors packed into the slots: keys, then hashes, through LDS
+    uint32_t at = 0, pos[S];
+#pragma unroll
+    for (int q = 0; q < S; ++q) {
+        pos[q] = at + below(win[q]);
+        if (win[q] && lane_in(win[q])) t.key[pos[q]] = k[q];
+        at += (uint32_t)__popcll(win[q]);
+    }
+    c = n;
+    wave_lds_order();
+#pragma unroll
+    for (int q = 0; q < ER; ++q) rk[q] = t.key[(uint32_t)q * 64u + lane];
+    wave_lds_order();
+#pragma unroll
+    for (int q = 0; q < S; ++q)
+        if (win[q] && lane_in(win[q])) t.key[pos[q]] = h[q];
+    wave_lds_order();
+#pragma unroll
+    for (int q = 0; q < ER; ++q) {
+        const bool live = lane_in(lanes_below(c, q));
+        rh[q] = live ? (uint32_t)t.key[(uint32_t)q * 64u + lane] : 0xffffffffu;
+        rk[q] = live ? rk[q] : ~0ull;
+    }
+    wave_lds_order();
+#pragma unroll
+    for (int q = 0; q < ER; ++q) t.key[(uint32_t)q * 64u + lane] = ~0ull;
+    wave_lds_order();
+    if constexpr (kRhalf) {
+        if (c == l_max) return;  // a full reservoir stays full: its groups are never read again
+        // the next best target of each hash, layer by layer
+#pragma unroll
+        for (int q = 0; q < ER; ++q)
+#pragma unroll
+            for (uint32_t j = 0; j < kRhalfGroup; ++j) g[q][j] = ~0ull;
+        for (uint32_t layer = 0; layer < quota; ++layer) {
+            uint64_t any = 0;
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+                in[q] = rest[q];
+                any |= in[q];
+            }
+            if (!any) break;
+            best_of_hash<R, true>(t, k, h, in, win, rest, lane);
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+                uint64_t m = win[q];
+                while (m) {
+                    const uint32_t j = (uint32_t)__builtin_ctzll(m);
+                    m &= m - 1ull;
+                    const uint64_t bk = readlane64(k[q], j);
+                    const uint32_t bh = readlane32(h[q], j);
+#pragma unroll
+                    for (int p = 0; p < ER; ++p)
+#pragma unroll
+                        for (uint32_t i = 0; i < kRhalfGroup; ++i)
+                            g[p][i] = i == layer && rh[p] == bh ? bk : g[p][i];
+                }
+            }
+        }
     }
 }
 
-template <int ER>
-__device__ __forceinline__ void merge_group(Reservoir<ER> &r, const uint4 *records, uint32_t ng, uint32_t cnt,
-                                            uint64_t first, uint32_t l_max, uint32_t lane) {
-    stream_group(records, ng, cnt, first, lane,
-                 [&](uint64_t ck, uint32_t ch, bool v) { res_chunk(r, ck, ch, v, l_max, lane); });
+// All vector loads in flight have arrived.
+__device__ __forceinline__ void wait_loads() {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0) only
+    __builtin_amdgcn_sched_barrier(0);
 }
 
-// Active sources in ascending source order (run-length encoding of the sorted
-// segment keys).  Each wave walks its sources with the next source's
-// segments and slots, and the one after's run, already in flight.
-template <int ER>
-__global__ __launch_bounds__(kHpThreads) void hp_merge_stream_kernel(const uint4 *records, const uint4 *sorted,
-                                                                     const uint32_t *run_src,
-                                                                     const uint32_t *run_start,
-                                                                     const uint32_t *run_len,
-                                                                     const uint32_t *num_runs, uint32_t num_points,
-                                                                     uint32_t l_max, uint64_t *slot_keys,
-                                                                     uint16_t *slot_hash, uint32_t *slot_count) {
+// Each wave walks its sources (segment runs, or with kGrouped the points of a
+// record batch grouped by source) with the next source's first batch and
+// slots, and the one after's run, already in flight.  They are waited for
+// after the merge and before its stores: a wait at their first use, in the
+// next iteration, would also wait for the stores, and for the loads issued
+// there (the branches between leave the compiler no exact count).
+template <int ER, bool kRhalf, bool kGrouped>
+__global__ __launch_bounds__(kHpThreads) void hp_merge_kernel(HpMergeArgs A) {
+    __shared__ HpWaveLds lds[kHpWaves];
     const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t wave = threadIdx.x >> 6;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    HpWaveLds &t = lds[wave];
     const uint32_t waves = gridDim.x * kHpWaves;
-    const uint32_t na = *num_runs;
+    const uint32_t na = kGrouped ? A.num_points : *A.num_runs;
     uint32_t a = blockIdx.x * kHpWaves + wave;
     if (a >= na) return;
-    SourceLoad<ER> cur;
-    load_source(cur, run_src[a], run_start[a], run_len[a], sorted, num_points, l_max, slot_keys, slot_hash,
-                slot_count, lane);
-    uint32_t d_src = num_points, d_start = 0, d_len = 0;  // run of the next source
-    if (a + waves < na) {
-        d_src = run_src[a + waves];
-        d_start = run_start[a + waves];
-        d_len = run_len[a + waves];
-    }
+    for (uint32_t i = lane; i < kHpBuckets; i += 64u) t.key[i] = ~0ull;
+    wave_lds_order();
+    const uint4 *safe = kGrouped ? A.records : A.sorted;
+    // stages: slots and batch of source a, segments of the next, run of the one after
+    HpRun raw = hp_run_load<kGrouped>(A, a, na), raw1 = hp_run_load<kGrouped>(A, a + waves, na),
+          raw2 = hp_run_load<kGrouped>(A, a + 2u * waves, na);
+    HpRun run = hp_run_ready<kGrouped>(A, raw, a, na), run1 = hp_run_ready<kGrouped>(A, raw1, a + waves, na);
+    uint4 seg = hp_segs_load<kGrouped>(A, run, 0u, lane), seg1 = hp_segs_load<kGrouped>(A, run1, 0u, lane);
+    HpSegs segs = hp_segs_ready<kGrouped>(run, seg, 0u, lane);
+    HpSlots<ER> slots = hp_slots<ER>(A, run.src, lane);
+    HpBatch batch;
+    hp_batch(batch, A.records, safe, segs, 0u, lane);
+    wait_loads();
     for (; a < na; a += waves) {
-        SourceLoad<ER> nxt;
-        load_source(nxt, d_src, d_start, d_len, sorted, num_points, l_max, slot_keys, slot_hash, slot_count, lane);
-        const uint32_t a2 = a + 2u * waves;
-        d_src = num_points;
-        d_len = 0;
-        if (a2 < na) {
-            d_src = run_src[a2];
-            d_start = run_start[a2];
-            d_len = run_len[a2];
-        }
-        const uint32_t src = cur.src;
-        if (src < num_points) {
-            Reservoir<ER> r;
-            r.c = (uint32_t)__builtin_amdgcn_readfirstlane((int)cur.c);
-#pragma unroll
-            for (int q = 0; q < ER; ++q) {
-                const bool live = (uint32_t)q * 64u + lane < r.c;
-                r.k[q] = live ? cur.k[q] : ~0ull;
-                r.h[q] = live ? cur.h[q] : 0xffffffffu;
-            }
-            merge_group(r, records, cur.len < 64u ? cur.len : 64u, cur.cnt, cur.first, l_max, lane);
-            for (uint32_t g0 = 64; g0 < cur.len; g0 += 64) {
-                // a source with more than 64 segments in the batch: the rest, 64 at a time
-                const uint32_t ng = cur.len - g0 < 64u ? cur.len - g0 : 64u;
-                uint32_t cnt = 0;
-                uint64_t first = 0;
-                if (lane < ng) {
-                    const uint4 g = sorted[(uint64_t)cur.start + g0 + lane];
-                    cnt = g.w;
-                    first = ((uint64_t)g.z << 32) | g.y;
-                }
-                merge_group(r, records, ng, cnt, first, l_max, lane);
-            }
-            const uint64_t sbase = (uint64_t)src * l_max;
+        HpSegs segs1 = hp_segs_ready<kGrouped>(run1, seg1, 0u, lane);
+        const HpRun run2 = hp_run_ready<kGrouped>(A, raw2, a + 2u * waves, na);
+        const HpSlots<ER> slots1 = hp_slots<ER>(A, run1.src, lane);
+        HpBatch batch1;
+        hp_batch(batch1, A.records, safe, segs1, 0u, lane);
+        seg1 = hp_segs_load<kGrouped>(A, run2, 0u, lane);
+        raw2 = hp_run_load<kGrouped>(A, a + 3u * waves, na);
+        uint64_t base = 0, rk[ER], g[ER][kRhalfGroup];
+        uint32_t rh[ER], c = 0;
+        if (run.src < A.num_points) {
+            c = uniform(slots.c);
+            base = (uint64_t)run.src * A.l_max;
 #pragma unroll
             for (int q = 0; q < ER; ++q) {
                 const uint32_t e = (uint32_t)q * 64u + lane;
-                if (e < r.c) {
-                    slot_keys[sbase + e] = r.k[q];
-                    slot_hash[sbase + e] = (uint16_t)r.h[q];
+                rk[q] = e < c ? slots.k[q] : ~0ull;
+                rh[q] = e < c ? slots.h[q] : 0xffffffffu;
+                if constexpr (kRhalf) {
+#pragma unroll
+                    for (uint32_t j = 0; j < kRhalfGroup; ++j)
+                        g[q][j] = c < A.l_max && e < c ? A.grp_keys[(base + e) * kRhalfGroup + j] : ~0ull;
                 }
             }
-            if (lane == 0) slot_count[src] = r.c;
+            for (uint32_t g0 = 0;;) {
+                for (uint32_t c0 = 0;; c0 += 64u * kHpNew) {
+                    if (g0 != 0u || c0 != 0u) hp_batch(batch, A.records, safe, segs, c0, lane);
+                    hp_absorb<ER, kRhalf>(t, batch, c0, rk, rh, c, g, A.l_max, A.quota, lane);
+                    if (batch.total - c0 <= 64u * kHpNew) break;
+                }
+                // a source with more than 64 segments in the batch: 64 at a time
+                g0 += 64u;
+                if (kGrouped || g0 >= run.len) break;
+                segs = hp_segs_ready<false>(run, hp_segs_load<false>(A, run, g0, lane), g0, lane);
+            }
         }
-        cur = nxt;
+        wait_loads();
+        if (run.src < A.num_points) {
+#pragma unroll
+            for (int q = 0; q < ER; ++q) {
+                const uint32_t e = (uint32_t)q * 64u + lane;
+                if (e < c) {
+                    A.slot_keys[base + e] = rk[q];
+                    A.slot_hash[base + e] = (uint16_t)rh[q];
+                    if constexpr (kRhalf) {
+                        if (c < A.l_max) {
+#pragma unroll
+                            for (uint32_t j = 0; j < kRhalfGroup; ++j)
+                                A.grp_keys[(base + e) * kRhalfGroup + j] = g[q][j];
+                        }
+                    }
+                }
+            }
+            if (lane == 0) A.slot_count[run.src] = c;
+        }
+        run = run1;
+        run1 = run2;
+        segs = segs1;
+        slots = slots1;
+        batch = batch1;
     }
 }
 
@@ -900,7 +894,7 @@ __global__ __launch_bounds__(kHpThreads) void hp_export_kernel(const uint64_t *s
             h[q] = e < c ? (uint32_t)slot_hash[base + e] : 0xffffffffu;
             k[q] = e < c ? slot_keys[base + e] : ~0ull;
         }
-        reg_bitonic<ER, true>(h, k, lane);
+        reg_bitonic<ER>(h, k, lane);
 #pragma unroll
         for (int q = 0; q < ER; ++q) {
             const uint32_t e = (uint32_t)q * 64u + lane;
@@ -935,359 +929,11 @@ __global__ __launch_bounds__(kHpThreads) void hp_export_kernel(const uint64_t *s
 // the reservoir sorts it in total order, the plain insert takes over, and the
 // groups are neither read nor written again.
 
-template <int ER>
-struct GroupReservoir {
-    Reservoir<ER> b;
-    uint64_t g[ER][kRhalfGroup];  // the lane's slot's group, ascending keys, ~0 = none
-};
-
-// The hash's best quota + 1 distinct targets (s[0] the slot key, s[1..] its
-// group, ascending, ~0 = none) with candidate bk added: its target keeps its
-// better key; a new target takes position quota when better than what is
-// there; one backward pass restores the order.
-static_assert(kRhalfGroup == 3, "a group is three keys");
-__device__ __forceinline__ void group_update(uint64_t (&s)[kRhalfGroup + 1], uint64_t bk, uint32_t quota) {
-    const uint32_t bt = (uint32_t)bk;
-    bool present = false;
-#pragma unroll
-    for (uint32_t j = 0; j <= kRhalfGroup; ++j) {
-        const bool m = j <= quota && s[j] != ~0ull && (uint32_t)s[j] == bt;
-        present = present || m;
-        s[j] = m && bk < s[j] ? bk : s[j];
-    }
-#pragma unroll
-    for (uint32_t j = 0; j <= kRhalfGroup; ++j) s[j] = !present && j == quota && bk < s[j] ? bk : s[j];
-#pragma unroll
-    for (int j = kRhalfGroup; j >= 1; --j) {
-        const uint64_t lo = s[j] < s[j - 1] ? s[j] : s[j - 1];
-        const uint64_t hi = s[j] < s[j - 1] ? s[j - 1] : s[j];
-        s[j - 1] = lo;
-        s[j] = hi;
-    }
-}
-
-// Inserts candidate (bk, bh) into a reservoir with a free slot.  While a slot
-// is free the slots are kept in no particular order (nothing is evicted, so no
-// rank is needed): a new hash is appended with an empty group, a repeat of a
-// slot's own (target, distance) (a pair seen forward and reverse) changes
-// nothing, and any other candidate of a slot's hash updates that slot's best
-// quota + 1 distinct targets in the owner lane (the slot key is the best of
-// them, the group the rest).  The first two are selects; only the third
-// branches.
-template <int ER>
-__device__ __forceinline__ void gres_fill_insert(GroupReservoir<ER> &r, uint64_t bk, uint32_t bh, uint32_t quota,
-                                                 uint32_t lane) {
-    uint32_t hit = 0xffffffffu;
-    uint64_t ek = 0;
-#pragma unroll
-    for (int q = 0; q < ER; ++q) {
-        const bool live = (uint32_t)q * 64u + lane < r.b.c;
-        const uint64_t m = ballot64(live && r.b.h[q] == bh);
-        if (m) {
-            const uint32_t l = (uint32_t)__builtin_ctzll(m);
-            hit = (uint32_t)q * 64u + l;
-            ek = readlane64(r.b.k[q], l);
-        }
-    }
-    const bool is_new = hit == 0xffffffffu;
-    const uint32_t e = r.b.c, eq = e >> 6;
-#pragma unroll
-    for (int q = 0; q < ER; ++q) {
-        const bool at = is_new && eq == (uint32_t)q && lane == (e & 63u);
-        r.b.k[q] = at ? bk : r.b.k[q];
-        r.b.h[q] = at ? bh : r.b.h[q];
-#pragma unroll
-        for (uint32_t j = 0; j < kRhalfGroup; ++j) r.g[q][j] = at ? ~0ull : r.g[q][j];
-    }
-    r.b.c = e + (is_new ? 1u : 0u);
-    if (is_new || ek == bk) return;
-    const uint32_t hq = hit >> 6, hl = hit & 63u;
-#pragma unroll
-    for (int q = 0; q < ER; ++q) {
-        if (hq != (uint32_t)q) continue;
-        uint64_t s[kRhalfGroup + 1] = {r.b.k[q], r.g[q][0], r.g[q][1], r.g[q][2]};
-        group_update(s, bk, quota);
-        const bool own = lane == hl;
-        r.b.k[q] = own ? s[0] : r.b.k[q];
-#pragma unroll
-        for (uint32_t j = 0; j < kRhalfGroup; ++j) r.g[q][j] = own ? s[j + 1] : r.g[q][j];
-    }
-}
-
 __device__ __forceinline__ uint64_t shfl_xor64(uint64_t v, int m) {
     const uint32_t lo = __shfl_xor((uint32_t)v, m);
     const uint32_t hi = __shfl_xor((uint32_t)(v >> 32), m);
     return ((uint64_t)hi << 32) | lo;
 }
-__device__ __forceinline__ uint64_t shfl_up64(uint64_t v) {
-    const uint32_t lo = __shfl_up((uint32_t)v, 1);
-    const uint32_t hi = __shfl_up((uint32_t)(v >> 32), 1);
-    return ((uint64_t)hi << 32) | lo;
-}
-__device__ __forceinline__ uint64_t shfl_down64(uint64_t v, uint32_t d) {
-    const uint32_t lo = __shfl_down((uint32_t)v, d);
-    const uint32_t hi = __shfl_down((uint32_t)(v >> 32), d);
-    return ((uint64_t)hi << 32) | lo;
-}
-__device__ __forceinline__ uint64_t permute64(uint32_t dest, uint64_t v) {
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_permute((int)(dest * 4u), (int)(uint32_t)v);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_ds_permute((int)(dest * 4u), (int)(uint32_t)(v >> 32));
-    return ((uint64_t)hi << 32) | lo;
-}
-
-// Ascending bitonic sort of one (a, b) pair per lane across the wave,
-// lexicographic.
-__device__ __forceinline__ void wave_sort_pair(uint64_t &a, uint64_t &b, uint32_t lane) {
-#pragma unroll
-    for (uint32_t kk = 2; kk <= 64u; kk <<= 1) {
-#pragma unroll
-        for (uint32_t j = kk >> 1; j > 0; j >>= 1) {
-            const uint64_t pa = shfl_xor64(a, (int)j), pb = shfl_xor64(b, (int)j);
-            const bool want_min = ((lane & j) == 0) == ((lane & kk) == 0);
-            const bool p_less = pa < a || (pa == a && pb < b);
-            const bool p_more = a < pa || (a == pa && b < pb);
-            const bool take = want_min ? p_less : p_more;
-            a = take ? pa : a;
-            b = take ? pb : b;
-        }
-    }
-}
-
-// A chunk (candidate (ck, ch) in each lane where v) into an empty reservoir,
-// by sorting instead of one insert per candidate: the candidates sorted by
-// (hash, target, key) drop repeats of a (hash, target); sorted by (hash,
-// key), each hash's first is its slot and the next `quota` its group.  With
-// l_max hashes or more the reservoir fills: each hash's best, the l_max best
-// of those, sorted in total order (select_sorted).  Otherwise the slots are
-// moved to positions [0, hashes) (one push permute per word).
-template <int ER>
-__device__ __forceinline__ void gres_batch_fill(GroupReservoir<ER> &r, uint64_t ck, uint32_t ch, bool v, uint32_t l_max,
-                                uint32_t quota, uint32_t lane) {
-    uint64_t a = v ? ((uint64_t)ch << 32) | (uint32_t)ck : ~0ull;  // (hash, target)
-    uint64_t b = v ? (ck >> 32) : ~0ull;                             // distance key
-    wave_sort_pair(a, b, lane);
-    const uint64_t ap = shfl_up64(a);
-    const bool keep = a != ~0ull && (lane == 0 || ap != a);  // a target's best within its hash
-    uint64_t hs = keep ? (a >> 32) : ~0ull;
-    uint64_t k = keep ? ((b << 32) | (uint32_t)a) : ~0ull;
-    wave_sort_pair(hs, k, lane);
-    const uint32_t h = (uint32_t)hs;  // 0xffffffff for the empty entries after the real ones
-    const uint32_t hp = __shfl_up(h, 1);
-    const bool start = h != 0xffffffffu && (lane == 0 || hp != h);
-    const uint64_t S = ballot64(start);
-    const uint32_t m = (uint32_t)__popcll(S);
-    if (m >= l_max) {
-        uint32_t rh[ER];
-        uint64_t rk[ER];
-#pragma unroll
-        for (int q = 0; q < ER; ++q) {
-            rh[q] = q == 0 ? h : 0xffffffffu;
-            rk[q] = q == 0 ? k : ~0ull;
-        }
-        r.b.c = (uint32_t)__builtin_amdgcn_readfirstlane((int)select_sorted<ER>(rh, rk, l_max, lane));
-#pragma unroll
-        for (int q = 0; q < ER; ++q) {
-            r.b.h[q] = rh[q];
-            r.b.k[q] = rk[q];
-        }
-        return;
-    }
-    // rank of each entry within its hash: lanes since the last start at or before it
-    const uint64_t upto = lane == 63u ? ~0ull : ((2ull << lane) - 1ull);
-    const uint32_t rank = lane - (63u - (uint32_t)__builtin_clzll(S & upto));
-    uint64_t g[kRhalfGroup];
-#pragma unroll
-    for (uint32_t j = 1; j <= kRhalfGroup; ++j) {
-        const uint64_t kd = shfl_down64(k, j);
-        const uint32_t rd = __shfl_down(rank, j);
-        const uint32_t hd = __shfl_down(h, j);
-        g[j - 1] = lane + j < 64u && j <= quota && hd == h && rd == j ? kd : ~0ull;
-    }
-    // slots to [0, m), the other entries after them
-    const uint32_t below = (uint32_t)__popcll(S & ((1ull << lane) - 1ull));
-    const uint32_t dest = start ? below : m + (lane - below);
-    const uint64_t sk = permute64(dest, k);
-    const uint32_t sh = (uint32_t)__builtin_amdgcn_ds_permute((int)(dest * 4u), (int)h);
-    uint64_t sg[kRhalfGroup];
-#pragma unroll
-    for (uint32_t j = 0; j < kRhalfGroup; ++j) sg[j] = permute64(dest, g[j]);
-    const bool live = lane < m;
-#pragma unroll
-    for (int q = 0; q < ER; ++q) {
-        r.b.k[q] = q == 0 && live ? sk : ~0ull;
-        r.b.h[q] = q == 0 && live ? sh : 0xffffffffu;
-#pragma unroll
-        for (uint32_t j = 0; j < kRhalfGroup; ++j) r.g[q][j] = q == 0 && live ? sg[j] : ~0ull;
-    }
-    r.b.c = m;
-}
-
-// Merges one chunk.  A full reservoir takes the plain path (res_chunk: slots
-// sorted in total order, the one-compare bound); a first chunk of at least
-// kBatchMin candidates into an empty one is sorted in (gres_batch_fill).
-// Otherwise the candidates go in one at a time; the insert that fills the
-// reservoir sorts its slots in total order (the plain path's invariant) and
-// the rest of the chunk takes the plain path.
-template <int ER>
-__device__ __forceinline__ void gres_chunk(GroupReservoir<ER> &r, uint64_t ck, uint32_t ch, bool v, uint32_t l_max, uint32_t quota,
-                           uint32_t lane) {
-    if (r.b.c == l_max) {
-        res_chunk(r.b, ck, ch, v, l_max, lane);
-        return;
-    }
-    uint64_t pm = ballot64(v);
-    if (r.b.c == 0 && (uint32_t)__popcll(pm) >= kBatchMin) {
-        gres_batch_fill(r, ck, ch, v, l_max, quota, lane);
-        return;
-    }
-    while (pm) {
-        const uint32_t j = (uint32_t)__builtin_ctzll(pm);
-        pm &= pm - 1ull;
-        gres_fill_insert(r, readlane64(ck, j), readlane32(ch, j), quota, lane);
-        if (r.b.c == l_max) {
-            reg_bitonic<ER, false>(r.b.h, r.b.k, lane);
-            res_chunk(r.b, ck, ch, v && lane > j, l_max, lane);
-            return;
-        }
-    }
-}
-
-// A source's run as the merge needs it: source (num_points: nothing to
-// merge), its sorted segments [start, start + len), the lane's segment
-// (records cnt from first), and its slot count.
-struct RunInfo {
-    uint32_t src, start, len, cnt, c;
-    uint64_t first;
-};
-
-template <bool kGrouped>
-__device__ __forceinline__ RunInfo run_info(uint32_t a, uint32_t na, const uint4 *sorted, const uint32_t *run_src,
-                                            const uint32_t *run_start, const uint32_t *run_len,
-                                            const uint32_t *offsets, uint32_t num_points,
-                                            const uint32_t *slot_count, uint32_t lane) {
-    RunInfo ri{num_points, 0u, 1u, 0u, 0u, 0ull};
-    if (a >= na) return ri;
-    if (kGrouped) {
-        const uint32_t o0 = offsets[a], o1 = offsets[a + 1];
-        if (o1 == o0) return ri;
-        ri.src = a;
-        ri.cnt = lane == 0 ? o1 - o0 : 0u;
-        ri.first = o0;
-    } else {
-        const uint32_t src = run_src[a];
-        if (src >= num_points) return ri;  // the run of empty / bad segments
-        ri.src = src;
-        ri.start = run_start[a];
-        ri.len = run_len[a];
-        if (lane < ri.len) {
-            const uint4 g = sorted[(uint64_t)ri.start + lane];
-            ri.cnt = g.w;
-            ri.first = ((uint64_t)g.z << 32) | g.y;
-        }
-    }
-    ri.c = slot_count[ri.src];
-    return ri;
-}
-
-// A source's live slots (prefetched one source ahead).
-template <int ER>
-__device__ __forceinline__ void load_slots(Reservoir<ER> &r, const RunInfo &ri, uint32_t num_points,
-                                           uint32_t l_max, const uint64_t *slot_keys, const uint16_t *slot_hash,
-                                           uint32_t lane) {
-    const bool real = ri.src < num_points;
-    const uint32_t c = real ? ri.c : 0u;
-    const uint64_t sbase = (uint64_t)(real ? ri.src : 0u) * l_max;
-#pragma unroll
-    for (int q = 0; q < ER; ++q) {
-        const uint32_t e = (uint32_t)q * 64u + lane;
-        const bool live = e < c;
-        r.k[q] = live ? slot_keys[sbase + e] : ~0ull;
-        r.h[q] = live ? (uint32_t)slot_hash[sbase + e] : 0xffffffffu;
-    }
-}
-
-// One wave per source with new records: its slots (and, while a slot is free,
-// their groups) in registers, its records streamed through them.  Sources
-// come from segment runs (as hp_merge_stream_kernel) or, kGrouped, from the
-// record batch grouped by source (offsets[src] .. offsets[src + 1]).  Each
-// wave walks its sources with the next source's slots, and the one after's
-// run and slot count, already in flight.  Five waves per SIMD (a few
-// registers of the rarely taken paths spill) beat the four that fit without
-// spilling: the kernel is bound by latency more than by its instructions.
-template <int ER, bool kGrouped>
-__global__ __launch_bounds__(kHpThreads) __attribute__((amdgpu_waves_per_eu(5))) void hp_merge_rhalf_kernel(
-    const uint4 *records, const uint4 *sorted, const uint32_t *run_src, const uint32_t *run_start,
-    const uint32_t *run_len, const uint32_t *num_runs, const uint32_t *offsets, uint32_t num_points, uint32_t l_max,
-    uint32_t quota, uint64_t *slot_keys, uint16_t *slot_hash, uint32_t *slot_count, uint64_t *grp_keys) {
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t waves = gridDim.x * kHpWaves;
-    const uint32_t na = kGrouped ? num_points : *num_runs;
-    uint32_t a = blockIdx.x * kHpWaves + (threadIdx.x >> 6);
-    if (a >= na) return;
-    auto info = [&](uint32_t i) {
-        return run_info<kGrouped>(i, na, sorted, run_src, run_start, run_len, offsets, num_points, slot_count,
-                                  lane);
-    };
-    RunInfo cur_ri = info(a);
-    Reservoir<ER> cur;
-    load_slots(cur, cur_ri, num_points, l_max, slot_keys, slot_hash, lane);
-    RunInfo nxt_ri = info(a + waves);
-    for (; a < na; a += waves) {
-        Reservoir<ER> nxt;
-        load_slots(nxt, nxt_ri, num_points, l_max, slot_keys, slot_hash, lane);
-        const RunInfo far_ri = info(a + 2u * waves);
-        const uint32_t src = cur_ri.src;
-        if (src < num_points) {
-            GroupReservoir<ER> r;
-            r.b = cur;
-            r.b.c = (uint32_t)__builtin_amdgcn_readfirstlane((int)cur_ri.c);
-            const uint64_t sbase = (uint64_t)src * l_max;
-            // the groups of a reservoir with a free slot (its slots' only)
-            const bool groups = r.b.c > 0u && r.b.c < l_max;
-#pragma unroll
-            for (int q = 0; q < ER; ++q) {
-                const uint32_t e = (uint32_t)q * 64u + lane;
-#pragma unroll
-                for (uint32_t j = 0; j < kRhalfGroup; ++j)
-                    r.g[q][j] = groups && e < r.b.c ? grp_keys[(sbase + e) * kRhalfGroup + j] : ~0ull;
-            }
-            const uint32_t len = cur_ri.len;
-            auto chunk = [&](uint64_t ck, uint32_t ch, bool v) { gres_chunk(r, ck, ch, v, l_max, quota, lane); };
-            stream_group(records, len < 64u ? len : 64u, cur_ri.cnt, cur_ri.first, lane, chunk);
-            for (uint32_t g0 = 64; g0 < len; g0 += 64) {
-                // a source with more than 64 segments in the batch: the rest, 64 at a time
-                const uint32_t ng = len - g0 < 64u ? len - g0 : 64u;
-                uint32_t c2 = 0;
-                uint64_t f2 = 0;
-                if (lane < ng) {
-                    const uint4 g = sorted[(uint64_t)cur_ri.start + g0 + lane];
-                    c2 = g.w;
-                    f2 = ((uint64_t)g.z << 32) | g.y;
-                }
-                stream_group(records, ng, c2, f2, lane, chunk);
-            }
-            const bool keep_groups = r.b.c < l_max;
-#pragma unroll
-            for (int q = 0; q < ER; ++q) {
-                const uint32_t e = (uint32_t)q * 64u + lane;
-                if (e < r.b.c) {
-                    slot_keys[sbase + e] = r.b.k[q];
-                    slot_hash[sbase + e] = (uint16_t)r.b.h[q];
-                    if (keep_groups) {
-#pragma unroll
-                        for (uint32_t j = 0; j < kRhalfGroup; ++j)
-                            grp_keys[(sbase + e) * kRhalfGroup + j] = r.g[q][j];
-                    }
-                }
-            }
-            if (lane == 0) slot_count[src] = r.b.c;
-        }
-        cur = nxt;
-        cur_ri = nxt_ri;
-        nxt_ri = far_ri;
-    }
-}
-
 __device__ __forceinline__ uint64_t total_key64(double d) {
     const uint64_t b = (uint64_t)__double_as_longlong(d);
     return (b & 0x8000000000000000ull) ? ~b : (b | 0x8000000000000000ull);
@@ -1395,7 +1041,7 @@ __global__ __launch_bounds__(kHpThreads) void hp_export_rhalf_kernel(
                 }
             }
         }
-        reg_bitonic<ER, true>(h, k, lane);
+        reg_bitonic<ER>(h, k, lane);
 #pragma unroll
         for (int q = 0; q < ER; ++q) {
             const uint32_t e = (uint32_t)q * 64u + lane;
@@ -1407,6 +1053,23 @@ __global__ __launch_bounds__(kHpThreads) void hp_export_rhalf_kernel(
         }
         if (counts && lane == 0) counts[p] = c + take;
     }
+}
+
+template <int ER, bool kGrouped>
+void launch_merge_er(const HpMergeArgs &A, bool rhalf, uint32_t grid, hipStream_t stream) {
+    if (rhalf)
+        hipLaunchKernelGGL((hp_merge_kernel<ER, true, kGrouped>), dim3(grid), dim3(kHpThreads), 0, stream, A);
+    else
+        hipLaunchKernelGGL((hp_merge_kernel<ER, false, kGrouped>), dim3(grid), dim3(kHpThreads), 0, stream, A);
+}
+template <bool kGrouped>
+void launch_merge(const HpMergeArgs &A, bool rhalf, uint32_t grid, hipStream_t stream) {
+    if (A.l_max <= 64)
+        launch_merge_er<1, kGrouped>(A, rhalf, grid, stream);
+    else if (A.l_max <= 128)
+        launch_merge_er<2, kGrouped>(A, rhalf, grid, stream);
+    else
+        launch_merge_er<4, kGrouped>(A, rhalf, grid, stream);
 }
 
 uint32_t grid_for(uint64_t n, uint32_t threads, uint32_t cap) {
@@ -1438,30 +1101,9 @@ int launch_hashprune_insert(HashPruneState &s, const uint4 *records, uint64_t co
     hipLaunchKernelGGL(hp_scan_apply, dim3(nb), dim3(kScanThreads), 0, stream, s.bucket, n, s.block_sums, s.offsets);
     hipLaunchKernelGGL(hp_scatter_kernel, dim3(grid_for(count, 256, 16384)), dim3(256), 0, stream, records, count, n,
                        s.bucket, s.offsets, s.grouped);
-    if (s.rhalf_mode) {
-        const uint32_t grid = grid_for(n, kHpWaves, 8192);
-        if (s.l_max <= 64)
-            hipLaunchKernelGGL((hp_merge_rhalf_kernel<1, true>), dim3(grid), dim3(kHpThreads), 0, stream, s.grouped,
-                               nullptr, nullptr, nullptr, nullptr, nullptr, s.offsets, n, s.l_max, s.rhalf_quota,
-                               s.slot_keys, s.slot_hash, s.slot_count, s.grp_keys);
-        else if (s.l_max <= 128)
-            hipLaunchKernelGGL((hp_merge_rhalf_kernel<2, true>), dim3(grid), dim3(kHpThreads), 0, stream, s.grouped,
-                               nullptr, nullptr, nullptr, nullptr, nullptr, s.offsets, n, s.l_max, s.rhalf_quota,
-                               s.slot_keys, s.slot_hash, s.slot_count, s.grp_keys);
-        else
-            hipLaunchKernelGGL((hp_merge_rhalf_kernel<4, true>), dim3(grid), dim3(kHpThreads), 0, stream, s.grouped,
-                               nullptr, nullptr, nullptr, nullptr, nullptr, s.offsets, n, s.l_max, s.rhalf_quota,
-                               s.slot_keys, s.slot_hash, s.slot_count, s.grp_keys);
-        return hipGetLastError() == hipSuccess ? 0 : -1;
-    }
-    // Both kernels decide from slots + new records; a merge never shrinks a
-    // reservoir, so after the large kernel every source it merged still counts
-    // more than kHpRegMax and the small kernel skips it (the reverse order
-    // could merge a source twice).
-    hipLaunchKernelGGL(hp_merge_large_kernel, dim3(grid_for(n, kHpWaves, 2048)), dim3(kHpThreads), 0, stream,
-                       s.grouped, s.offsets, n, s.l_max, s.slot_keys, s.slot_hash, s.slot_count);
-    hipLaunchKernelGGL(hp_merge_small_kernel, dim3(grid_for(n, kHpWaves, 8192)), dim3(kHpThreads), 0, stream,
-                       s.grouped, s.offsets, n, s.l_max, s.slot_keys, s.slot_hash, s.slot_count);
+    const HpMergeArgs A{s.grouped, nullptr, nullptr, nullptr, nullptr, nullptr, s.offsets, n, s.l_max, s.rhalf_quota,
+                        s.slot_keys, s.slot_hash, s.slot_count, s.grp_keys};
+    launch_merge<true>(A, s.rhalf_mode != 0, grid_for(n, kHpWaves, kHpMergeGrid), stream);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -1493,35 +1135,9 @@ int launch_hashprune_insert_segments(HashPruneState &s, const uint4 *records, co
         return -1;
     hipLaunchKernelGGL(hp_seg_gather_kernel, dim3(grid_for(nseg, 256, 16384)), dim3(256), 0, stream, segs,
                        w.vals_out, nseg, w.sorted);
-    const uint32_t grid = grid_for(nseg, kHpWaves, 8192);
-    const uint32_t l = s.l_max;
-    if (s.rhalf_mode) {
-        if (l <= 64)
-            hipLaunchKernelGGL((hp_merge_rhalf_kernel<1, false>), dim3(grid), dim3(kHpThreads), 0, stream, records,
-                               w.sorted, w.run_src, w.run_start, w.run_len, w.num_runs, nullptr, n, l, s.rhalf_quota,
-                               s.slot_keys, s.slot_hash, s.slot_count, s.grp_keys);
-        else if (l <= 128)
-            hipLaunchKernelGGL((hp_merge_rhalf_kernel<2, false>), dim3(grid), dim3(kHpThreads), 0, stream, records,
-                               w.sorted, w.run_src, w.run_start, w.run_len, w.num_runs, nullptr, n, l, s.rhalf_quota,
-                               s.slot_keys, s.slot_hash, s.slot_count, s.grp_keys);
-        else
-            hipLaunchKernelGGL((hp_merge_rhalf_kernel<4, false>), dim3(grid), dim3(kHpThreads), 0, stream, records,
-                               w.sorted, w.run_src, w.run_start, w.run_len, w.num_runs, nullptr, n, l, s.rhalf_quota,
-                               s.slot_keys, s.slot_hash, s.slot_count, s.grp_keys);
-        return hipGetLastError() == hipSuccess ? 0 : -1;
-    }
-    if (l <= 64)
-        hipLaunchKernelGGL(hp_merge_stream_kernel<1>, dim3(grid), dim3(kHpThreads), 0, stream, records, w.sorted,
-                           w.run_src, w.run_start, w.run_len, w.num_runs, n, l, s.slot_keys, s.slot_hash,
-                           s.slot_count);
-    else if (l <= 128)
-        hipLaunchKernelGGL(hp_merge_stream_kernel<2>, dim3(grid), dim3(kHpThreads), 0, stream, records, w.sorted,
-                           w.run_src, w.run_start, w.run_len, w.num_runs, n, l, s.slot_keys, s.slot_hash,
-                           s.slot_count);
-    else
-        hipLaunchKernelGGL(hp_merge_stream_kernel<4>, dim3(grid), dim3(kHpThreads), 0, stream, records, w.sorted,
-                           w.run_src, w.run_start, w.run_len, w.num_runs, n, l, s.slot_keys, s.slot_hash,
-                           s.slot_count);
+    const HpMergeArgs A{records, w.sorted, w.run_src, w.run_start, w.run_len, w.num_runs, nullptr, n, s.l_max,
+                        s.rhalf_quota, s.slot_keys, s.slot_hash, s.slot_count, s.grp_keys};
+    launch_merge<false>(A, s.rhalf_mode != 0, grid_for(nseg, kHpWaves, kHpMergeGrid), stream);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

@@ -7,9 +7,7 @@
 
 namespace tessa {
 
-// Largest reservoir (l_max) the reduce kernel takes: one wave merges at most
-// kHpMergeCap candidates per round, l_max of them the reservoir's own slots.
-constexpr uint32_t kHpMergeCap = 512;
+// Largest reservoir (l_max) the merge takes: four slots per lane of its wave.
 constexpr uint32_t kHpMaxLMax = 256;
 
 struct HashPruneState {

@@ -505,6 +505,14 @@ typedef struct tessa_roots_output {
 tessa_status tessa_session_partition_roots(tessa_session *session, const tessa_sq8_view *sq8,
                                            const tessa_roots_request *req, tessa_roots_output *out);
 
+/* The same for roots that tessa_session_partition_roots does not take: each
+ * of at most leaf_max rows and, with a fanout probe, n * fanout_second within
+ * small_node_limit.  Each is split as tessa_session_run_subtree splits a
+ * resident set of its rows alone with the same seed and max_depth; leaves come
+ * in root order. */
+tessa_status tessa_session_partition_small_roots(tessa_session *session, const tessa_sq8_view *sq8,
+                                                 const tessa_roots_request *req, tessa_roots_output *out);
+
 /* ---- candidate records -> HashPrune edge records ------------------------
  * Replaces the host conversion flush_compact_topk_batch_into_edges
  * (leaf_build.rs:1679-1829) that SHEAR runs on every CompactTopKBatch the

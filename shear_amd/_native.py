@@ -349,6 +349,10 @@ SIGNATURES = {
         TessaStatus,
         [_P, C.POINTER(Sq8View), C.POINTER(RootsRequest), C.POINTER(RootsOutput)],
     ),
+    "tessa_session_partition_small_roots": (
+        TessaStatus,
+        [_P, C.POINTER(Sq8View), C.POINTER(RootsRequest), C.POINTER(RootsOutput)],
+    ),
     "tessa_session_submit_subtree": (
         TessaStatus,
         [_P, C.POINTER(Sq8View), C.POINTER(SubtreeRequest), C.POINTER(_U64)],

@@ -150,6 +150,17 @@ struct PartResult {
     const char *failed_step;
 };
 
+// Workspace of a many-small-roots run (device): the roots' leaf rows (SQ8
+// rows, root r's from root_offsets[r] * fanout), leaf sizes (128 per root) and
+// leaf counts, and where each root's leaves and leaf rows go.
+struct SmallRoots {
+    uint32_t *rows;
+    uint32_t *sizes;
+    uint32_t *count;
+    uint64_t *leaf_base;
+    uint64_t *row_base;
+};
+
 // Assignment tasks seen by the COUNT passes (capture, host side): per task
 // depth, attempt, fanout and its member / leader resident rows.  Filled only
 // when a PartCapture is passed; tasks outside the capture bins (fewer than
@@ -178,5 +189,11 @@ void partition_capacity(uint64_t rows, uint32_t famp, uint32_t leaf_max, uint64_
 // walk's watchdog fired (also flagged as WATCHDOG_STALLED).
 int run_partition(const PartArgs &a, hipStream_t stream, LevelHeader *host_hdr, PartResult *res,
                   PartCapture *capture = nullptr);
+
+// Partitions the roots of `a` (root_count > 0, each a small one: at most
+// leaf_max rows and n * fanout within small_node_limit) side by side, each as
+// a single-root run over its rows alone.
+int run_small_roots(const PartArgs &a, const SmallRoots &m, hipStream_t stream, LevelHeader *host_hdr,
+                    PartResult *res);
 
 }  // namespace tessa

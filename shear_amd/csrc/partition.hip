@@ -1135,70 +1135,77 @@ __global__ __launch_bounds__(64 * kScatterWavesPerBlock) void scatter_kernel(Par
     scatter_item_wave(a, cur, item, a.item_node[item], wl[wave]);
 }
 
-// ---- small root (compute_backend.rs:12648-13078) -----------------------------
+// ---- small roots (compute_backend.rs:12648-13078) ----------------------------
 // A subtree root with n <= leaf_max rows (and n * fanout within the 4096-row
 // small-node scratch) is split by gpu_persistent_process_node: hash-ranked
 // leaders, up to 6 attempts, children below leaf_min merged.  Its rows are
 // 0..n-1 (already sorted and unique), so every child is a set of row ids
 // kept here as a 4096-bit bitmap, and sort_unique / merge become bitwise ORs.
+//
+// One workgroup takes one root.  With kMany the grid is the roots of a run
+// (PartArgs::root_offsets, rows read in place through row_map): a root alone
+// keeps one CU busy for 40-360 us, and a build has tens to hundreds of them.
+// Each root writes its leaves' rows into a place of its own (m.rows from
+// root_offsets[r] * fanout: a root publishes at most n * fanout rows) and its
+// leaf sizes into m.sizes; small_scan_kernel numbers the leaves in root order
+// and small_publish_kernel packs them.
 constexpr int kSmallThreads = 1024;
+constexpr int kSmallWaves = kSmallThreads / 64;
 constexpr uint32_t kSmallMaxRows = 4096;
 constexpr uint32_t kSmallWords = kSmallMaxRows / 32;  // 128
 constexpr size_t kSmallLdsBytes = kSmallMaxRows * 8                                  // keys
                                   + (size_t)kPartMaxLeaders * kSmallWords * 4;       // child bitmaps
 
-__device__ void push_leaf_rows_from_bitmap(PartArgs &a, const uint32_t *bm, uint32_t size, uint64_t li,
-                                           uint64_t start, uint32_t *wpref) {
-    // rows in ascending order: prefix popcount over the 128 words
-    const uint32_t t = threadIdx.x;
-    if (t < kSmallWords) wpref[t] = __popc(bm[t]);
-    __syncthreads();
-    if (t == 0) {
-        uint32_t acc = 0;
-        for (uint32_t w = 0; w < kSmallWords; ++w) {
-            const uint32_t c = wpref[w];
-            wpref[w] = acc;
-            acc += c;
-        }
+// Inclusive scan of v over the wave.
+__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v, uint32_t lane) {
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t y = __shfl_up(v, off);
+        if (lane >= (uint32_t)off) v += y;
     }
-    __syncthreads();
-    if (t < kSmallWords) {
-        uint32_t bits = bm[t];
-        uint32_t pos = wpref[t];
-        while (bits) {
-            const uint32_t b = __ffs(bits) - 1u;
-            bits &= bits - 1u;
-            a.leaf_row_ids[start + pos++] = t * 32u + b;
-        }
-    }
-    if (t == 0) {
-        a.leaf_starts[li] = start;
-        a.leaf_sizes[li] = size;
-        a.leaf_sizes32[li] = size;
-        a.leaf_out_offsets[li] = start * a.k;
-        pc_min(a.counters, TESSA_P_LEAF_SIZE_MIN, size);
-        pc_max(a.counters, TESSA_P_LEAF_SIZE_MAX, size);
-        pc_add(a.counters, TESSA_P_LEAF_SIZE_SUM, size);
-        pc_add(a.counters, TESSA_P_LEAF_SIZE_COUNT, 1);
-    }
-    __syncthreads();
+    return v;
 }
 
-__global__ __launch_bounds__(kSmallThreads) void small_root_kernel(PartArgs a) {
+// Rows of a bitmap in ascending order to out[0, ...), by one wave (two words
+// per lane); row i is written as map[i] when map is given.
+__device__ void wave_rows_of_bitmap(const uint32_t *bm, uint32_t lane, const uint32_t *map, uint32_t *out) {
+    const uint32_t w0 = bm[2u * lane], w1 = bm[2u * lane + 1u];
+    uint32_t pos = wave_incl_scan(__popc(w0) + __popc(w1), lane) - (uint32_t)(__popc(w0) + __popc(w1));
+    uint64_t bits = ((uint64_t)w1 << 32) | w0;
+    while (bits) {
+        const uint32_t i = 64u * lane + (uint32_t)__builtin_ctzll(bits);
+        bits &= bits - 1ull;
+        out[pos++] = map ? map[i] : i;
+    }
+}
+
+template <bool kMany>
+__global__ __launch_bounds__(kSmallThreads) void small_root_kernel(PartArgs a, SmallRoots m) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     uint64_t *keys = reinterpret_cast<uint64_t *>(smem);
-    uint32_t *bm = reinterpret_cast<uint32_t *>(smem + kSmallMaxRows * 8);  // [128][128]
+    uint32_t *cand = reinterpret_cast<uint32_t *>(smem + kSmallMaxRows * 8);  // shares the bitmaps' place
+    uint32_t *bm = reinterpret_cast<uint32_t *>(smem + kSmallMaxRows * 8);    // [128][128]
     __shared__ uint32_t leaders[kPartMaxLeaders];
     __shared__ uint32_t child_cnt[kPartMaxLeaders + 1];
-    __shared__ uint32_t wpref[kSmallWords];
-    __shared__ uint32_t s_split, s_ok, s_stop;
+    __shared__ uint32_t child_start[kPartMaxLeaders + 1];
+    __shared__ uint32_t s_split, s_ok, s_stop, s_cand;
 
     const uint32_t t = threadIdx.x;
-    const uint32_t n = a.rows;  // root rows 0..n-1
+    const uint32_t lane = t & 63u, wave = t >> 6;
+    const uint32_t root = blockIdx.x;
+    const uint64_t row0 = kMany ? a.root_offsets[root] : 0ull;  // the root's rows 0..n-1 are resident rows row0..
+    const uint32_t n = kMany ? (uint32_t)(a.root_offsets[root + 1u] - row0) : a.rows;
+    const uint64_t seed = kMany ? a.root_seeds[root] : a.seed;
+    const uint32_t *map = kMany ? a.row_map + row0 : nullptr;
+    auto sq8_row = [&](uint32_t i) -> uint64_t { return kMany ? map[i] : i; };
     const uint32_t terminal = a.leaf_max;
     const uint32_t merge_min = a.leaf_min;
     const bool probe = a.fanout_second > 1u && n > 1u;  // relative depth 0
     if (t == 0) {
+        if (kMany) {
+            m.count[root] = 0u;
+            m.row_base[root] = 0ull;
+        }
         pc_add(a.counters, TESSA_P_PARTITION_POPS, 1);
         pc_add(a.counters, TESSA_P_PARTITION_LEVEL_ROUNDS, 1);
         s_stop = 0u;
@@ -1211,24 +1218,61 @@ __global__ __launch_bounds__(kSmallThreads) void small_root_kernel(PartArgs a) {
     }
     __syncthreads();
     if (s_stop) return;
+    // child_cnt / bm [0, split) published as leaves
+    auto publish = [&](uint32_t split) {
+        uint32_t rows_total = 0;
+        for (uint32_t c = 0; c < split; ++c) rows_total += child_cnt[c];
+        if (!kMany && ((uint64_t)split > a.max_leaf_count || rows_total > a.max_leaf_rows)) {
+            if (t == 0)
+                pc_flag(a.counters, (uint64_t)split > a.max_leaf_count ? TESSA_OVF_LEAF_DESC : TESSA_OVF_LEAF_ROW);
+            return;
+        }
+        if (t == 0) {
+            uint32_t at = 0, lo = 0xffffffffu, hi = 0u;
+            for (uint32_t c = 0; c < split; ++c) {
+                child_start[c] = at;
+                at += child_cnt[c];
+                lo = child_cnt[c] < lo ? child_cnt[c] : lo;
+                hi = child_cnt[c] > hi ? child_cnt[c] : hi;
+            }
+            pc_min(a.counters, TESSA_P_LEAF_SIZE_MIN, lo);
+            pc_max(a.counters, TESSA_P_LEAF_SIZE_MAX, hi);
+            pc_add(a.counters, TESSA_P_LEAF_SIZE_SUM, rows_total);
+            pc_add(a.counters, TESSA_P_LEAF_SIZE_COUNT, split);
+            if (kMany) {
+                m.count[root] = split;
+                m.row_base[root] = rows_total;  // small_scan_kernel turns it into the root's first row
+            } else {
+                a.hdr->leaf_count = split;
+                a.hdr->leaf_rows = rows_total;
+                a.counters[TESSA_P_OUTPUT_LEAF_COUNT] = split;
+                a.counters[TESSA_P_OUTPUT_ROWS] = rows_total;
+            }
+        }
+        __syncthreads();
+        uint32_t *out = kMany ? m.rows + row0 * a.fanout_second : a.leaf_row_ids;
+        for (uint32_t c = wave; c < split; c += kSmallWaves)
+            wave_rows_of_bitmap(bm + c * kSmallWords, lane, map, out + child_start[c]);
+        if (t < split) {
+            if (kMany) {
+                m.sizes[root * kPartMaxLeaders + t] = child_cnt[t];
+            } else {
+                a.leaf_starts[t] = child_start[t];
+                a.leaf_sizes[t] = child_cnt[t];
+                a.leaf_sizes32[t] = child_cnt[t];
+                a.leaf_out_offsets[t] = (uint64_t)child_start[t] * a.k;
+            }
+        }
+    };
     // all rows as one bitmap (child slot 0)
     auto whole_leaf = [&]() {
         if (t < kSmallWords) {
             const uint32_t lo = t * 32u;
             bm[t] = lo >= n ? 0u : (n - lo >= 32u ? 0xffffffffu : ((1u << (n - lo)) - 1u));
         }
+        if (t == 0) child_cnt[0] = n;
         __syncthreads();
-        if (1ull > a.max_leaf_count || (uint64_t)n > a.max_leaf_rows) {
-            if (t == 0) pc_flag(a.counters, 1ull > a.max_leaf_count ? TESSA_OVF_LEAF_DESC : TESSA_OVF_LEAF_ROW);
-            return;
-        }
-        push_leaf_rows_from_bitmap(a, bm, n, 0, 0, wpref);
-        if (t == 0) {
-            a.hdr->leaf_count = 1;
-            a.hdr->leaf_rows = n;
-            a.counters[TESSA_P_OUTPUT_LEAF_COUNT] = 1;
-            a.counters[TESSA_P_OUTPUT_ROWS] = n;
-        }
+        publish(1u);
     };
     if (!probe) {  // n <= terminal here
         whole_leaf();
@@ -1262,20 +1306,37 @@ __global__ __launch_bounds__(kSmallThreads) void small_root_kernel(PartArgs a) {
         if (use_root) {
             if (t < nl) leaders[t] = a.root_leaders[t];
         } else {
-            // compute_backend.rs:12770-12800: the nl smallest (key, point)
+            // compute_backend.rs:12770-12800: the nl smallest (key, point).
+            // The keys are hashes, so the ones below (4 nl + 32) / n of the
+            // range hold them nearly always and only those are ranked
+            // against each other (the rank of every key against every other
+            // took 150 us for 2,048 rows); fewer than nl of them: all are.
             for (uint32_t i = t; i < n; i += kSmallThreads)
-                keys[i] = hash64(a.seed ^ ((uint64_t)attempt * 0xbf58476d1ce4e5b9ull) ^
+                keys[i] = hash64(seed ^ ((uint64_t)attempt * 0xbf58476d1ce4e5b9ull) ^
                                  (((uint64_t)a.root_depth) << 19) ^ (((uint64_t)i) << 7) ^ (((uint64_t)i) << 31));
-            __syncthreads();
-            for (uint32_t i = t; i < n; i += kSmallThreads) {
+            uint64_t top = 4u * nl + 32u < n ? (~0ull / n) * (4u * nl + 32u) : ~0ull;
+            for (;;) {
+                if (t == 0) s_cand = 0u;
+                __syncthreads();
+                for (uint32_t i = t; i < n; i += kSmallThreads)
+                    if (keys[i] <= top) cand[atomicAdd(&s_cand, 1u)] = i;
+                __syncthreads();
+                if (s_cand >= nl || top == ~0ull) break;
+                top = ~0ull;
+                __syncthreads();
+            }
+            const uint32_t nc = s_cand;
+            for (uint32_t j = t; j < nc; j += kSmallThreads) {
+                const uint32_t i = cand[j];
                 const uint64_t ki = keys[i];
                 uint32_t rank = 0;
-                for (uint32_t jj = 0; jj < n; ++jj) {
-                    const uint64_t kj = keys[jj];
-                    rank += (kj < ki || (kj == ki && jj < i)) ? 1u : 0u;
+                for (uint32_t jj = 0; jj < nc; ++jj) {
+                    const uint64_t kj = keys[cand[jj]];
+                    rank += (kj < ki || (kj == ki && cand[jj] < i)) ? 1u : 0u;
                 }
                 if (rank < nl) leaders[rank] = i;
             }
+            __syncthreads();  // cand is read before the bitmaps take its place
         }
         const uint32_t fanout = req < nl ? req : nl;
         for (uint32_t w = t; w < nl * kSmallWords; w += kSmallThreads) bm[w] = 0u;
@@ -1284,19 +1345,38 @@ __global__ __launch_bounds__(kSmallThreads) void small_root_kernel(PartArgs a) {
             pc_max(a.counters, TESSA_P_EFFECTIVE_DEEPER_FANOUT, 1u);
         }
         __syncthreads();
-        // assignment: one thread per row, leaders in slot order
+        // assignment: one thread per row, leaders in slot order (four dots
+        // at a time share the row's loads)
         for (uint32_t i = t; i < n; i += kSmallThreads) {
             float bd[4] = {kEmptyDist, kEmptyDist, kEmptyDist, kEmptyDist};
             uint32_t bs[4] = {kEmptyId, kEmptyId, kEmptyId, kEmptyId};
             uint32_t bl[4] = {kEmptyId, kEmptyId, kEmptyId, kEmptyId};
-            const int8_t *ci = a.codes + (uint64_t)i * pd;
-            const float ps = a.scales[i], pn = a.norms[i];
+            const uint64_t ri = sq8_row(i);
+            const int4 *ci = reinterpret_cast<const int4 *>(a.codes + ri * pd);
+            const float ps = a.scales[ri], pn = a.norms[ri];
             auto run = [&](auto fc) {
                 constexpr int F = decltype(fc)::value;
-                for (uint32_t s = 0; s < nl; ++s) {
-                    const uint32_t l = leaders[s];
-                    const int dot = dot_i8_rows(ci, a.codes + (uint64_t)l * pd, pd);
-                    insert_slot<F>(assign_l2(dot, ps, pn, a.scales[l], a.norms[l]), i, l, s, bd, bs, bl);
+                for (uint32_t s0 = 0; s0 < nl; s0 += 4u) {
+                    uint64_t lr[4];
+                    int dot[4] = {0, 0, 0, 0};
+#pragma unroll
+                    for (uint32_t j = 0; j < 4u; ++j) lr[j] = sq8_row(leaders[s0 + j < nl ? s0 + j : s0]);
+                    for (uint32_t q = 0; q < pd / 16u; ++q) {
+                        const int4 x = ci[q];
+#pragma unroll
+                        for (uint32_t j = 0; j < 4u; ++j) {
+                            const int4 y = reinterpret_cast<const int4 *>(a.codes + lr[j] * pd)[q];
+                            dot[j] = __builtin_amdgcn_sdot4(x.x, y.x, dot[j], false);
+                            dot[j] = __builtin_amdgcn_sdot4(x.y, y.y, dot[j], false);
+                            dot[j] = __builtin_amdgcn_sdot4(x.z, y.z, dot[j], false);
+                            dot[j] = __builtin_amdgcn_sdot4(x.w, y.w, dot[j], false);
+                        }
+                    }
+#pragma unroll
+                    for (uint32_t j = 0; j < 4u; ++j)
+                        if (s0 + j < nl)
+                            insert_slot<F>(assign_l2(dot[j], ps, pn, a.scales[lr[j]], a.norms[lr[j]]), i,
+                                           leaders[s0 + j], s0 + j, bd, bs, bl);
                 }
             };
             switch (fanout) {
@@ -1393,23 +1473,68 @@ __global__ __launch_bounds__(kSmallThreads) void small_root_kernel(PartArgs a) {
         return;
     }
     // Every child has <= n <= leaf_max rows, so all become leaves (:13023-13045).
-    uint64_t rows_total = 0;
-    for (uint32_t c = 0; c < split; ++c) rows_total += child_cnt[c];
-    if ((uint64_t)split > a.max_leaf_count || rows_total > a.max_leaf_rows) {
-        if (t == 0) pc_flag(a.counters, (uint64_t)split > a.max_leaf_count ? TESSA_OVF_LEAF_DESC : TESSA_OVF_LEAF_ROW);
-        return;
+    publish(split);
+}
+
+// First leaf and first leaf row of each root, in root order (one workgroup).
+__global__ __launch_bounds__(1024) void small_scan_kernel(PartArgs a, SmallRoots m) {
+    __shared__ uint64_t sh[1024];
+    uint64_t leaves = 0, rows = 0;
+    for (uint32_t r0 = 0; r0 < a.root_count; r0 += 1024u) {
+        const uint32_t r = r0 + threadIdx.x;
+        uint64_t c = 0, z = 0, tc, tz;
+        if (r < a.root_count) {
+            c = m.count[r];
+            z = m.row_base[r];
+        }
+        const uint64_t ec = block_exclusive_scan(c, sh, &tc);
+        __syncthreads();
+        const uint64_t ez = block_exclusive_scan(z, sh, &tz);
+        __syncthreads();
+        if (r < a.root_count) {
+            m.leaf_base[r] = leaves + ec;
+            m.row_base[r] = rows + ez;
+        }
+        leaves += tc;
+        rows += tz;
     }
-    uint64_t start = 0;
-    for (uint32_t c = 0; c < split; ++c) {
-        push_leaf_rows_from_bitmap(a, bm + c * kSmallWords, child_cnt[c], c, start, wpref);
-        start += child_cnt[c];
+    if (threadIdx.x == 0) {
+        if (leaves > a.max_leaf_count) pc_flag(a.counters, TESSA_OVF_LEAF_DESC);
+        if (rows > a.max_leaf_rows) pc_flag(a.counters, TESSA_OVF_LEAF_ROW);
+        const bool fits = leaves <= a.max_leaf_count && rows <= a.max_leaf_rows;
+        a.hdr->leaf_count = fits ? leaves : 0ull;  // small_publish_kernel writes only what fits
+        a.hdr->leaf_rows = fits ? rows : 0ull;
+        a.counters[TESSA_P_OUTPUT_LEAF_COUNT] = leaves;
+        a.counters[TESSA_P_OUTPUT_ROWS] = rows;
     }
-    if (t == 0) {
-        a.hdr->leaf_count = split;
-        a.hdr->leaf_rows = rows_total;
-        a.counters[TESSA_P_OUTPUT_LEAF_COUNT] = split;
-        a.counters[TESSA_P_OUTPUT_ROWS] = rows_total;
+}
+
+// A root's leaves to their final place (one workgroup per root).
+__global__ __launch_bounds__(256) void small_publish_kernel(PartArgs a, SmallRoots m) {
+    if (a.hdr->leaf_count == 0ull) return;
+    __shared__ uint32_t start[kPartMaxLeaders];
+    const uint32_t root = blockIdx.x, t = threadIdx.x, c = m.count[root];
+    const uint64_t leaf0 = m.leaf_base[root], row0 = m.row_base[root];
+    if (t < 64u) {
+        // 128 leaf slots, two per lane
+        const uint32_t z0 = 2u * t < c ? m.sizes[root * kPartMaxLeaders + 2u * t] : 0u;
+        const uint32_t z1 = 2u * t + 1u < c ? m.sizes[root * kPartMaxLeaders + 2u * t + 1u] : 0u;
+        const uint32_t end = wave_incl_scan(z0 + z1, t);
+        start[2u * t] = end - z0 - z1;
+        start[2u * t + 1u] = end - z1;
     }
+    __syncthreads();
+    if (c == 0u) return;
+    if (t < c) {
+        a.leaf_starts[leaf0 + t] = row0 + start[t];
+        a.leaf_sizes32[leaf0 + t] = m.sizes[root * kPartMaxLeaders + t];
+        if (a.leaf_root) a.leaf_root[leaf0 + t] = root;
+        // a split root's leaves are one level below it; a whole root is its own leaf
+        if (a.leaf_depth) a.leaf_depth[leaf0 + t] = a.root_depth + (c > 1u ? 1u : 0u);
+    }
+    const uint32_t rows = start[c - 1u] + m.sizes[root * kPartMaxLeaders + c - 1u];
+    const uint32_t *src = m.rows + a.root_offsets[root] * a.fanout_second;
+    for (uint32_t i = t; i < rows; i += blockDim.x) a.leaf_row_ids[row0 + i] = src[i];
 }
 
 // ---- the persistent walk ----------------------------------------------------
@@ -1730,8 +1855,8 @@ int run_partition(const PartArgs &args, hipStream_t s, LevelHeader *hh, PartResu
     const bool probe = a.fanout_second > 1u && a.rows > 1u;
     const bool probe_overflow = probe && (uint64_t)a.rows * a.fanout_second > (uint64_t)a.small_node_limit;
     if (a.rows <= a.leaf_max && !probe_overflow) {
-        if (ensure_lds_limit(reinterpret_cast<const void *>(small_root_kernel), (int)kSmallLdsBytes)) return -1;
-        hipLaunchKernelGGL(small_root_kernel, dim3(1), dim3(kSmallThreads), kSmallLdsBytes, s, a);
+        if (ensure_lds_limit(reinterpret_cast<const void *>(small_root_kernel<false>), (int)kSmallLdsBytes)) return -1;
+        hipLaunchKernelGGL(small_root_kernel<false>, dim3(1), dim3(kSmallThreads), kSmallLdsBytes, s, a, SmallRoots{});
         if (hipGetLastError() != hipSuccess) return -1;
         res->levels = 1;
         if (read_header()) return -1;
@@ -1743,6 +1868,23 @@ int run_partition(const PartArgs &args, hipStream_t s, LevelHeader *hh, PartResu
     hipLaunchKernelGGL(root_kernel, dim3((a.rows + 255u) / 256u), dim3(256), 0, s, a);
     if (hipGetLastError() != hipSuccess) return -1;
     return run_levels(a, s, hh, res, capture, level_nodes, level_rows);
+}
+
+int run_small_roots(const PartArgs &a, const SmallRoots &m, hipStream_t s, LevelHeader *hh, PartResult *res) {
+    *res = PartResult{};
+    hipLaunchKernelGGL(init_kernel, dim3(1), dim3(256), 0, s, a);
+    if (ensure_lds_limit(reinterpret_cast<const void *>(small_root_kernel<true>), (int)kSmallLdsBytes)) return -1;
+    hipLaunchKernelGGL(small_root_kernel<true>, dim3(a.root_count), dim3(kSmallThreads), kSmallLdsBytes, s, a, m);
+    hipLaunchKernelGGL(small_scan_kernel, dim3(1), dim3(1024), 0, s, a, m);
+    hipLaunchKernelGGL(small_publish_kernel, dim3(a.root_count), dim3(256), 0, s, a, m);
+    if (hipError_t e = hipGetLastError(); e != hipSuccess) return part_fail(res, e, "small roots launch");
+    hipError_t e = hipMemcpyAsync(hh, a.hdr, sizeof(LevelHeader), hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e != hipSuccess) return part_fail(res, e, "small roots header read-back");
+    res->levels = 1;
+    res->leaf_count = hh->leaf_count;
+    res->leaf_rows = hh->leaf_rows;
+    return 0;
 }
 
 // The level loop from the nodes of level 0 (in the first arena): the

@@ -1362,8 +1362,10 @@ tessa_status tessa_session_run_subtree(tessa_session *s, const tessa_subtree_req
     return tessa_session_run_subtree_locked(s, rq, out);
 }
 
-static tessa_status tessa_session_partition_roots_locked(tessa_session *s, const tessa_sq8_view *sq8,
-                                                         const tessa_roots_request *rq, tessa_roots_output *out) {
+// The request checks of both many-root entries; `small` says which kind of
+// root the entry takes.
+static tessa_status check_roots_request(const tessa_sq8_view *sq8, const tessa_roots_request *rq,
+                                        tessa_roots_output *out, bool small) {
     if (!sq8 || !rq || !out) return make_status(TESSA_ERR_INVALID_ARGUMENT, 0, "partition roots: null argument");
     out->leaf_count = out->leaf_rows_total = 0;
     out->levels = 0;
@@ -1398,12 +1400,119 @@ static tessa_status tessa_session_partition_roots_locked(tessa_session *s, const
         const uint64_t n = b - a;
         const bool large = n > rq->leaf_max ||
                            (rq->fanout_second > 1 && n * rq->fanout_second > (uint64_t)rq->small_node_limit);
-        if (!large)
+        if (small && large)
+            return make_status(TESSA_ERR_INVALID_ARGUMENT, 0,
+                               "partition roots: root %u of %llu rows is a large root (run it with "
+                               "tessa_session_partition_roots)",
+                               i, (unsigned long long)n);
+        if (!small && !large)
             return make_status(TESSA_ERR_INVALID_ARGUMENT, 0,
                                "partition roots: root %u of %llu rows is a small root (run it with "
                                "tessa_session_run_subtree)",
                                i, (unsigned long long)n);
     }
+    return ok_status();
+}
+
+// Grows the session's partition workspace.
+static tessa_status reserve_partition(tessa_session *s, size_t need) {
+    if (s->part_bytes >= need) return ok_status();
+    TESSA_HIP_TRY(hipStreamSynchronize(s->stream));
+    if (s->part) (void)hipFree(s->part);
+    s->part = nullptr;
+    s->part_bytes = 0;
+    if (hipMalloc(&s->part, need) != hipSuccess)
+        return make_status(TESSA_ERR_OUT_OF_MEMORY, TESSA_OVF_WORKSPACE_BUDGET,
+                           "Failed to allocate CUDA GPU persistent subtree workspace (HIP, %zu bytes) "
+                           "overflow_flags=0x%llx overflow_labels=WORKSPACE_BUDGET",
+                           need, (unsigned long long)TESSA_OVF_WORKSPACE_BUDGET);
+    s->part_bytes = need;
+    return ok_status();
+}
+
+// The roots' offsets and seeds to the device; every row id must be an SQ8 row
+// (the kernels read codes through it).
+static tessa_status upload_roots(tessa_session *s, const tessa_sq8_view *sq8, const tessa_roots_request *rq,
+                                 uint64_t *d_roff, uint64_t *d_seed, uint32_t *d_chk) {
+    TESSA_HIP_TRY(hipMemcpyAsync(d_roff, rq->root_offsets, (rq->root_count + 1ull) * 8, hipMemcpyHostToDevice,
+                                 s->stream));
+    TESSA_HIP_TRY(hipMemcpyAsync(d_seed, rq->root_seeds, rq->root_count * 8ull, hipMemcpyHostToDevice, s->stream));
+    hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, s->stream, d_chk, 1u, 0u);
+    hipLaunchKernelGGL(max_u32_kernel, dim3(1024), dim3(256), 0, s->stream, rq->rows, rq->root_offsets[rq->root_count],
+                       d_chk);
+    uint32_t max_row = 0;
+    TESSA_HIP_TRY(hipMemcpyAsync(&max_row, d_chk, 4, hipMemcpyDeviceToHost, s->stream));
+    TESSA_HIP_TRY(hipStreamSynchronize(s->stream));
+    if (max_row >= sq8->rows)
+        return make_status(TESSA_ERR_INVALID_ARGUMENT, TESSA_OVF_INVALID_ASSIGN_POINT_ID,
+                           "partition roots: row id %u outside the %llu SQ8 rows overflow_flags=0x%llx "
+                           "overflow_labels=INVALID_ASSIGN_POINT_ID",
+                           max_row, (unsigned long long)sq8->rows, (unsigned long long)TESSA_OVF_INVALID_ASSIGN_POINT_ID);
+    return ok_status();
+}
+
+// The request's fields that both many-root runs hand to the kernels.
+static tessa::PartArgs roots_args(const tessa_session *s, const tessa_sq8_view *sq8, const tessa_roots_request *rq,
+                                  const tessa_roots_output *out, const uint64_t *d_roff, const uint64_t *d_seed) {
+    const uint64_t rows = rq->root_offsets[rq->root_count];
+    PartArgs a{};
+    a.codes = sq8->codes;
+    a.scales = sq8->scales;
+    a.norms = sq8->norms;
+    a.row_map = rq->rows;
+    a.rows = (uint32_t)rows;
+    a.padded_dim = sq8->padded_dim;
+    a.root_offsets = d_roff;
+    a.root_seeds = d_seed;
+    a.root_count = rq->root_count;
+    a.root_depth = rq->root_depth;
+    a.max_depth = rq->max_depth;
+    a.max_leaders = rq->max_leaders;
+    a.fanout_second = rq->fanout_second;
+    a.leaf_min = rq->leaf_min;
+    a.leaf_max = rq->leaf_max;
+    a.small_node_limit = rq->small_node_limit;
+    a.psamp = rq->psamp_fraction;
+    a.large_scratch_rows = rows * rq->fanout_second;
+    a.max_leaf_count = rq->max_leaf_count;
+    a.max_leaf_rows = rq->max_leaf_rows;
+    a.leaf_row_ids = out->leaf_rows;
+    a.leaf_starts = out->leaf_starts;
+    a.leaf_sizes32 = out->leaf_sizes;
+    a.leaf_root = out->leaf_roots;
+    a.leaf_depth = out->leaf_depths;
+    a.counters = s->part_counters;
+    a.hdr = s->part_hdr;
+    return a;
+}
+
+// After the run: counters and leaf totals to the caller, leaf members through
+// `map` (resident indices -> SQ8 row ids; not after an overflow, when the
+// leaf totals may exceed the outputs), the time since ev0.
+static tessa_status finish_roots(tessa_session *s, const PartResult &pr, const uint32_t *map,
+                                 tessa_roots_output *out) {
+    uint64_t c[TESSA_SUBTREE_COUNTER_WORDS];
+    TESSA_HIP_TRY(hipMemcpyAsync(c, s->part_counters, sizeof(c), hipMemcpyDeviceToHost, s->stream));
+    TESSA_HIP_TRY(hipStreamSynchronize(s->stream));
+    if (out->counters) std::memcpy(out->counters, c, sizeof(c));
+    out->levels = pr.levels;
+    out->leaf_count = pr.leaf_count;
+    out->leaf_rows_total = pr.leaf_rows;
+    const bool overflow = c[TESSA_P_OVERFLOW_FLAGS] != 0;
+    if (map && pr.leaf_rows && !overflow)
+        hipLaunchKernelGGL(map_rows_kernel, dim3((uint32_t)std::min<uint64_t>((pr.leaf_rows + 255) / 256, 8192)),
+                           dim3(256), 0, s->stream, out->leaf_rows, pr.leaf_rows, map);
+    TESSA_HIP_TRY(hipEventRecord(s->ev1, s->stream));
+    TESSA_HIP_TRY(hipEventSynchronize(s->ev1));
+    float ms = 0.0f;
+    (void)hipEventElapsedTime(&ms, s->ev0, s->ev1);
+    out->partition_ms = ms;
+    return overflow ? subtree_overflow(s, c, ms) : ok_status();
+}
+
+static tessa_status tessa_session_partition_roots_locked(tessa_session *s, const tessa_sq8_view *sq8,
+                                                         const tessa_roots_request *rq, tessa_roots_output *out) {
+    if (tessa_status st = check_roots_request(sq8, rq, out, false); st.code) return st;
     const uint64_t rows = rq->root_offsets[rq->root_count];
     const uint32_t famp = rq->fanout_second;
     if (rows * famp > 0xffffffffull)
@@ -1416,71 +1525,16 @@ static tessa_status tessa_session_partition_roots_locked(tessa_session *s, const
     const size_t off_roff = align256(L.bytes), off_seed = off_roff + align256((rq->root_count + 1ull) * 8),
                  off_sz64 = off_seed + align256(rq->root_count * 8ull),
                  off_chk = off_sz64 + align256(rq->max_leaf_count * 8ull), need = off_chk + 256;
-    if (s->part_bytes < need) {
-        TESSA_HIP_TRY(hipStreamSynchronize(s->stream));
-        if (s->part) (void)hipFree(s->part);
-        s->part = nullptr;
-        s->part_bytes = 0;
-        if (hipMalloc(&s->part, need) != hipSuccess)
-            return make_status(TESSA_ERR_OUT_OF_MEMORY, TESSA_OVF_WORKSPACE_BUDGET,
-                               "Failed to allocate CUDA GPU persistent subtree workspace (HIP, %zu bytes) "
-                               "overflow_flags=0x%llx overflow_labels=WORKSPACE_BUDGET",
-                               need, (unsigned long long)TESSA_OVF_WORKSPACE_BUDGET);
-        s->part_bytes = need;
-    }
+    if (tessa_status st = reserve_partition(s, need); st.code) return st;
     char *base = static_cast<char *>(s->part);
     uint64_t *d_roff = reinterpret_cast<uint64_t *>(base + off_roff);
     uint64_t *d_seed = reinterpret_cast<uint64_t *>(base + off_seed);
     uint32_t *d_chk = reinterpret_cast<uint32_t *>(base + off_chk);
-    TESSA_HIP_TRY(hipMemcpyAsync(d_roff, rq->root_offsets, (rq->root_count + 1ull) * 8, hipMemcpyHostToDevice,
-                                 s->stream));
-    TESSA_HIP_TRY(hipMemcpyAsync(d_seed, rq->root_seeds, rq->root_count * 8ull, hipMemcpyHostToDevice, s->stream));
-    // every row id must be an SQ8 row (the kernels read codes through it)
-    hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, s->stream, d_chk, 1u, 0u);
-    hipLaunchKernelGGL(max_u32_kernel, dim3(1024), dim3(256), 0, s->stream, rq->rows, rows, d_chk);
-    uint32_t max_row = 0;
-    TESSA_HIP_TRY(hipMemcpyAsync(&max_row, d_chk, 4, hipMemcpyDeviceToHost, s->stream));
-    TESSA_HIP_TRY(hipStreamSynchronize(s->stream));
-    if (max_row >= sq8->rows)
-        return make_status(TESSA_ERR_INVALID_ARGUMENT, TESSA_OVF_INVALID_ASSIGN_POINT_ID,
-                           "partition roots: row id %u outside the %llu SQ8 rows overflow_flags=0x%llx "
-                           "overflow_labels=INVALID_ASSIGN_POINT_ID",
-                           max_row, (unsigned long long)sq8->rows, (unsigned long long)TESSA_OVF_INVALID_ASSIGN_POINT_ID);
+    if (tessa_status st = upload_roots(s, sq8, rq, d_roff, d_seed, d_chk); st.code) return st;
 
-    PartArgs a{};
-    a.codes = sq8->codes;
-    a.scales = sq8->scales;
-    a.norms = sq8->norms;
-    a.row_map = rq->rows;
-    a.rows = (uint32_t)rows;
-    a.padded_dim = sq8->padded_dim;
-    a.root_offsets = d_roff;
-    a.root_seeds = d_seed;
-    a.root_count = rq->root_count;
-    a.root_leaders = nullptr;
-    a.root_leader_count = 0;
-    a.root_depth = rq->root_depth;
-    a.max_depth = rq->max_depth;
-    a.max_leaders = rq->max_leaders;
-    a.fanout_second = rq->fanout_second;
-    a.leaf_min = rq->leaf_min;
-    a.leaf_max = rq->leaf_max;
-    a.small_node_limit = rq->small_node_limit;
-    a.k = 0;
-    a.psamp = rq->psamp_fraction;
-    a.seed = 0;
-    a.large_scratch_rows = rows * famp;
-    a.max_leaf_count = rq->max_leaf_count;
-    a.max_leaf_rows = rq->max_leaf_rows;
-    a.leaf_row_ids = out->leaf_rows;
-    a.leaf_starts = out->leaf_starts;
+    PartArgs a = roots_args(s, sq8, rq, out, d_roff, d_seed);
     a.leaf_sizes = reinterpret_cast<uint64_t *>(base + off_sz64);
-    a.leaf_sizes32 = out->leaf_sizes;
     a.leaf_out_offsets = reinterpret_cast<uint64_t *>(base + L.off_outoff);
-    a.leaf_root = out->leaf_roots;
-    a.leaf_depth = out->leaf_depths;
-    a.counters = s->part_counters;
-    a.hdr = s->part_hdr;
     for (int i = 0; i < 2; ++i) {
         a.arena[i] = reinterpret_cast<uint32_t *>(base + L.off_arena[i]);
         a.nodes[i] = reinterpret_cast<NodeDesc *>(base + L.off_nodes[i]);
@@ -1501,31 +1555,44 @@ static tessa_status tessa_session_partition_roots_locked(tessa_session *s, const
     const int rc = run_partition(a, s->stream, s->part_hdr_host, &pr, nullptr);
     if (rc != 0)
         return partition_failure(rc, pr);
-    uint64_t c[TESSA_SUBTREE_COUNTER_WORDS];
-    TESSA_HIP_TRY(hipMemcpyAsync(c, s->part_counters, sizeof(c), hipMemcpyDeviceToHost, s->stream));
-    TESSA_HIP_TRY(hipStreamSynchronize(s->stream));
-    if (out->counters) std::memcpy(out->counters, c, sizeof(c));
-    out->levels = pr.levels;
-    out->leaf_count = pr.leaf_count;
-    out->leaf_rows_total = pr.leaf_rows;
-    if (c[TESSA_P_OVERFLOW_FLAGS] != 0) {
-        TESSA_HIP_TRY(hipEventRecord(s->ev1, s->stream));
-        TESSA_HIP_TRY(hipEventSynchronize(s->ev1));
-        float ms = 0.0f;
-        (void)hipEventElapsedTime(&ms, s->ev0, s->ev1);
-        out->partition_ms = ms;
-        return subtree_overflow(s, c, ms);
-    }
-    // leaf members: resident indices -> SQ8 row ids
-    if (pr.leaf_rows)
-        hipLaunchKernelGGL(map_rows_kernel, dim3((uint32_t)std::min<uint64_t>((pr.leaf_rows + 255) / 256, 8192)),
-                           dim3(256), 0, s->stream, out->leaf_rows, pr.leaf_rows, rq->rows);
-    TESSA_HIP_TRY(hipEventRecord(s->ev1, s->stream));
-    TESSA_HIP_TRY(hipEventSynchronize(s->ev1));
-    float ms = 0.0f;
-    (void)hipEventElapsedTime(&ms, s->ev0, s->ev1);
-    out->partition_ms = ms;
-    return ok_status();
+    return finish_roots(s, pr, rq->rows, out);
+}
+
+static tessa_status tessa_session_partition_small_roots_locked(tessa_session *s, const tessa_sq8_view *sq8,
+                                                               const tessa_roots_request *rq,
+                                                               tessa_roots_output *out) {
+    if (tessa_status st = check_roots_request(sq8, rq, out, true); st.code) return st;
+    const uint64_t rows = rq->root_offsets[rq->root_count], nr = rq->root_count;
+    if (rows * rq->fanout_second > 0xffffffffull || nr * kLeaderStride > 0xffffffffull)
+        return make_status(TESSA_ERR_UNSUPPORTED, 0, "partition roots: rows x fanout must stay below 2^32");
+    TESSA_HIP_TRY(hipSetDevice(s->device));
+    // workspace: offsets, seeds, check word, then SmallRoots' arrays
+    size_t at = 0;
+    auto place = [&](size_t bytes) {
+        const size_t o = at;
+        at += align256(bytes);
+        return o;
+    };
+    const size_t off_roff = place((nr + 1) * 8), off_seed = place(nr * 8), off_chk = place(4),
+                 off_rows = place(rows * rq->fanout_second * 4), off_sizes = place(nr * kLeaderStride * 4),
+                 off_count = place(nr * 4), off_lb = place(nr * 8), off_rb = place(nr * 8);
+    if (tessa_status st = reserve_partition(s, at); st.code) return st;
+    char *base = static_cast<char *>(s->part);
+    uint64_t *d_roff = reinterpret_cast<uint64_t *>(base + off_roff);
+    uint64_t *d_seed = reinterpret_cast<uint64_t *>(base + off_seed);
+    if (tessa_status st = upload_roots(s, sq8, rq, d_roff, d_seed, reinterpret_cast<uint32_t *>(base + off_chk));
+        st.code)
+        return st;
+    const PartArgs a = roots_args(s, sq8, rq, out, d_roff, d_seed);
+    const tessa::SmallRoots m{
+        reinterpret_cast<uint32_t *>(base + off_rows),  reinterpret_cast<uint32_t *>(base + off_sizes),
+        reinterpret_cast<uint32_t *>(base + off_count), reinterpret_cast<uint64_t *>(base + off_lb),
+        reinterpret_cast<uint64_t *>(base + off_rb)};
+    TESSA_HIP_TRY(hipEventRecord(s->ev0, s->stream));
+    PartResult pr{};
+    const int rc = tessa::run_small_roots(a, m, s->stream, s->part_hdr_host, &pr);
+    if (rc != 0) return partition_failure(rc, pr);
+    return finish_roots(s, pr, nullptr, out);
 }
 
 tessa_status tessa_session_partition_roots(tessa_session *s, const tessa_sq8_view *sq8, const tessa_roots_request *rq,
@@ -1533,6 +1600,13 @@ tessa_status tessa_session_partition_roots(tessa_session *s, const tessa_sq8_vie
     if (!s) return make_status(TESSA_ERR_INVALID_ARGUMENT, 0, "session is null");
     std::lock_guard<std::mutex> lock(s->exec_mu);
     return tessa_session_partition_roots_locked(s, sq8, rq, out);
+}
+
+tessa_status tessa_session_partition_small_roots(tessa_session *s, const tessa_sq8_view *sq8,
+                                                 const tessa_roots_request *rq, tessa_roots_output *out) {
+    if (!s) return make_status(TESSA_ERR_INVALID_ARGUMENT, 0, "session is null");
+    std::lock_guard<std::mutex> lock(s->exec_mu);
+    return tessa_session_partition_small_roots_locked(s, sq8, rq, out);
 }
 
 }  // extern "C"

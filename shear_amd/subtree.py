@@ -253,14 +253,15 @@ class SubtreeSession:
 
     def partition_roots(self, sq8, rows: torch.Tensor, root_offsets: np.ndarray, root_seeds: np.ndarray,
                         params: PiPNNSubtreeParams, depth: int = 1, max_depth: int | None = None,
-                        memory_budget_bytes: int | None = None) -> RootsDeviceOutput:
+                        memory_budget_bytes: int | None = None, small: bool = False) -> RootsDeviceOutput:
         """Partition many subtree roots in one run (tessa_session_partition_roots):
         root i owns the SQ8 rows rows[root_offsets[i]:root_offsets[i+1]]
         (``rows`` a device int32 view of u32 row ids into ``sq8``, ascending per
         root) and starts from root_seeds[i] at ``depth``.  Each root is planned
         as a task of its own (``plan_subtree`` under ``memory_budget_bytes``);
         every root must be a large one (more than leaf_max rows or a fanout
-        probe beyond the small-node scratch)."""
+        probe beyond the small-node scratch), or with ``small`` every root a
+        small one (tessa_session_partition_small_roots)."""
         offs = np.ascontiguousarray(root_offsets, np.uint64)
         seeds = np.ascontiguousarray(root_seeds, np.uint64)
         famp = max(params.fanout_second, 1)
@@ -295,8 +296,8 @@ class SubtreeSession:
         out = N.RootsOutput(out_rows.data_ptr(), out_starts.data_ptr(), out_sizes.data_ptr(), out_roots.data_ptr(),
                             out_depths.data_ptr(), counters.ctypes.data, 0, 0, 0, 0.0)
         torch.cuda.synchronize(dev)  # inputs and outputs come from torch's stream
-        N.check(self._lib.tessa_session_partition_roots(self._h, C.byref(view), C.byref(rq), C.byref(out)),
-                "tessa_session_partition_roots")
+        name = "tessa_session_partition_small_roots" if small else "tessa_session_partition_roots"
+        N.check(getattr(self._lib, name)(self._h, C.byref(view), C.byref(rq), C.byref(out)), name)
         return RootsDeviceOutput(out_rows, out_starts, out_sizes, out_roots, out_depths, int(out.leaf_count),
                                  int(out.leaf_rows_total), int(out.levels), float(out.partition_ms), counters)
 

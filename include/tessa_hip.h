@@ -670,6 +670,21 @@ typedef struct tessa_hashprune_backfill {
 tessa_status tessa_hashprune_create_backfill(uint32_t num_points, uint32_t l_max,
                                              const tessa_hashprune_backfill *policy, tessa_hashprune **out);
 
+/* A reducer in the caller's device memory: `memory`, 256-byte aligned, holds
+ * the tessa_hashprune_state_bytes of the same shape and policy (NULL policy:
+ * none), its earlier work has finished, and it outlives the reducer.  The
+ * caller may also lend the workspace of tessa_hashprune_insert_segments
+ * (tessa_hashprune_segment_bytes of the largest batch; a batch that needs more
+ * allocates its own; NULL takes it back).  A program that makes one reducer
+ * after another keeps this memory instead of returning gigabytes to the
+ * driver and asking for them again, which has stalled for 0.1-1.4 s. */
+tessa_status tessa_hashprune_state_bytes(uint32_t num_points, uint32_t l_max, const tessa_hashprune_backfill *policy,
+                                         uint64_t *bytes);
+tessa_status tessa_hashprune_create_in(uint32_t num_points, uint32_t l_max, const tessa_hashprune_backfill *policy,
+                                       void *memory, uint64_t bytes, tessa_hashprune **out);
+tessa_status tessa_hashprune_segment_bytes(const tessa_hashprune *hp, uint64_t segment_count, uint64_t *bytes);
+tessa_status tessa_hashprune_lend_segment_memory(tessa_hashprune *hp, void *memory, uint64_t bytes);
+
 /* ---- TierLift: the bounded host reducer of the record stream ---------------
  * Replaces SpillEdgeSink + ExternalHashPruneReducer
  * (shear-core/src/algorithm/pipnn/spill_hashprune.rs:349-651 routing, shard

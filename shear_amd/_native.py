@@ -365,6 +365,10 @@ SIGNATURES = {
     ),
     "tessa_hashprune_create": (TessaStatus, [_U32, _U32, C.POINTER(_P)]),
     "tessa_hashprune_create_backfill": (TessaStatus, [_U32, _U32, C.POINTER(HashPruneBackfill), C.POINTER(_P)]),
+    "tessa_hashprune_state_bytes": (TessaStatus, [_U32, _U32, C.POINTER(HashPruneBackfill), C.POINTER(_U64)]),
+    "tessa_hashprune_create_in": (TessaStatus, [_U32, _U32, C.POINTER(HashPruneBackfill), _P, _U64, C.POINTER(_P)]),
+    "tessa_hashprune_segment_bytes": (TessaStatus, [_P, _U64, C.POINTER(_U64)]),
+    "tessa_hashprune_lend_segment_memory": (TessaStatus, [_P, _P, _U64]),
     "tessa_hashprune_destroy": (TessaStatus, [_P]),
     "tessa_hashprune_insert": (TessaStatus, [_P, _P, _U64, _P]),
     "tessa_hashprune_neighbors": (TessaStatus, [_P, _P, _P, _P, _P, _P]),

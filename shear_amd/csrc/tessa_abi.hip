@@ -2077,17 +2077,38 @@ tessa_status tessa_emit_edge_segments_unique(const uint32_t *global_ids, uint64_
 struct tessa_hashprune {
     int device = 0;
     tessa::HashPruneState st;
+    bool own_state = true;   // the state's arrays are freed with the reducer (else the caller's memory)
+    bool own_seg_ws = true;  // so is the segment workspace
 };
 
 namespace {
 
 void free_hashprune(tessa_hashprune *hp) {
     auto &s = hp->st;
-    for (void *ptr : {(void *)s.slot_keys, (void *)s.slot_hash, (void *)s.slot_count, (void *)s.bucket,
-                      (void *)s.offsets, (void *)s.block_sums, (void *)s.grouped, (void *)s.status,
-                      (void *)s.seg_ws, (void *)s.grp_keys})
-        if (ptr) (void)hipFree(ptr);
+    if (hp->own_state && s.slot_keys) (void)hipFree(s.slot_keys);  // the first array: one block holds all
+    if (s.grouped) (void)hipFree(s.grouped);
+    if (hp->own_seg_ws && s.seg_ws) (void)hipFree(s.seg_ws);
     delete hp;
+}
+
+// The state's arrays in one block from `base` (or their total size).
+uint64_t hashprune_state_layout(tessa::HashPruneState &s, void *base) {
+    uint64_t at = 0;
+    auto place = [&](auto *&p, uint64_t bytes) {
+        p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(static_cast<char *>(base) + at);
+        at += align256(bytes ? bytes : 16);
+    };
+    const uint64_t n = s.num_points, slots = n * s.l_max;
+    s.block_sums_capacity = tessa::hashprune_scan_blocks(s.num_points);
+    place(s.slot_keys, slots * 8);
+    place(s.slot_hash, slots * 2);
+    place(s.slot_count, n * 4);
+    place(s.bucket, n * 4);
+    place(s.offsets, (n + 1) * 4);
+    place(s.block_sums, s.block_sums_capacity * 4);
+    place(s.status, 8 * 4);
+    if (s.rhalf_mode) place(s.grp_keys, slots * 8 * tessa::kRhalfGroup);
+    return at;
 }
 
 tessa_status hp_alloc(void **ptr, uint64_t bytes, const char *what) {
@@ -2134,39 +2155,46 @@ tessa_status resolve_backfill(const tessa_hashprune_backfill *bf, uint32_t l_max
     return ok_status();
 }
 
-tessa_status hashprune_make(uint32_t num_points, uint32_t l_max, const tessa_hashprune_backfill *bf,
-                            tessa_hashprune **out) {
-    if (!out) return make_status(TESSA_ERR_INVALID_ARGUMENT, 0, "hashprune: null output");
-    *out = nullptr;
+// The checked shape and policy of a reducer, no memory yet.
+tessa_status hashprune_shape(uint32_t num_points, uint32_t l_max, const tessa_hashprune_backfill *bf,
+                             tessa::HashPruneState &s) {
     if (l_max == 0) return make_status(TESSA_ERR_INVALID_ARGUMENT, 0, "l_max must be > 0");
     if (l_max > tessa::kHpMaxLMax)
         return make_status(TESSA_ERR_UNSUPPORTED, 0, "hashprune: l_max=%u above %u", l_max, tessa::kHpMaxLMax);
+    tessa_status st = resolve_backfill(bf, l_max, s);
+    s.num_points = num_points;
+    s.l_max = l_max;
+    return st;
+}
+
+// mem: the caller's block of `bytes` (null: allocated here).
+tessa_status hashprune_make(uint32_t num_points, uint32_t l_max, const tessa_hashprune_backfill *bf, void *mem,
+                            uint64_t bytes, tessa_hashprune **out) {
+    if (!out) return make_status(TESSA_ERR_INVALID_ARGUMENT, 0, "hashprune: null output");
+    *out = nullptr;
     tessa::HashPruneState probe;
-    tessa_status st = resolve_backfill(bf, l_max, probe);
+    tessa_status st = hashprune_shape(num_points, l_max, bf, probe);
     if (st.code) return st;
+    const uint64_t need = hashprune_state_layout(probe, nullptr);
+    if (mem && (bytes < need || (reinterpret_cast<uintptr_t>(mem) & 255u) != 0))
+        return make_status(TESSA_ERR_INVALID_ARGUMENT, 0,
+                           "hashprune: the caller's memory must be 256-byte aligned and hold %llu bytes (got %llu)",
+                           (unsigned long long)need, (unsigned long long)bytes);
     auto *hp = new (std::nothrow) tessa_hashprune();
     if (!hp) return make_status(TESSA_ERR_OUT_OF_MEMORY, 0, "hashprune: host allocation failed");
     if (hipGetDevice(&hp->device) != hipSuccess) {
         delete hp;
         return make_status(TESSA_ERR_HIP, 0, "hashprune: hipGetDevice failed");
     }
+    hp->own_state = mem == nullptr;
+    if (!mem) st = hp_alloc(&mem, need, "hashprune reservoirs");
+    if (st.code) {
+        delete hp;
+        return st;
+    }
     auto &s = hp->st;
     s = probe;
-    s.num_points = num_points;
-    s.l_max = l_max;
-    const uint64_t slots = (uint64_t)num_points * l_max;
-    st = hp_alloc((void **)&s.slot_keys, slots * 8, "hashprune slot keys");
-    if (!st.code && s.rhalf_mode)
-        st = hp_alloc((void **)&s.grp_keys, slots * 8 * tessa::kRhalfGroup, "hashprune backfill groups");
-    if (!st.code) st = hp_alloc((void **)&s.slot_hash, slots * 2, "hashprune slot hashes");
-    if (!st.code) st = hp_alloc((void **)&s.slot_count, (uint64_t)num_points * 4, "hashprune slot counts");
-    if (!st.code) st = hp_alloc((void **)&s.bucket, (uint64_t)num_points * 4, "hashprune source counts");
-    if (!st.code) st = hp_alloc((void **)&s.offsets, ((uint64_t)num_points + 1) * 4, "hashprune source offsets");
-    if (!st.code) {
-        s.block_sums_capacity = tessa::hashprune_scan_blocks(num_points);
-        st = hp_alloc((void **)&s.block_sums, s.block_sums_capacity * 4, "hashprune scan partials");
-    }
-    if (!st.code) st = hp_alloc((void **)&s.status, 8 * 4, "hashprune status");
+    hashprune_state_layout(s, mem);
     if (!st.code && tessa::launch_hashprune_clear(s, nullptr) != 0)
         st = make_status(TESSA_ERR_HIP, 0, "hashprune clear launch failed");
     if (!st.code && hipStreamSynchronize(nullptr) != hipSuccess)
@@ -2184,12 +2212,52 @@ tessa_status hashprune_make(uint32_t num_points, uint32_t l_max, const tessa_has
 extern "C" {
 
 tessa_status tessa_hashprune_create(uint32_t num_points, uint32_t l_max, tessa_hashprune **out) {
-    return hashprune_make(num_points, l_max, nullptr, out);
+    return hashprune_make(num_points, l_max, nullptr, nullptr, 0, out);
 }
 
 tessa_status tessa_hashprune_create_backfill(uint32_t num_points, uint32_t l_max,
                                              const tessa_hashprune_backfill *policy, tessa_hashprune **out) {
-    return hashprune_make(num_points, l_max, policy, out);
+    return hashprune_make(num_points, l_max, policy, nullptr, 0, out);
+}
+
+tessa_status tessa_hashprune_state_bytes(uint32_t num_points, uint32_t l_max, const tessa_hashprune_backfill *policy,
+                                         uint64_t *bytes) {
+    if (!bytes) return make_status(TESSA_ERR_INVALID_ARGUMENT, 0, "hashprune: null output");
+    tessa::HashPruneState s;
+    tessa_status st = hashprune_shape(num_points, l_max, policy, s);
+    *bytes = st.code ? 0 : hashprune_state_layout(s, nullptr);
+    return st;
+}
+
+tessa_status tessa_hashprune_create_in(uint32_t num_points, uint32_t l_max, const tessa_hashprune_backfill *policy,
+                                       void *memory, uint64_t bytes, tessa_hashprune **out) {
+    if (!memory) return make_status(TESSA_ERR_INVALID_ARGUMENT, 0, "hashprune: null memory");
+    return hashprune_make(num_points, l_max, policy, memory, bytes, out);
+}
+
+tessa_status tessa_hashprune_segment_bytes(const tessa_hashprune *hp, uint64_t segment_count, uint64_t *bytes) {
+    if (!hp || !bytes) return make_status(TESSA_ERR_INVALID_ARGUMENT, 0, "hashprune is null");
+    if (segment_count >= 0x7fffffffull)
+        return make_status(TESSA_ERR_UNSUPPORTED, 0, "hashprune: %llu segments in one batch (limit 2^31-2)",
+                           (unsigned long long)segment_count);
+    *bytes = tessa::hashprune_segment_workspace_bytes(segment_count, hp->st.num_points);
+    return ok_status();
+}
+
+tessa_status tessa_hashprune_lend_segment_memory(tessa_hashprune *hp, void *memory, uint64_t bytes) {
+    if (!hp) return make_status(TESSA_ERR_INVALID_ARGUMENT, 0, "hashprune is null");
+    if (memory && (reinterpret_cast<uintptr_t>(memory) & 255u) != 0)
+        return make_status(TESSA_ERR_INVALID_ARGUMENT, 0, "hashprune: segment memory must be 256-byte aligned");
+    auto &s = hp->st;
+    if (hp->own_seg_ws && s.seg_ws) {
+        TESSA_HIP_TRY(hipSetDevice(hp->device));
+        TESSA_HIP_TRY(hipDeviceSynchronize());
+        TESSA_HIP_TRY(hipFree(s.seg_ws));
+    }
+    hp->own_seg_ws = false;
+    s.seg_ws = memory;
+    s.seg_ws_bytes = memory ? bytes : 0;
+    return ok_status();
 }
 
 tessa_status tessa_hashprune_destroy(tessa_hashprune *hp) {
@@ -2288,9 +2356,10 @@ tessa_status tessa_hashprune_insert_segments(tessa_hashprune *hp, const tessa_ed
     const uint64_t need = tessa::hashprune_segment_workspace_bytes(segment_count, s.num_points);
     if (need > s.seg_ws_bytes) {
         TESSA_HIP_TRY(hipStreamSynchronize(hs));
-        if (s.seg_ws) TESSA_HIP_TRY(hipFree(s.seg_ws));
+        if (s.seg_ws && hp->own_seg_ws) TESSA_HIP_TRY(hipFree(s.seg_ws));
         s.seg_ws = nullptr;
         s.seg_ws_bytes = 0;
+        hp->own_seg_ws = true;
         tessa_status st = hp_alloc(&s.seg_ws, need, "hashprune segment workspace");
         if (st.code) return st;
         s.seg_ws_bytes = need;

@@ -74,20 +74,26 @@ class HashPruneReducer:
         self.device = torch.device(device)
         self.backfill = backfill if backfill is not None and backfill.mode != "off" else None
         self._lib = N.load()
-        h = C.c_void_p()
+        self._h = h = C.c_void_p()
+        self._state = self._seg = None
+        pol = None if self.backfill is None else C.byref(self.backfill.native())
         with torch.cuda.device(self.device):
-            if self.backfill is None:
-                st = self._lib.tessa_hashprune_create(self.num_points, self.l_max, C.byref(h))
-            else:
-                pol = self.backfill.native()
-                st = self._lib.tessa_hashprune_create_backfill(self.num_points, self.l_max, C.byref(pol), C.byref(h))
-            N.check(st, "hashprune create")
-        self._h = h
+            # the reservoirs lie in torch's memory: made and dropped once per
+            # build, gigabytes went back to the driver and came again, which
+            # stalled for 0.1-1.4 s now and then
+            need = C.c_uint64(0)
+            N.check(self._lib.tessa_hashprune_state_bytes(self.num_points, self.l_max, pol, C.byref(need)),
+                    "hashprune create")
+            self._state = torch.empty(need.value, dtype=torch.uint8, device=self.device)
+            torch.cuda.current_stream().synchronize()  # what used that memory before; the reducer runs on any stream
+            N.check(self._lib.tessa_hashprune_create_in(self.num_points, self.l_max, pol, self._state.data_ptr(),
+                                                        need.value, C.byref(h)), "hashprune create")
 
     def close(self) -> None:
         if self._h:
-            N.check(self._lib.tessa_hashprune_destroy(self._h), "hashprune destroy")
+            N.check(self._lib.tessa_hashprune_destroy(self._h), "hashprune destroy")  # waits for the device
             self._h = C.c_void_p()
+        self._state = self._seg = None
 
     def __enter__(self):
         return self
@@ -127,6 +133,17 @@ class HashPruneReducer:
         n = segments.shape[0] if count is None else int(count)
         if n > segments.shape[0]:
             raise ValueError(f"count {n} exceeds the {segments.shape[0]} segments given")
+        need = C.c_uint64(0)
+        N.check(self._lib.tessa_hashprune_segment_bytes(self._h, n, C.byref(need)), "hashprune insert segments")
+        if self._seg is None or self._seg.numel() < need.value:
+            # every insert is over when it returns, so the old workspace is idle; the new one is ordered on the
+            # stream that will use it first
+            N.check(self._lib.tessa_hashprune_lend_segment_memory(self._h, None, 0), "hashprune insert segments")
+            self._seg = None
+            with torch.cuda.stream(stream if stream is not None else torch.cuda.current_stream(self.device)):
+                self._seg = torch.empty(need.value, dtype=torch.uint8, device=self.device)
+            N.check(self._lib.tessa_hashprune_lend_segment_memory(self._h, self._seg.data_ptr(), need.value),
+                    "hashprune insert segments")
         N.check(self._lib.tessa_hashprune_insert_segments(self._h, _ptr(records), _ptr(segments), n,
                                                           _stream_ptr(stream)), "hashprune insert segments")
 

@@ -236,7 +236,8 @@ def build_graph_sq8(sq8: T.Sq8Matrix, sketches: torch.Tensor, leader_rows: np.nd
     top-k and record emission in chunks of at most ``p.leaf_chunk_rows`` leaf
     rows.  The small children are grouped and run the same way (a run alone
     keeps a few CUs busy and costs some thirty launches: 20,000 x 100 points in
-    54 small children, 37 ms one by one, 9 ms grouped).  Each child's
+    54 small children, 37 ms one by one, 9 ms grouped,
+    measured before anything else changed).  Each child's
     leaves are those of its own run, so the graph is the same either way.
 
     ``observer`` (optional) is called after each batch of records is emitted,
@@ -278,7 +279,14 @@ def build_graph_sq8(sq8: T.Sq8Matrix, sketches: torch.Tensor, leader_rows: np.nd
     firsts = pts[fidx].cpu().numpy().view(np.uint32) if pts.numel() else np.zeros(len(osz), np.uint32)
     start = _entry_point_of(osz, firsts)
     torch.cuda.synchronize()
-    torch.cuda.empty_cache()  # the library allocates the reservoirs and workspaces itself, outside torch's cache
+    # The library allocates its workspaces itself, outside torch's cache: at
+    # most a few GB for the leaf operator and about 16 bytes per replicated row
+    # of a partition run.  Only when that much is not free does torch's cache
+    # go back to the driver (asking for it again cost 1.5 ms a build, and
+    # 0.1-1.4 s when the driver was still clearing it).
+    if torch.cuda.mem_get_info(dev)[0] < (16 << 30) + 32 * max(p.fanout_second, 1) * min(rows * max(p.fanout_top, 1),
+                                                                                    2 * p.roots_rows_per_run):
+        torch.cuda.empty_cache()
     w1 = time.perf_counter()
     sess = S.SubtreeSession(0)
     hp = tl = None
@@ -475,19 +483,22 @@ def _run_root_group(sess, sq8, gids, pts, offs_h, sizes, group, parent_points, p
         # the largest leaf there is (the kernels size their LDS by it); a bound past the operator's limit is its error
         widest = int(lsz[l0:l1].max()) if leaf_max <= SMALL_NODE_LIMIT else leaf_max
         lay = T.LeafLayouts(ro.leaf_rows, off, ro.leaf_sizes[l0:l1], (off - r0) * k, widest, (r1 - r0) * k)
-        side.wait_stream(main)  # the layout tensors above were made on the caller's stream
+        # the outputs come from the caller's stream's memory (each stream of torch's pool would keep its own)
+        ids = torch.empty(lay.output_len, dtype=torch.int32, device=dev)
+        d = torch.empty(lay.output_len, dtype=torch.float32, device=dev)
+        ctr = torch.zeros(N.COUNTER_WORDS, dtype=torch.int64, device=dev)
+        side.wait_stream(main)  # these and the layout tensors were made there
         e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-        with torch.cuda.stream(side):
-            e0.record(side)
-            ids, d, ctr = T.leaf_topk(sq8, gids, lay, k, executor=sp.executor, stream=side)
-            e1.record(side)
+        e0.record(side)
+        T.leaf_topk(sq8, gids, lay, k, executor=sp.executor, out_ids=ids, out_dists=d, counters=ctr, stream=side)
+        e1.record(side)
+        for t in (ids, d, ctr, off, lay.output_offsets):
+            t.record_stream(side)
         return l0, l1, r0, r1, off, lay, ids, d, ctr, e0, e1
 
     def finish(job):
         l0, l1, r0, r1, off, lay, ids, d, ctr, e0, e1 = job
         main.wait_event(e1)
-        for t in (ids, d, ctr):
-            t.record_stream(main)  # used on the caller's stream from here on
         T.raise_on_overflow(ctr, "leaf top-k")
         st["leaf_ms"] += e0.elapsed_time(e1)
         q0 = time.perf_counter()

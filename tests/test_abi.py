@@ -112,3 +112,19 @@ def test_backfill_policy_validation_without_gpu(policy, l_max, code, text):
     st = lib.tessa_hashprune_create_backfill(16, l_max, C.byref(N.HashPruneBackfill(*policy)), C.byref(h))
     assert st.code == code and not h.value
     assert text in st.msg.decode()
+
+
+@pytest.mark.parametrize("policy,per_slot", [(None, 10), ((3, 0, 3, 1.02), 34)])
+def test_reservoirs_in_the_callers_memory_without_gpu(policy, per_slot):
+    # the size covers the slots (8 + 2 bytes, 24 more with backfill groups);
+    # too little, misaligned or no memory is refused before any device work
+    lib = N.load()
+    pol = None if policy is None else C.byref(N.HashPruneBackfill(*policy))
+    need = C.c_uint64(0)
+    assert lib.tessa_hashprune_state_bytes(1000, 64, pol, C.byref(need)).code == 0
+    assert per_slot * 64 * 1000 <= need.value <= per_slot * 64 * 1000 + 64 * 1024
+    h = C.c_void_p()
+    for mem, size in ((256, need.value - 1), (256 + 16, need.value), (None, need.value)):
+        st = lib.tessa_hashprune_create_in(1000, 64, pol, mem, size, C.byref(h))
+        assert st.code == 1 and not h.value
+    assert lib.tessa_hashprune_state_bytes(1000, 257, pol, C.byref(need)).code == 4 and need.value == 0

@@ -30,7 +30,8 @@ namespace tessa {
 namespace {
 
 constexpr int kThreads = 512;
-constexpr int kWaves = kThreads / 64;
+constexpr int kWideThreads = 1024;  // emit pass, reference order, where one workgroup's arrays take the CU
+constexpr int kMaxWaves = kWideThreads / 64;
 constexpr int kCountUnroll = 4;  // rows per half-wave in flight (count pass)
 constexpr int kEmitUnroll = 4;   // rows per half-wave in flight (emit pass)
 constexpr uint32_t kNoKey = 0xffffffffu;
@@ -82,8 +83,10 @@ __device__ __forceinline__ uint32_t leaf_rows(const EdgeParams &p, uint32_t leaf
 // All threads call it.
 // Each half-wave owns a row (lane q = rank); kCountUnroll rows per half-wave
 // have their loads in flight together.
+template <int kThreads>
 __device__ uint32_t row_counts_scan(const EdgeParams &p, uint32_t leaf, uint32_t n, uint32_t kl, uint32_t *cnt,
                                     uint32_t *wsum, bool &regular) {
+    constexpr int kWaves = kThreads / 64;
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63u;
     const uint32_t wave = tid >> 6;
@@ -150,11 +153,11 @@ __device__ uint32_t row_counts_scan(const EdgeParams &p, uint32_t leaf, uint32_t
 __global__ __launch_bounds__(kThreads) void edge_count_kernel(EdgeParams p) {
     extern __shared__ uint32_t lds[];
     uint32_t *wsum = lds;
-    uint32_t *cnt = lds + kWaves;
+    uint32_t *cnt = lds + kMaxWaves;
     for (uint32_t leaf = blockIdx.x; leaf < p.leaf_count; leaf += gridDim.x) {
         const uint32_t n = leaf_rows(p, leaf, true);
         bool regular;
-        const uint32_t total = row_counts_scan(p, leaf, n, leaf_k(p, n), cnt, wsum, regular);
+        const uint32_t total = row_counts_scan<kThreads>(p, leaf, n, leaf_k(p, n), cnt, wsum, regular);
         // total <= 4096 * 32: bit 31 is free for the regular-leaf flag
         if (threadIdx.x == 0) p.leaf_totals[leaf] = total | (regular ? kLeafRegular : 0u);
     }
@@ -207,6 +210,8 @@ __global__ __launch_bounds__(1024) void edge_scan_kernel(EdgeParams p) {
 }
 
 // compute_hash(s_i, s_j) and compute_hash(s_j, s_i) over m_bits coordinates.
+// a - c >= 0 is c - a <= 0 for all floats (the rounded difference changes
+// sign exactly, zeros of either sign satisfy both, NaN neither).
 // kVec4: both rows are 16-byte aligned with at least ceil(m_bits/4)*4 floats.
 template <bool kVec4>
 __device__ __forceinline__ void pair_hashes(const float *si, const float *sj, uint32_t m_bits, uint32_t &hf,
@@ -226,16 +231,17 @@ __device__ __forceinline__ void pair_hashes(const float *si, const float *sj, ui
             for (int e = 0; e < 4; ++e) {
                 const uint32_t bit = 4u * v + e;
                 if (bit < m_bits) {
-                    hf |= (cv[e] - av[e] >= 0.0f ? 1u : 0u) << bit;
-                    hr |= (av[e] - cv[e] >= 0.0f ? 1u : 0u) << bit;
+                    const float t = cv[e] - av[e];
+                    hf |= (t >= 0.0f ? 1u : 0u) << bit;
+                    hr |= (t <= 0.0f ? 1u : 0u) << bit;
                 }
             }
         }
     } else {
         for (uint32_t bit = 0; bit < m_bits; ++bit) {
-            const float a = si[bit], c = sj[bit];
-            hf |= (c - a >= 0.0f ? 1u : 0u) << bit;
-            hr |= (a - c >= 0.0f ? 1u : 0u) << bit;
+            const float t = sj[bit] - si[bit];
+            hf |= (t >= 0.0f ? 1u : 0u) << bit;
+            hr |= (t <= 0.0f ? 1u : 0u) << bit;
         }
     }
 }
@@ -249,12 +255,14 @@ enum SketchMode : int {
 
 // LDS words of the emit kernel: wave sums and the leaf's record base (two
 // words) | row counts | member ids | table keys | table values (u16) |
-// (16-byte aligned) staged sketches.  Grouped order adds two arrays of
-// max_rows words: per row its record count (then a cursor over its reverse
-// records) and the mask of its slots whose reverse record is left out.
-__host__ __device__ inline uint32_t emit_sketch_offset(uint32_t max_rows, uint32_t table_bits, bool grouped) {
-    const uint32_t words = kWaves + 2u + 2u * max_rows + (1u << table_bits) + (1u << table_bits) / 2u +
-                           (grouped ? 2u * max_rows : 0u);
+// (16-byte aligned) staged sketches.  Grouped order adds an array of max_rows
+// words (per row its record count, then a cursor over its reverse records),
+// and without mutual repeats another (the mask of its slots whose reverse
+// record is left out).
+enum EmitOrder : int { kOrderReference = 0, kOrderGrouped = 1, kOrderUnique = 2 };
+__host__ __device__ inline uint32_t emit_sketch_offset(uint32_t max_rows, uint32_t table_bits, int order) {
+    const uint32_t words = kMaxWaves + 2u + 2u * max_rows + (1u << table_bits) + (1u << table_bits) / 2u +
+                           (uint32_t)order * max_rows;
     return (words + 3u) & ~3u;
 }
 
@@ -322,19 +330,22 @@ __device__ __forceinline__ bool slot_listed(const EdgeParams &p, uint64_t slot0,
     return pos != kNoKey && __float_as_uint(p.topk_dists[slot0 + pos]) == db;
 }
 
-template <int kMode, bool kGrouped>
+template <int kMode, int kOrder, int kThreads>
 __global__ __launch_bounds__(kThreads) void edge_emit_kernel(EdgeParams p) {
+    constexpr bool kGrouped = kOrder != kOrderReference;
+    constexpr bool kUnique = kOrder == kOrderUnique;
+    constexpr int kWaves = kThreads / 64;
     extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
     const uint32_t tbits = p.table_bits;
     const uint32_t tmask = (1u << tbits) - 1u;
-    uint32_t *wsum = lds;  // kWaves sums, then the leaf's record base (lo, hi)
-    uint32_t *cnt = lds + kWaves + 2u;
+    uint32_t *wsum = lds;  // kMaxWaves sums, then the leaf's record base (lo, hi)
+    uint32_t *cnt = lds + kMaxWaves + 2u;
     uint32_t *gid = cnt + p.max_leaf_rows;
     uint32_t *tkey = gid + p.max_leaf_rows;
     uint16_t *tval = reinterpret_cast<uint16_t *>(tkey + (1u << tbits));
     uint32_t *tot = tkey + (1u << tbits) + (1u << tbits) / 2u;  // grouped order only
-    uint32_t *dup = tot + p.max_leaf_rows;
-    float *sk_lds = reinterpret_cast<float *>(lds + emit_sketch_offset(p.max_leaf_rows, tbits, kGrouped));
+    uint32_t *dup = tot + p.max_leaf_rows;                      // without mutual repeats only
+    float *sk_lds = reinterpret_cast<float *>(lds + emit_sketch_offset(p.max_leaf_rows, tbits, kOrder));
     const uint32_t mw = (p.m_bits + 3u) & ~3u;  // staged row stride (floats)
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63u;
@@ -355,19 +366,19 @@ __global__ __launch_bounds__(kThreads) void edge_emit_kernel(EdgeParams p) {
         // else counted again and scanned into cnt.
         const bool regular = (p.leaf_totals[leaf] & kLeafRegular) != 0u;
         if (kGrouped) {
-            // with p.unique, cnt holds each row's largest listed distance
+            // without mutual repeats, cnt holds each row's largest listed distance
             // until the segment scan below overwrites it
             const uint64_t o0 = p.output_offsets[leaf];
             for (uint32_t c = tid; c < n; c += kThreads) {
                 tot[c] = 0u;
-                if (p.unique) cnt[c] = __float_as_uint(list_max_dist(p, o0 + (uint64_t)c * p.k, kl));
+                if (kUnique) cnt[c] = __float_as_uint(list_max_dist(p, o0 + (uint64_t)c * p.k, kl));
             }
             __syncthreads();
         } else if (regular) {
             __syncthreads();
         } else {
             bool unused;
-            row_counts_scan(p, leaf, n, kl, cnt, wsum, unused);  // ends with a barrier
+            row_counts_scan<kThreads>(p, leaf, n, kl, cnt, wsum, unused);  // ends with a barrier
         }
         // Member ids, the membership table (global id -> member position) and,
         // in LDS mode, the m_bits leading coordinates of every member's sketch
@@ -413,7 +424,7 @@ __global__ __launch_bounds__(kThreads) void edge_emit_kernel(EdgeParams p) {
             // Per member: its forward records (its valid slots) and its
             // reverse records (valid slots of other rows naming it); the
             // member's segment holds the forward ones, then the reverse ones.
-            // With p.unique a slot whose reverse record another row's forward
+            // Without mutual repeats a slot whose reverse record another row's forward
             // record repeats (slot_listed) gets a bit in dup[row] and its
             // reverse record is neither counted nor written.
             for (uint32_t r0 = 2u * wave + h; r0 < n + h; r0 += kStep * kEmitUnroll) {
@@ -447,15 +458,15 @@ __global__ __launch_bounds__(kThreads) void edge_emit_kernel(EdgeParams p) {
                         }
                     }
                     bool same = false;
-                    if (p.unique && cj != kNoKey && d[u] <= __uint_as_float(cnt[cj])) {
+                    if (kUnique && cj != kNoKey && d[u] <= __uint_as_float(cnt[cj])) {
                         const uint32_t gi = gid[r];  // r < n: the slot is valid
                         if (gi != kNoKey) same = slot_listed(p, out0 + (uint64_t)cj * p.k, kl, gi, __float_as_uint(d[u]));
                     }
                     if (cj != kNoKey && !same) atomicAdd(&tot[cj], 1u);
-                    const uint64_t sm = __ballot(same);
-                    if (r < n && q == 0u) {
-                        atomicAdd(&tot[r], (uint32_t)__popc((uint32_t)(h ? (m >> 32) : m)));
-                        dup[r] = (uint32_t)(h ? (sm >> 32) : sm);
+                    if (r < n && q == 0u) atomicAdd(&tot[r], (uint32_t)__popc((uint32_t)(h ? (m >> 32) : m)));
+                    if constexpr (kUnique) {
+                        const uint64_t sm = __ballot(same);
+                        if (r < n && q == 0u) dup[r] = (uint32_t)(h ? (sm >> 32) : sm);
                     }
                 }
             }
@@ -480,17 +491,17 @@ __global__ __launch_bounds__(kThreads) void edge_emit_kernel(EdgeParams p) {
                 base += (uint32_t)w < wave ? wsum[w] : 0u;
                 leaf_total += wsum[w];
             }
-            if (p.unique) {
+            if (kUnique) {
                 // the leaf's place in the output: its records once the
                 // repeats are left out, taken from the batch's cursor
                 if (tid == 0) {
                     const uint64_t at = atomicAdd((unsigned long long *)&p.status[kEdgeKept],
                                                   (unsigned long long)leaf_total);
-                    wsum[kWaves] = (uint32_t)at;
-                    wsum[kWaves + 1] = (uint32_t)(at >> 32);
+                    wsum[kMaxWaves] = (uint32_t)at;
+                    wsum[kMaxWaves + 1] = (uint32_t)(at >> 32);
                 }
                 __syncthreads();
-                rec0 = (uint64_t)wsum[kWaves] | ((uint64_t)wsum[kWaves + 1] << 32);
+                rec0 = (uint64_t)wsum[kMaxWaves] | ((uint64_t)wsum[kMaxWaves + 1] << 32);
             }
             uint32_t run = base + x - sum;
             const uint64_t sbase = p.leaf_seg_base[leaf];
@@ -567,7 +578,7 @@ __global__ __launch_bounds__(kThreads) void edge_emit_kernel(EdgeParams p) {
                         // the last free place of j's segment
                         const uint32_t fpos = cnt[r] + (uint32_t)__popc(half & ((1u << q) - 1u));
                         store_record<true>(p.out, rec0 + fpos, gi, j[u], hf, db);
-                        if (((dup[r] >> q) & 1u) == 0u) {
+                        if (!kUnique || ((dup[r] >> q) & 1u) == 0u) {
                             const uint32_t rpos = atomicSub(&tot[cj], 1u) - 1u;
                             store_record<true>(p.out, rec0 + rpos, j[u], gi, hr, db);
                         }
@@ -616,42 +627,51 @@ uint32_t edge_table_bits(uint32_t max_leaf_rows) {
     return bits;
 }
 
+namespace {
+template <int kMode, int kOrder, int kThreads>
+int launch_emit_as(const EdgeParams &p, uint32_t grid, size_t lds, hipStream_t stream) {
+    if (ensure_lds_limit(reinterpret_cast<const void *>(edge_emit_kernel<kMode, kOrder, kThreads>), (int)lds)) return -1;
+    hipLaunchKernelGGL((edge_emit_kernel<kMode, kOrder, kThreads>), dim3(grid), dim3(kThreads), lds, stream, p);
+    return 0;
+}
+template <int kMode, int kThreads>
+int launch_emit_mode(const EdgeParams &p, int order, uint32_t grid, size_t lds, hipStream_t stream) {
+    if (order == kOrderReference) return launch_emit_as<kMode, kOrderReference, kThreads>(p, grid, lds, stream);
+    if (order == kOrderGrouped) return launch_emit_as<kMode, kOrderGrouped, kThreads>(p, grid, lds, stream);
+    return launch_emit_as<kMode, kOrderUnique, kThreads>(p, grid, lds, stream);
+}
+template <int kThreads>
+int launch_emit(const EdgeParams &p, int mode, int order, uint32_t grid, size_t lds, hipStream_t stream) {
+    if (mode == kSketchLds) return launch_emit_mode<kSketchLds, kThreads>(p, order, grid, lds, stream);
+    if (mode == kSketchGlobalV4) return launch_emit_mode<kSketchGlobalV4, kThreads>(p, order, grid, lds, stream);
+    return launch_emit_mode<kSketchGlobal, kThreads>(p, order, grid, lds, stream);
+}
+}  // namespace
+
 int launch_edge_records(const EdgeParams &p, hipStream_t stream) {
     hipLaunchKernelGGL(edge_status_init_kernel, dim3(1), dim3(64), 0, stream, p.status);
     if (p.leaf_count == 0) return hipGetLastError() == hipSuccess ? 0 : -1;
     const uint32_t grid = p.leaf_count < 8192u ? p.leaf_count : 8192u;
-    const size_t count_lds = (kWaves + (size_t)p.max_leaf_rows) * sizeof(uint32_t);
+    const size_t count_lds = (kMaxWaves + (size_t)p.max_leaf_rows) * sizeof(uint32_t);
     hipLaunchKernelGGL(edge_count_kernel, dim3(grid), dim3(kThreads), count_lds, stream, p);
     hipLaunchKernelGGL(edge_scan_kernel, dim3(1), dim3(1024), 0, stream, p);
     // Stage the leaf's sketch rows in LDS when they fit; else read them from
     // HBM (float4 loads when rows are 16-byte aligned).
-    const bool grouped = p.segments != nullptr;
-    const size_t base_lds = (size_t)emit_sketch_offset(p.max_leaf_rows, p.table_bits, grouped) * sizeof(uint32_t);
+    const int order = !p.segments ? kOrderReference : p.unique ? kOrderUnique : kOrderGrouped;
+    const size_t base_lds = (size_t)emit_sketch_offset(p.max_leaf_rows, p.table_bits, order) * sizeof(uint32_t);
     const size_t staged = (size_t)p.max_leaf_rows * ((p.m_bits + 3u) & ~3u) * sizeof(float);
     const bool vec4 = p.width % 4u == 0u && (reinterpret_cast<uintptr_t>(p.sketches) & 15u) == 0u;
     const bool in_lds = base_lds + staged <= kEmitLdsBudget;
     const size_t lds = in_lds ? base_lds + staged : base_lds;
-    const void *emit_fn = grouped ? (in_lds ? reinterpret_cast<const void *>(edge_emit_kernel<kSketchLds, true>)
-                                            : vec4 ? reinterpret_cast<const void *>(edge_emit_kernel<kSketchGlobalV4, true>)
-                                                   : reinterpret_cast<const void *>(edge_emit_kernel<kSketchGlobal, true>))
-                                  : (in_lds ? reinterpret_cast<const void *>(edge_emit_kernel<kSketchLds, false>)
-                                            : vec4 ? reinterpret_cast<const void *>(edge_emit_kernel<kSketchGlobalV4, false>)
-                                                   : reinterpret_cast<const void *>(edge_emit_kernel<kSketchGlobal, false>));
-    if (ensure_lds_limit(emit_fn, (int)lds)) return -1;
-    if (grouped) {
-        if (in_lds)
-            hipLaunchKernelGGL((edge_emit_kernel<kSketchLds, true>), dim3(grid), dim3(kThreads), lds, stream, p);
-        else if (vec4)
-            hipLaunchKernelGGL((edge_emit_kernel<kSketchGlobalV4, true>), dim3(grid), dim3(kThreads), lds, stream, p);
-        else
-            hipLaunchKernelGGL((edge_emit_kernel<kSketchGlobal, true>), dim3(grid), dim3(kThreads), lds, stream, p);
+    const int mode = in_lds ? kSketchLds : vec4 ? kSketchGlobalV4 : kSketchGlobal;
+    // One workgroup fills a CU's LDS: in the reference's order 16 waves instead
+    // of 8 hide its latencies (512 leaves of 2,048 rows, k 32: 433 -> 387 us,
+    // 1,600 of 1,300 rows 905 -> 758).  Source-grouped, the scattered reverse
+    // records bound it and more waves only spread them wider (844 -> 884 us).
+    if (order == kOrderReference && lds > kEmitLdsBudget / 2) {
+        if (launch_emit<kWideThreads>(p, mode, order, grid, lds, stream)) return -1;
     } else {
-        if (in_lds)
-            hipLaunchKernelGGL((edge_emit_kernel<kSketchLds, false>), dim3(grid), dim3(kThreads), lds, stream, p);
-        else if (vec4)
-            hipLaunchKernelGGL((edge_emit_kernel<kSketchGlobalV4, false>), dim3(grid), dim3(kThreads), lds, stream, p);
-        else
-            hipLaunchKernelGGL((edge_emit_kernel<kSketchGlobal, false>), dim3(grid), dim3(kThreads), lds, stream, p);
+        if (launch_emit<kThreads>(p, mode, order, grid, lds, stream)) return -1;
     }
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }

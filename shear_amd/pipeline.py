@@ -236,8 +236,7 @@ def build_graph_sq8(sq8: T.Sq8Matrix, sketches: torch.Tensor, leader_rows: np.nd
     top-k and record emission in chunks of at most ``p.leaf_chunk_rows`` leaf
     rows.  The small children are grouped and run the same way (a run alone
     keeps a few CUs busy and costs some thirty launches: 20,000 x 100 points in
-    54 small children, 37 ms one by one, 9 ms grouped,
-    measured before anything else changed).  Each child's
+    54 small children, 38.5 ms one by one, 9.1 ms grouped).  Each child's
     leaves are those of its own run, so the graph is the same either way.
 
     ``observer`` (optional) is called after each batch of records is emitted,

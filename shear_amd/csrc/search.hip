@@ -13,241 +13,425 @@
 // list leaves the L smallest of (list, neighbours) under the total order
 // (distance, id), and the queue's cursor is then the first not-visited entry
 // (an insert in front of the cursor moves it there; entries before it are all
-// visited).  So the wave inserts a whole batch at once: the up-to-64 new
-// neighbours of a chunk of the row are scored one per lane, sorted across the
-// wave, and merged with the list by rank (each entry's new position is its
-// old one plus the number of entries of the other side below it); entries
-// ranked L and past drop off.  Same list, same cursor as the one-by-one
-// inserts.
+// visited).  So the wave inserts the up-to-64 new neighbours of a chunk of the
+// row at once, each entry going to its old place plus the number of entries of
+// the other side below it; entries placed L and past drop off.  Same list,
+// same cursor as the one-by-one inserts.
 //
 // Distances: squared L2 summed over the coordinates in order in f32, each
 // product rounded before the add (no contraction), one lane per candidate
 // (the harness's stated order; the reference's SIMD kernel may associate
 // differently).  With SQ8 rows (sets too large to keep as f32) a row's
 // coordinate i is the f32 product scale * code[i], rounded, then the same sum:
-// the search over the dequantized vectors.  Keys are (distance bits << 32 | id): for the non-negative
-// distances this computes, the integer order is (distance, id).
+// the search over the dequantized vectors.  Keys are (distance bits << 32 |
+// id): for the non-negative distances this computes, the integer order is
+// (distance, id).
 //
-// Visited set: a tag per (slot, point) holding query index + 1; tags are
-// zeroed once per call, so a slot's next query needs no clearing.  The tag is
-// claimed with an atomic exchange so a point listed twice in one row enters
-// the list once.
+// Visited set: a bit per (slot, point), set by an atomic or, so a point listed
+// twice in one row enters the list once; zeroed once per call, and by the
+// slot's wave before its next query.
+//
+// The kernel waits, it does not compute: one wavefront per query and a chain of
+// about L + 10 expansions, each of them neighbour ids -> visited bits -> rows ->
+// distances -> list.  What it does about that:
+//  * a chunk's rows go to LDS by LDS-DMA, whole rows by consecutive lanes and
+//    all in flight together with the visited bits' atomics (the rows of
+//    neighbours that turn out visited are read for nothing); one lane then
+//    sums one row from LDS.  Each lane reading its own row from memory, 64
+//    lines per load and a few loads in flight, took some 16 us an expansion;
+//  * the neighbour ids of the entry that is next in line so far are read
+//    meanwhile;
+//  * the list is held in registers, and a pass over the new neighbours that can
+//    still enter it gives every position by counting, without sorting;
+//  * the visited set is one bit per point (25 KB per query at 200,000 points,
+//    in L2) instead of a 4-byte tag: no 0.14 ms to clear 800 MB, and 32 times
+//    the queries at a time on a set whose tags fill the scratch limit.
+// 1,000 queries, 200,000 x 128: L = 64 1,652 -> 929 us, L = 128 4,187 -> 2,380;
+// 3,000 queries, 150,000 x 200: 4,531 -> 3,075; 64 queries over SQ8 rows,
+// 100,000 x 256: 1,095 -> 961 (there the conversions bound it).
 #include "search_kernels.h"
 #include "tessa_device.h"
+#include "kernel_attr.h"
 
 namespace tessa {
 
 namespace {
 
-constexpr uint32_t kThreads = kSearchWaves * 64;
 constexpr uint64_t kNoKey = ~0ull;
-
-struct alignas(16) WaveLists {
-    uint64_t key[2][kSearchMaxL];     // double-buffered list, ascending
-    uint32_t visited[2][kSearchMaxL];
-    uint64_t fresh[64];               // one chunk's new neighbours, sorted
-};
+constexpr uint32_t kStagedMaxDim = 2048;    // the query lies in LDS too
 
 __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-
-__device__ __forceinline__ uint64_t shfl_u64(uint64_t v, uint32_t src) {
-    const uint32_t lo = __shfl((uint32_t)v, src), hi = __shfl((uint32_t)(v >> 32), src);
-    return ((uint64_t)hi << 32) | lo;
+__device__ __forceinline__ uint32_t readlane32(uint32_t v, uint32_t l) {
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)l);
+}
+__device__ __forceinline__ uint64_t readlane64(uint64_t v, uint32_t l) {
+    return ((uint64_t)readlane32((uint32_t)(v >> 32), l) << 32) | readlane32((uint32_t)v, l);
 }
 
-// Ascending bitonic sort of one u64 per lane across the wave.
-__device__ __forceinline__ uint64_t wave_sort64(uint64_t v, uint32_t lane) {
-#pragma unroll
-    for (uint32_t k = 2; k <= 64; k <<= 1) {
-#pragma unroll
-        for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-            const uint64_t o = shfl_u64(v, lane ^ j);
-            const bool lower = (lane & j) == 0;
-            const bool up = (lane & k) == 0;
-            const uint64_t lo = v < o ? v : o, hi = v < o ? o : v;
-            v = (lower == up) ? lo : hi;
-        }
-    }
-    return v;
+// One more coordinate of a squared L2 distance, in order.
+__device__ __forceinline__ float l2_step(float s, float x, float q) {
+    const float t = __fsub_rn(x, q);
+    return __fadd_rn(s, __fmul_rn(t, t));
 }
 
-// number of entries of a[0, n) (ascending, distinct from x) below x
-__device__ __forceinline__ uint32_t rank_in(const uint64_t *a, uint32_t n, uint64_t x) {
-    uint32_t lo = 0, hi = n;
-    while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (a[mid] < x) lo = mid + 1;
-        else hi = mid;
-    }
-    return lo;
-}
+// Where the rows come from.
+enum SearchRows : int {
+    kRowsF32x4 = 0,   // f32, 16-byte aligned rows of dim % 4 == 0
+    kRowsF32 = 1,     // f32, any
+    kRowsSq8x16 = 2,  // SQ8, 16-byte aligned rows
+    kRowsDirect = 3   // read by each lane from memory: wider than kStagedMaxDim, or SQ8 unaligned
+};
 
-// Squared L2 of the dequantized SQ8 row (scale * code[i], rounded) and the
-// query, coordinates in order; 16 codes per load when kVec16.
-template <bool kVec16>
-__device__ float sq8_l2_ordered(const int8_t *__restrict__ c, float sc, const float *__restrict__ q, uint32_t dim) {
-    float s = 0.0f;
-    if constexpr (kVec16) {
-        typedef int v4i_t __attribute__((ext_vector_type(4)));
-        const v4i_t *cv = reinterpret_cast<const v4i_t *>(c);
-        const float4 *qv = reinterpret_cast<const float4 *>(q);
-        for (uint32_t i = 0; i < dim / 16; ++i) {
-            const v4i_t w = cv[i];
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const float4 b = qv[4 * i + g];
-                const uint32_t word = (uint32_t)w[g];
-                const float bq[4] = {b.x, b.y, b.z, b.w};
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float x = __fmul_rn(sc, (float)(int8_t)(word >> (8 * e)));
-                    const float t = __fsub_rn(x, bq[e]);
-                    s = __fadd_rn(s, __fmul_rn(t, t));
-                }
-            }
-        }
-    } else {
-        for (uint32_t i = 0; i < dim; ++i) {
-            const float t = __fsub_rn(__fmul_rn(sc, (float)c[i]), q[i]);
-            s = __fadd_rn(s, __fmul_rn(t, t));
-        }
+// LDS of a query's wave: the query (dim floats, to a multiple of 4), the new
+// list's keys and visited flags, the rows.
+struct SearchLds {
+    uint32_t keys, flags, rows, row_stride, cols, bytes;  // byte offsets; columns of a row at a time
+};
+__host__ __device__ inline SearchLds search_lds(uint32_t dim, uint32_t L, int rows, uint32_t row_bytes) {
+    SearchLds s;
+    const uint32_t q = rows == kRowsDirect ? 0u : (dim + 3u) / 4u * 16u;
+    s.keys = q;
+    s.flags = s.keys + L * 8u;
+    s.rows = (s.flags + L * 4u + 15u) & ~15u;
+    s.cols = 0;
+    s.row_stride = 0;
+    if (rows == kRowsSq8x16) {
+        s.cols = dim < row_bytes ? (dim + 15u) / 16u * 16u : row_bytes;
+        s.row_stride = s.cols + 16u;
+    } else if (rows != kRowsDirect) {
+        s.cols = dim < row_bytes / 4u ? dim : row_bytes / 4u;
+        // the row lanes read different banks: 4 words past a multiple of 4, or an odd number of words
+        s.row_stride = rows == kRowsF32x4 ? s.cols * 4u + 16u : (s.cols | 1u) * 4u;
     }
+    s.bytes = s.rows + 64u * s.row_stride;
     return s;
 }
 
-// kMode 0: f32 rows, scalar; 1: f32 rows, float4 loads; 2: SQ8 rows, scalar;
-// 3: SQ8 rows, 16 codes per load.
-template <int kMode>
-__device__ __forceinline__ float row_dist(const GraphSearchParams &p, uint32_t id, const float *q) {
-    if constexpr (kMode < 2) return l2_ordered<kMode == 1>(p.data + (uint64_t)id * p.dim, q, p.dim);
-    else return sq8_l2_ordered<kMode == 3>(p.codes + (uint64_t)id * p.padded_dim, p.scales[id], q, p.dim);
+// Per-lane distance from memory (kRowsDirect).
+__device__ __forceinline__ float direct_dist(const GraphSearchParams &p, uint32_t id, const float *q) {
+    if (p.data) {
+        const float *x = p.data + (uint64_t)id * p.dim;
+        if (p.dim % 4u == 0u && ((reinterpret_cast<uintptr_t>(p.data) | reinterpret_cast<uintptr_t>(p.queries)) & 15u) == 0u)
+            return l2_ordered<true>(x, q, p.dim);
+        return l2_ordered<false>(x, q, p.dim);
+    }
+    const int8_t *c = p.codes + (uint64_t)id * p.padded_dim;
+    const float sc = p.scales[id];
+    float s = 0.0f;
+    for (uint32_t i = 0; i < p.dim; ++i) s = l2_step(s, __fmul_rn(sc, (float)c[i]), q[i]);
+    return s;
 }
 
-template <int kMode>
-__global__ __launch_bounds__(kThreads) void graph_search_kernel(GraphSearchParams p) {
-    __shared__ WaveLists lists[kSearchWaves];
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t slot = blockIdx.x * kSearchWaves + wave;
-    WaveLists &w = lists[wave];
-    uint32_t *tags = p.tags + (uint64_t)slot * p.num_points;
+// E: list entries per lane (entry e * 64 + lane), L <= 64 * E.
+template <int kRows, int E>
+__global__ __launch_bounds__(64) void graph_search_kernel(GraphSearchParams p) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    const SearchLds o = search_lds(p.dim, p.L, kRows, p.row_bytes);
+    float *ql = reinterpret_cast<float *>(lds);
+    uint64_t *skey = reinterpret_cast<uint64_t *>(lds + o.keys);
+    uint32_t *sflag = reinterpret_cast<uint32_t *>(lds + o.flags);
+    unsigned char *rows = lds + o.rows;
+    const uint32_t lane = threadIdx.x;
+    const uint32_t words = search_words(p.num_points);
+    uint32_t *seen = p.visited + (uint64_t)blockIdx.x * words;
+    uint32_t pre_node = 0, pre_id = 0, pre_cnt = 0;  // neighbour ids read ahead
+    bool pre = false;
 
-    for (uint32_t qi = slot; qi < p.num_queries; qi += p.slots) {
+    // neighbours [s0, s0 + 64) of a node (the ids past its degree are read too, where the row has them)
+    auto load_ids = [&](uint32_t node, uint32_t s0) -> uint32_t {
+        return s0 + lane < p.row_stride ? p.targets[(uint64_t)node * p.row_stride + s0 + lane] : 0xFFFFFFFFu;
+    };
+
+    // Marks the valid lanes' ids as visited; returns the lanes that were not
+    // yet, with their distance in d.  next: a node whose ids are read ahead.
+    auto score = [&](uint64_t valid, uint32_t id, const float *q, float &d, bool ahead, uint32_t next) -> uint64_t {
+        const bool mine = (valid >> lane) & 1ull;
+        uint32_t old = ~0u;
+        if (mine) old = atomicOr(&seen[id >> 5], 1u << (id & 31u));
+        uint64_t fresh = 0;
+        float s = 0.0f, sc = 0.0f;
+        auto claim = [&]() { fresh = __ballot(mine && !((old >> (id & 31u)) & 1u)); };
+        auto read_ahead = [&]() {
+            if (ahead) {
+                pre_cnt = p.counts[next];
+                pre_id = load_ids(next, 0u);
+            }
+        };
+        if constexpr (kRows == kRowsDirect) {
+            read_ahead();
+            claim();
+            if ((fresh >> lane) & 1ull) s = direct_dist(p, id, q);
+        } else {
+            using lds_ptr = __attribute__((address_space(3))) void *;
+            if (kRows == kRowsSq8x16 && mine) sc = p.scales[id];
+            const uint64_t at = kRows == kRowsSq8x16
+                                    ? reinterpret_cast<uint64_t>(p.codes) + (uint64_t)id * p.padded_dim
+                                    : reinterpret_cast<uint64_t>(p.data) + (uint64_t)id * p.dim * 4u;
+            for (uint32_t c0 = 0; c0 < p.dim; c0 += o.cols) {
+                const uint32_t n = p.dim - c0 < o.cols ? p.dim - c0 : o.cols;
+                uint64_t m = c0 ? fresh : valid;
+                wave_lds_sync();
+                __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): what lies in the rows' place has been read
+                // Row j's address by two lane reads.  Nearly all rows of a
+                // full chunk: an unrolled loop over all 64 (the others read
+                // row 0), half the instructions of walking the mask.
+                auto each = [&](auto &&dma) {
+                    auto one = [&](uint32_t j) {
+                        dma(reinterpret_cast<const unsigned char *>(readlane64(at, j)) + c0 * (kRows == kRowsSq8x16 ? 1u : 4u),
+                            rows + j * o.row_stride);
+                    };
+                    if (__popcll(m) > 48) {
+#pragma unroll 8
+                        for (uint32_t j = 0; j < 64u; ++j) one(j);
+                    } else {
+                        for (; m; m &= m - 1ull) one((uint32_t)__builtin_ctzll(m));
+                    }
+                };
+                if constexpr (kRows == kRowsF32) {
+                    each([&](const unsigned char *src, unsigned char *dst) {
+                        for (uint32_t t = 0; t < n; t += 64u)
+                            if (t + lane < n)
+                                __builtin_amdgcn_global_load_lds(static_cast<const void *>(src + (t + lane) * 4u),
+                                                                 (lds_ptr)(dst + t * 4u), 4, 0, 0);
+                    });
+                } else {
+                    // 16 bytes per lane, a row of at most 512 bytes by 32 lanes
+                    const uint32_t bytes = kRows == kRowsF32x4 ? n * 4u : (n + 15u) & ~15u;
+                    if (lane * 16u < bytes)
+                        each([&](const unsigned char *src, unsigned char *dst) {
+                            __builtin_amdgcn_global_load_lds(static_cast<const void *>(src + lane * 16u), (lds_ptr)dst, 16,
+                                                             0, 0);
+                        });
+                }
+                if (c0 == 0) read_ahead();
+                __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the rows are in LDS
+                wave_lds_sync();
+                if (c0 == 0) {
+                    claim();
+                    if (!fresh) break;
+                }
+                const unsigned char *row = rows + lane * o.row_stride;
+                if constexpr (kRows == kRowsF32x4) {
+                    const float4 *x4 = reinterpret_cast<const float4 *>(row);
+                    const float4 *q4 = reinterpret_cast<const float4 *>(ql + c0);
+#pragma unroll 4
+                    for (uint32_t t = 0; t < n / 4u; ++t) {
+                        const float4 a = x4[t], b = q4[t];
+                        s = l2_step(s, a.x, b.x);
+                        s = l2_step(s, a.y, b.y);
+                        s = l2_step(s, a.z, b.z);
+                        s = l2_step(s, a.w, b.w);
+                    }
+                } else if constexpr (kRows == kRowsF32) {
+                    const float *x = reinterpret_cast<const float *>(row);
+#pragma unroll 8
+                    for (uint32_t t = 0; t < n; ++t) s = l2_step(s, x[t], ql[c0 + t]);
+                } else {
+                    const int8_t *c = reinterpret_cast<const int8_t *>(row);
+                    const uint4 *c16 = reinterpret_cast<const uint4 *>(row);
+                    for (uint32_t t = 0; t < n / 16u; ++t) {
+                        const uint4 w = c16[t];
+                        const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) {
+                            const float4 b = *reinterpret_cast<const float4 *>(ql + c0 + 16u * t + 4u * g);
+                            const float bq[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+                            for (int e = 0; e < 4; ++e)
+                                s = l2_step(s, __fmul_rn(sc, (float)(int8_t)(ww[g] >> (8 * e))), bq[e]);
+                        }
+                    }
+                    for (uint32_t t = n & ~15u; t < n; ++t) s = l2_step(s, __fmul_rn(sc, (float)c[t]), ql[c0 + t]);
+                }
+            }
+        }
+        d = s;
+        return fresh;
+    };
+
+    for (uint32_t qi = blockIdx.x; qi < p.num_queries; qi += p.slots) {
         const float *q = p.queries + (uint64_t)qi * p.dim;
-        const uint32_t epoch = qi + 1u;
-        uint32_t buf = 0, size = 1, cur = 0, cmps = 0;
-        if (lane == 0) {
-            tags[p.start] = epoch;
-            const float d0 = row_dist<kMode>(p, p.start, q);
-            w.key[0][0] = ((uint64_t)__float_as_uint(d0) << 32) | p.start;
-            w.visited[0][0] = 0u;
-        }
-        wave_lds_sync();
-        while (cur < size) {
-            // closest_notvisited: expand the entry at the cursor
-            const uint32_t node = (uint32_t)w.key[buf][cur];
+        if (qi != blockIdx.x) {
+            // the slot's next query: its visited bits are cleared by its own wave
+            uint4 *v = reinterpret_cast<uint4 *>(seen);
+            for (uint32_t i = lane; i < words / 4u; i += 64u) v[i] = make_uint4(0u, 0u, 0u, 0u);
+            __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): cleared before the atomics
             wave_lds_sync();
-            if (lane == 0) w.visited[buf][cur] = 1u;
-            const uint32_t cnt = p.counts[node];
+        }
+        if constexpr (kRows != kRowsDirect) {
+            wave_lds_sync();
+            for (uint32_t i = lane; i < p.dim; i += 64u) ql[i] = q[i];
+            wave_lds_sync();
+        }
+        uint64_t lk[E];  // the list, ascending; kNoKey past its size
+        bool open[E];    // entries not yet expanded
+        uint32_t size = 1, cmps = 0;
+        float d0;
+        pre = false;
+        score(1ull, p.start, q, d0, false, 0u);
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            lk[e] = e == 0 && lane == 0 ? ((uint64_t)__float_as_uint(d0) << 32) | p.start : kNoKey;
+            open[e] = e == 0 && lane == 0;
+        }
+        // the first open entry (closest_notvisited)
+        auto first_open = [&](uint32_t &node) -> bool {
+            bool any = false;
+#pragma unroll
+            for (int e = E - 1; e >= 0; --e) {
+                const uint64_t m = __ballot(open[e]);
+                if (m) {
+                    node = readlane32((uint32_t)lk[e], (uint32_t)__builtin_ctzll(m));
+                    any = true;
+                }
+            }
+            return any;
+        };
+        uint32_t node = 0;
+        while (first_open(node)) {
+#pragma unroll
+            for (int e = 0; e < E; ++e) open[e] = open[e] && (uint32_t)lk[e] != node;
+            uint32_t next = 0;
+            const bool ahead = first_open(next);
+            const bool have = pre && pre_node == node;
+            const uint32_t cnt = readlane32(have ? pre_cnt : p.counts[node], 0u);
+            uint32_t ids = have ? pre_id : load_ids(node, 0u);
+            pre = ahead;
+            pre_node = next;
             const uint32_t deg = cnt < p.row_stride ? cnt : p.row_stride;
-            const uint32_t *row = p.targets + (uint64_t)node * p.row_stride;
-            for (uint32_t s0 = 0; s0 < deg; s0 += 64) {
-                const uint32_t s = s0 + lane;
-                const uint32_t id = s < deg ? row[s] : 0xFFFFFFFFu;
-                bool fresh = id < p.num_points;
-                if (fresh) fresh = atomicExch(&tags[id], epoch) != epoch;
-                uint64_t key = kNoKey;
-                if (fresh) {
-                    const float d = row_dist<kMode>(p, id, q);
-                    key = ((uint64_t)__float_as_uint(d) << 32) | id;
+            for (uint32_t s0 = 0; s0 < deg; s0 += 64u) {
+                if (s0) ids = load_ids(node, s0);
+                const uint64_t valid = __ballot(s0 + lane < deg && ids < p.num_points);
+                if (!valid) {
+                    if (s0 == 0u) pre = false;  // nothing was read ahead
+                    continue;
                 }
-                const uint32_t nf = (uint32_t)__popcll(__ballot(fresh));
-                if (nf == 0) continue;
-                cmps += nf;
-                key = wave_sort64(key, lane);
-                w.fresh[lane] = key;
+                const uint32_t id = (valid >> lane) & 1ull ? ids : 0u;
+                float d;
+                const uint64_t fresh = score(valid, id, q, d, s0 == 0u && ahead, next);
+                cmps += (uint32_t)__popcll(fresh);
+                const uint64_t key = ((uint64_t)__float_as_uint(d) << 32) | id;
+                // a full list takes what is better than its last entry
+                uint64_t last = kNoKey;
+                if (size == p.L) {
+#pragma unroll
+                    for (int e = 0; e < E; ++e)
+                        if ((p.L - 1u) / 64u == (uint32_t)e) last = readlane64(lk[e], (p.L - 1u) & 63u);
+                }
+                const uint64_t pass = fresh & __ballot(key < last || size < p.L);
+                if (!pass) continue;
+                // each passing key's place among them and in the list, each
+                // entry's shift, by counting
+                uint32_t place = 0, shift[E];
+#pragma unroll
+                for (int e = 0; e < E; ++e) shift[e] = 0;
+                uint64_t m = pass;
+                while (m) {
+                    const uint32_t j = (uint32_t)__builtin_ctzll(m);
+                    m &= m - 1ull;
+                    const uint64_t kj = readlane64(key, j);
+                    uint32_t under = 0;
+#pragma unroll
+                    for (int e = 0; e < E; ++e) {
+                        const bool lt = lk[e] < kj;
+                        under += (uint32_t)__popcll(__ballot(lt));
+                        shift[e] += lt ? 0u : 1u;
+                    }
+                    place += kj < key ? 1u : 0u;
+                    place += lane == j ? under : 0u;
+                }
                 wave_lds_sync();
-                const uint32_t nb = buf ^ 1u;
-                const uint32_t new_size = size + nf < p.L ? size + nf : p.L;
-                for (uint32_t i = lane; i < size; i += 64) {
-                    const uint64_t k = w.key[buf][i];
-                    const uint32_t pos = i + rank_in(w.fresh, nf, k);
-                    if (pos < p.L) {
-                        w.key[nb][pos] = k;
-                        w.visited[nb][pos] = w.visited[buf][i];
+#pragma unroll
+                for (int e = 0; e < E; ++e) {
+                    const uint32_t at = (uint32_t)e * 64u + lane, pos = at + shift[e];
+                    if (at < size && pos < p.L) {
+                        skey[pos] = lk[e];
+                        sflag[pos] = open[e] ? 1u : 0u;
                     }
                 }
-                if (lane < nf) {
-                    const uint32_t pos = lane + rank_in(w.key[buf], size, key);
-                    if (pos < p.L) {
-                        w.key[nb][pos] = key;
-                        w.visited[nb][pos] = 0u;
+                if (((pass >> lane) & 1ull) && place < p.L) {
+                    skey[place] = key;
+                    sflag[place] = 1u;
+                }
+                const uint32_t grown = size + (uint32_t)__popcll(pass);
+                size = grown < p.L ? grown : p.L;
+                wave_lds_sync();
+#pragma unroll
+                for (int e = 0; e < E; ++e) {
+                    const uint32_t at = (uint32_t)e * 64u + lane;
+                    lk[e] = kNoKey;
+                    open[e] = false;
+                    if (at < size) {
+                        lk[e] = skey[at];
+                        open[e] = sflag[at] != 0u;
                     }
                 }
-                wave_lds_sync();
-                buf = nb;
-                size = new_size;
             }
-            // the cursor: first entry not yet expanded
-            wave_lds_sync();
-            cur = size;
-            for (uint32_t c = 0; c < size; c += 64) {
-                const uint32_t i = c + lane;
-                const uint64_t open = __ballot(i < size && w.visited[buf][i] == 0u);
-                if (open) {
-                    cur = c + (uint32_t)__ffsll((unsigned long long)open) - 1u;
-                    break;
-                }
-            }
+            if (deg == 0u) pre = false;
         }
-        for (uint32_t i = lane; i < p.K; i += 64) {
-            const uint64_t k = i < size ? w.key[buf][i] : kNoKey;
-            p.out_ids[(uint64_t)qi * p.K + i] = i < size ? (uint32_t)k : 0xFFFFFFFFu;
-            if (p.out_dists) p.out_dists[(uint64_t)qi * p.K + i] = i < size ? __uint_as_float((uint32_t)(k >> 32)) : 0.0f;
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const uint32_t i = (uint32_t)e * 64u + lane;
+            if (i < p.K) {
+                p.out_ids[(uint64_t)qi * p.K + i] = i < size ? (uint32_t)lk[e] : 0xFFFFFFFFu;
+                if (p.out_dists)
+                    p.out_dists[(uint64_t)qi * p.K + i] = i < size ? __uint_as_float((uint32_t)(lk[e] >> 32)) : 0.0f;
+            }
         }
         if (p.out_cmps && lane == 0) p.out_cmps[qi] = cmps;
-        wave_lds_sync();
     }
 }
 
-__global__ void zero_tags(uint32_t *tags, uint64_t n) {
+__global__ void zero_words(uint4 *v, uint64_t n) {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
-        tags[i] = 0u;
+        v[i] = make_uint4(0u, 0u, 0u, 0u);
+}
+
+template <int kRows>
+int launch_rows(const GraphSearchParams &p, hipStream_t stream) {
+    const uint32_t bytes = search_lds(p.dim, p.L, kRows, p.row_bytes).bytes;
+    auto go = [&](auto kernel) -> int {
+        if (ensure_lds_limit(reinterpret_cast<const void *>(kernel), (int)bytes)) return -1;
+        hipLaunchKernelGGL(kernel, dim3(p.slots), dim3(64), bytes, stream, p);
+        return hipGetLastError() == hipSuccess ? 0 : -1;
+    };
+    if (p.L <= 64) return go(graph_search_kernel<kRows, 1>);
+    if (p.L <= 128) return go(graph_search_kernel<kRows, 2>);
+    return go(graph_search_kernel<kRows, 4>);
 }
 
 }  // namespace
 
 uint32_t search_slots(uint32_t num_points, uint32_t num_queries) {
-    // at most 1 GiB of tags and 4096 slots, at least one workgroup
-    const uint64_t by_mem = (1ull << 30) / (4ull * (num_points ? num_points : 1));
+    // at most 1 GiB of visited bits and 4096 slots, at least one
+    const uint64_t by_mem = (1ull << 30) / (4ull * search_words(num_points));
     uint64_t s = num_queries < 4096u ? num_queries : 4096u;
     if (s > by_mem) s = by_mem;
-    s = (s + kSearchWaves - 1) / kSearchWaves * kSearchWaves;
-    return (uint32_t)(s < kSearchWaves ? kSearchWaves : s);
+    return (uint32_t)(s < 1 ? 1 : s);
 }
 
-int launch_graph_search(const GraphSearchParams &p, hipStream_t stream) {
-    const uint64_t ntags = (uint64_t)p.slots * p.num_points;
-    uint64_t zg = (ntags + 255) / 256;
-    zg = zg < 1 ? 1 : (zg > 8192 ? 8192 : zg);
-    hipLaunchKernelGGL(zero_tags, dim3((uint32_t)zg), dim3(256), 0, stream, p.tags, ntags);
-    const dim3 grid(p.slots / kSearchWaves);
+int launch_graph_search(const GraphSearchParams &params, hipStream_t stream) {
+    GraphSearchParams p = params;
+    // A row's bytes in LDS at a time: 512 (four waves per CU) when every
+    // query has a SIMD to itself and only its own latency counts, 256 (twice
+    // the waves) when waves must hide each other's.
+    p.row_bytes = p.num_queries <= 1024u ? 512u : 256u;
+    const uint64_t n = (uint64_t)p.slots * search_words(p.num_points) / 4u;
+    uint64_t zg = (n + 255) / 256;
+    zg = zg < 1 ? 1 : (zg > 2048 ? 2048 : zg);
+    hipLaunchKernelGGL(zero_words, dim3((uint32_t)zg), dim3(256), 0, stream, reinterpret_cast<uint4 *>(p.visited), n);
+    auto aligned = [](const void *x) { return (reinterpret_cast<uintptr_t>(x) & 15u) == 0u; };
+    if (p.dim > kStagedMaxDim) return launch_rows<kRowsDirect>(p, stream);
     if (p.data) {
-        const bool vec4 = p.dim % 4 == 0 && reinterpret_cast<uintptr_t>(p.data) % 16 == 0 &&
-                          reinterpret_cast<uintptr_t>(p.queries) % 16 == 0;
-        if (vec4) hipLaunchKernelGGL(graph_search_kernel<1>, grid, dim3(kThreads), 0, stream, p);
-        else hipLaunchKernelGGL(graph_search_kernel<0>, grid, dim3(kThreads), 0, stream, p);
-    } else {
-        const bool vec16 = p.dim % 16 == 0 && p.padded_dim % 16 == 0 &&
-                           reinterpret_cast<uintptr_t>(p.codes) % 16 == 0 &&
-                           reinterpret_cast<uintptr_t>(p.queries) % 16 == 0;
-        if (vec16) hipLaunchKernelGGL(graph_search_kernel<3>, grid, dim3(kThreads), 0, stream, p);
-        else hipLaunchKernelGGL(graph_search_kernel<2>, grid, dim3(kThreads), 0, stream, p);
+        if (p.dim % 4u == 0u && aligned(p.data)) return launch_rows<kRowsF32x4>(p, stream);
+        return launch_rows<kRowsF32>(p, stream);
     }
-    return hipGetLastError() == hipSuccess ? 0 : -1;
+    if (p.padded_dim % 16u == 0u && aligned(p.codes)) return launch_rows<kRowsSq8x16>(p, stream);
+    return launch_rows<kRowsDirect>(p, stream);
 }
 
 }  // namespace tessa

@@ -7,8 +7,7 @@
 
 namespace tessa {
 
-constexpr uint32_t kSearchMaxL = 256;   // search list capacity held in LDS
-constexpr uint32_t kSearchWaves = 4;    // waves (query slots) per workgroup
+constexpr uint32_t kSearchMaxL = 256;   // search list capacity: four entries per lane
 
 struct GraphSearchParams {
     const float *data;        // num_points x dim, or null with SQ8 rows
@@ -28,11 +27,14 @@ struct GraphSearchParams {
     uint32_t *out_ids;        // num_queries x K (0xFFFFFFFF past the list)
     float *out_dists;         // num_queries x K, or null
     uint32_t *out_cmps;       // num_queries, or null
-    uint32_t *tags;           // slots x num_points visited tags (query index + 1)
-    uint32_t slots;           // a multiple of kSearchWaves
+    uint32_t *visited;        // slots x search_words(num_points) visited bits, 16-byte aligned
+    uint32_t slots;           // queries at a time, one wave each
+    uint32_t row_bytes;       // of a row staged in LDS at a time (set by the launch)
 };
 
-// Query slots for a call: each slot owns num_points tags of scratch.
+// Words of visited bits per slot (a multiple of 4).
+__host__ __device__ inline uint32_t search_words(uint32_t num_points) { return (num_points / 128u + 1u) * 4u; }
+// Query slots for a call.
 uint32_t search_slots(uint32_t num_points, uint32_t num_queries);
 int launch_graph_search(const GraphSearchParams &p, hipStream_t stream);
 

@@ -2466,8 +2466,8 @@ static tessa_status graph_search_impl(const float *data, const int8_t *codes, co
     if (st.code) return st;
     tessa::GraphSearchParams p{};
     p.slots = tessa::search_slots(num_points, num_queries);
-    st = grow(&ws->search_tags, &ws->search_tags_capacity, (uint64_t)p.slots * num_points, sizeof(uint32_t),
-              "search visited tags");
+    st = grow(&ws->search_tags, &ws->search_tags_capacity, (uint64_t)p.slots * tessa::search_words(num_points),
+              sizeof(uint32_t), "search visited bits");
     if (st.code) return st;
     p.data = data;
     p.codes = codes;
@@ -2486,7 +2486,7 @@ static tessa_status graph_search_impl(const float *data, const int8_t *codes, co
     p.out_ids = out_ids;
     p.out_dists = out_dists;
     p.out_cmps = out_cmps;
-    p.tags = ws->search_tags;
+    p.visited = ws->search_tags;
     if (tessa::launch_graph_search(p, s) != 0) return make_status(TESSA_ERR_HIP, 0, "graph search launch failed");
     return ok_status();
 }

@@ -1,0 +1,90 @@
+"""Greedy search where its row staging changes: the width of a staged piece
+(128 floats or 512 codes, half that above 1,024 queries), rows of odd widths and
+unaligned sets, list lengths at register edges, degrees around a wave, a slot's
+second query.  Bar: bit-identical to the oracle."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_helpers import require_gpu
+from shear_amd import graph as G
+from shear_amd import tessa as T
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    return require_gpu()
+
+
+def _graph(rng, n, stride):
+    t = rng.integers(0, n + 2, (n, stride)).astype(np.uint32)  # some ids past the set
+    c = rng.integers(0, stride + 2, n).astype(np.uint32)        # some counts past the row
+    return t, c
+
+
+def _run(gpu, orc, x, q, t, c, L, K, data=None):
+    f = G.greedy_search_sq8 if isinstance(data, T.Sq8Matrix) else G.greedy_search
+    ids, d, cmps = f(torch.from_numpy(x).to(gpu) if data is None else data, torch.from_numpy(t.view(np.int32)).to(gpu),
+                     torch.from_numpy(c.view(np.int32)).to(gpu), 3, torch.from_numpy(q).to(gpu), L, K)
+    torch.cuda.synchronize()
+    wi, wd, wc = orc.greedy_search(x, t, c, 3, q, L, K)
+    assert np.array_equal(ids.cpu().numpy().view(np.uint32), wi)
+    assert np.array_equal(d.cpu().numpy().view(np.uint32), np.asarray(wd).view(np.uint32))
+    assert np.array_equal(cmps.cpu().numpy().view(np.uint32), wc)
+
+
+@pytest.mark.parametrize("dim", [1, 4, 63, 64, 124, 127, 128, 129, 132, 256, 260, 513, 2048, 2052])
+@pytest.mark.parametrize("L,stride,nq", [(16, 65, 5), (65, 130, 5)])
+def test_row_widths(gpu, orc, dim, L, stride, nq):
+    rng = np.random.default_rng(dim + L)
+    x = rng.standard_normal((400, dim)).astype(np.float32)
+    q = rng.standard_normal((nq, dim)).astype(np.float32)
+    t, c = _graph(rng, 400, stride)
+    _run(gpu, orc, x, q, t, c, L, 7)
+
+
+@pytest.mark.parametrize("L", [1, 2, 63, 64, 65, 128, 129, 256])
+@pytest.mark.parametrize("stride", [1, 63, 64, 200])
+def test_list_lengths_and_degrees(gpu, orc, L, stride):
+    rng = np.random.default_rng(L * 7 + stride)
+    x = rng.integers(-3, 4, (900, 8)).astype(np.float32)  # many equal distances
+    q = rng.integers(-3, 4, (9, 8)).astype(np.float32)
+    t, c = _graph(rng, 900, stride)
+    _run(gpu, orc, x, q, t, c, L, min(L, 20))
+
+
+@pytest.mark.parametrize("nq", [1025, 4100])
+def test_many_queries(gpu, orc, nq):
+    # above 1,024: half-width pieces; above 4,096: a slot's wave clears its visited bits for a second query
+    rng = np.random.default_rng(nq)
+    x = rng.standard_normal((300, 132)).astype(np.float32)
+    q = rng.standard_normal((nq, 132)).astype(np.float32)
+    t, c = _graph(rng, 300, 20)
+    _run(gpu, orc, x, q, t, c, 12, 5)
+
+
+def test_unaligned_rows(gpu, orc):
+    rng = np.random.default_rng(8)
+    x = rng.standard_normal((500, 128)).astype(np.float32)
+    q = rng.standard_normal((6, 128)).astype(np.float32)
+    t, c = _graph(rng, 500, 40)
+    flat = torch.empty(500 * 128 + 1, device=gpu)
+    flat[1:] = torch.from_numpy(x.reshape(-1)).to(gpu)
+    _run(gpu, orc, x, q, t, c, 30, 10, data=flat[1:].view(500, 128))
+
+
+@pytest.mark.parametrize("dim,shift", [(16, 0), (100, 0), (512, 0), (528, 0), (1000, 0), (100, 4)])
+def test_sq8_rows(gpu, orc, dim, shift):
+    rng = np.random.default_rng(dim)
+    x = rng.standard_normal((400, dim)).astype(np.float32)
+    q = rng.standard_normal((7, dim)).astype(np.float32)
+    t, c = _graph(rng, 400, 66)
+    m = T.quantize_sq_int8_matrix(torch.from_numpy(x).to(gpu))
+    if shift:  # codes that do not start on 16 bytes
+        flat = torch.empty(m.codes.numel() + shift, dtype=torch.int8, device=gpu)
+        flat[shift:] = m.codes.view(-1)
+        m = T.Sq8Matrix(flat[shift:].view(m.codes.shape), m.scales, m.norms, m.dim)
+    deq = m.codes.cpu().numpy()[:, :dim].astype(np.float32) * m.scales.cpu().numpy()[:, None]
+    _run(gpu, orc, deq, q, t, c, 24, 9, data=m)

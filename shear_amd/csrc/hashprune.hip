@@ -190,48 +190,78 @@ __global__ void hp_scatter_kernel(const uint4 *rec, uint64_t count, uint32_t num
     }
 }
 
-// Register bitonic sort of P = 64*E elements, element q*64 + lane in lane
-// `lane`'s slot q, by (hash, key).
-template <int E>
-__device__ __forceinline__ void reg_bitonic(uint32_t (&h)[E], uint64_t (&k)[E], uint32_t lane) {
-    auto less = [](uint32_t ha, uint64_t ka, uint32_t hb, uint64_t kb) {
-        return ha < hb || (ha == hb && ka < kb);
-    };
+template <int kCtrl>
+__device__ __forceinline__ uint32_t dpp_mov(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, kCtrl, 0xf, 0xf, false);
+}
+// The value of lane ^ j (j a power of two, known at compile time): data moves
+// inside a row of 16 lanes cost no LDS operation.
+template <uint32_t j>
+__device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
+    if constexpr (j == 1u) return dpp_mov<0xb1>(v);                 // quad_perm [1,0,3,2]
+    else if constexpr (j == 2u) return dpp_mov<0x4e>(v);            // quad_perm [2,3,0,1]
+    else if constexpr (j == 4u) return dpp_mov<0x141>(dpp_mov<0x1b>(v));  // half mirror (^7) of quad_perm [3,2,1,0] (^3)
+    else if constexpr (j == 8u) return dpp_mov<0x128>(v);           // rotation of a row by 8
+    else return __shfl_xor(v, (int)j);
+}
+
+// Ascending bitonic sort of 64 * E values, value q * 64 + lane in register q.
+template <int E, uint32_t kk, uint32_t j>
+__device__ __forceinline__ void sort_step(uint32_t (&x)[E], uint32_t lane) {
+    if constexpr (j >= 64u) {
 #pragma unroll
-    for (uint32_t kk = 2; kk <= 64u * E; kk <<= 1) {
+        for (int q = 0; q < E; ++q) {
+            constexpr int jq = (int)(j / 64u);
+            if ((q & jq) != 0) continue;
+            const bool up = (((uint32_t)q * 64u) & kk) == 0u;  // kk > 64 here
+            const uint32_t a = x[q], b = x[q | jq], lo = a < b ? a : b, hi = a < b ? b : a;
+            x[q] = up ? lo : hi;
+            x[q | jq] = up ? hi : lo;
+        }
+    } else {
 #pragma unroll
-        for (uint32_t j = kk >> 1; j > 0; j >>= 1) {
-            if (j >= 64) {
-                const uint32_t jq = j / 64;
-#pragma unroll
-                for (int q = 0; q < E; ++q) {
-                    if ((q & jq) != 0) continue;
-                    const int l = q | jq;
-                    const bool up = (((uint32_t)q * 64u + lane) & kk) == 0;
-                    const bool sw = up ? less(h[l], k[l], h[q], k[q]) : less(h[q], k[q], h[l], k[l]);
-                    const uint32_t th = h[q];
-                    const uint64_t tk = k[q];
-                    h[q] = sw ? h[l] : h[q];
-                    k[q] = sw ? k[l] : k[q];
-                    h[l] = sw ? th : h[l];
-                    k[l] = sw ? tk : k[l];
-                }
-            } else {
-#pragma unroll
-                for (int q = 0; q < E; ++q) {
-                    const uint32_t ph = __shfl_xor(h[q], (int)j);
-                    const uint32_t plo = __shfl_xor((uint32_t)k[q], (int)j);
-                    const uint32_t phi = __shfl_xor((uint32_t)(k[q] >> 32), (int)j);
-                    const uint64_t pk = ((uint64_t)phi << 32) | plo;
-                    const bool up = (((uint32_t)q * 64u + lane) & kk) == 0;
-                    const bool want_min = ((lane & j) == 0) == up;
-                    const bool take = want_min ? less(ph, pk, h[q], k[q]) : less(h[q], k[q], ph, pk);
-                    h[q] = take ? ph : h[q];
-                    k[q] = take ? pk : k[q];
-                }
-            }
+        for (int q = 0; q < E; ++q) {
+            const uint32_t o = lane_xor<j>(x[q]);
+            const bool up = (((uint32_t)q * 64u + lane) & kk) == 0u;
+            const bool low = ((lane & j) == 0u) == up;
+            const uint32_t lo = x[q] < o ? x[q] : o, hi = x[q] < o ? o : x[q];
+            x[q] = low ? lo : hi;
         }
     }
+    if constexpr (j > 1u) sort_step<E, kk, j / 2u>(x, lane);
+}
+template <int E, uint32_t kk = 2u>
+__device__ __forceinline__ void sort_values(uint32_t (&x)[E], uint32_t lane) {
+    sort_step<E, kk, kk / 2u>(x, lane);
+    if constexpr (kk < 64u * E) sort_values<E, kk * 2u>(x, lane);
+}
+
+// A reservoir's slots in ascending hash order (the hashes are distinct): one
+// word per slot, hash and position, is sorted, then the keys are fetched from
+// their positions.  h: the hash, 0xffffffff for an unused slot (after the used
+// ones); k: the key.
+template <int E>
+__device__ __forceinline__ void sort_slots(uint32_t (&h)[E], uint64_t (&k)[E], uint32_t lane) {
+    uint32_t x[E];
+#pragma unroll
+    for (int q = 0; q < E; ++q) x[q] = h[q] > 0xffffu ? 0xffffffffu : (h[q] << 8) | ((uint32_t)q * 64u + lane);
+    sort_values<E>(x, lane);
+    uint64_t r[E];
+#pragma unroll
+    for (int q = 0; q < E; ++q) {
+        const uint32_t from = x[q] & 63u, reg = (x[q] >> 6) & 3u;
+        uint32_t lo = 0, hi = 0;
+#pragma unroll
+        for (int p = 0; p < E; ++p) {
+            const uint32_t l = __shfl((uint32_t)k[p], (int)from), m = __shfl((uint32_t)(k[p] >> 32), (int)from);
+            lo = reg == (uint32_t)p ? l : lo;
+            hi = reg == (uint32_t)p ? m : hi;
+        }
+        r[q] = ((uint64_t)hi << 32) | lo;
+        h[q] = x[q] == 0xffffffffu ? 0xffffffffu : x[q] >> 8;
+    }
+#pragma unroll
+    for (int q = 0; q < E; ++q) k[q] = r[q];
 }
 
 // ---- segment mode: records left where the emitter put them ------------------
@@ -875,7 +905,10 @@ SegWs seg_ws_layout(void *base, uint64_t nseg, uint32_t num_points) {
 }
 
 // One wave per point: its slots sorted by hash (a reservoir's hashes are
-// distinct, so the order is the reference's emit order, ascending hash).
+// distinct, so the order is the reference's emit order, ascending hash).  The
+// sort's exchanges bound it while they carried hash and key through LDS
+// permutes: 524,288 points of 64 slots 378 us, one word through row moves 147
+// (4.6 TB/s).
 template <int ER>
 __global__ __launch_bounds__(kHpThreads) void hp_export_kernel(const uint64_t *slot_keys, const uint16_t *slot_hash,
                                                                const uint32_t *slot_count, uint32_t num_points,
@@ -894,7 +927,7 @@ __global__ __launch_bounds__(kHpThreads) void hp_export_kernel(const uint64_t *s
             h[q] = e < c ? (uint32_t)slot_hash[base + e] : 0xffffffffu;
             k[q] = e < c ? slot_keys[base + e] : ~0ull;
         }
-        reg_bitonic<ER>(h, k, lane);
+        sort_slots<ER>(h, k, lane);
 #pragma unroll
         for (int q = 0; q < ER; ++q) {
             const uint32_t e = (uint32_t)q * 64u + lane;
@@ -1041,7 +1074,7 @@ __global__ __launch_bounds__(kHpThreads) void hp_export_rhalf_kernel(
                 }
             }
         }
-        reg_bitonic<ER>(h, k, lane);
+        sort_slots<ER>(h, k, lane);
 #pragma unroll
         for (int q = 0; q < ER; ++q) {
             const uint32_t e = (uint32_t)q * 64u + lane;

@@ -874,7 +874,7 @@ def hashprune_leg(rec, count, num_points, stream, steps, warmup, check=True, l_m
         f"{np.mean(ms_seg):.3f} ms (without mutual repeats {np.mean(ms[True][1]):.3f}), records "
         f"{np.mean(ms_rec):.3f} ms, identical {same}")
     return {
-        "kernels": "hp_seg_keys + radix sort + run-length encode + scan + hp_seg_gather + hp_merge_stream_kernel",
+        "kernels": "hp_seg_keys + radix sort + run-length encode + scan + hp_seg_gather + hp_merge_kernel",
         "records": int(count),
         "records_without_mutual_repeats": int(kept[True]),
         "segments": int(nseg),

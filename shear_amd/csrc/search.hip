@@ -38,7 +38,9 @@
 //    all in flight together with the visited bits' atomics (the rows of
 //    neighbours that turn out visited are read for nothing); one lane then
 //    sums one row from LDS.  Each lane reading its own row from memory, 64
-//    lines per load and a few loads in flight, took some 16 us an expansion;
+//    lines per load and a few loads in flight, took some 16 us an expansion.
+//    Waiting for the atomics ahead of the rows costs 1,000 queries of L = 64
+//    960 us instead of 792;
 //  * the neighbour ids of the entry that is next in line so far are read
 //    meanwhile;
 //  * the list is held in registers, and a pass over the new neighbours that can
@@ -154,7 +156,11 @@ __global__ __launch_bounds__(64) void graph_search_kernel(GraphSearchParams p) {
         if (mine) old = atomicOr(&seen[id >> 5], 1u << (id & 31u));
         uint64_t fresh = 0;
         float s = 0.0f, sc = 0.0f;
-        auto claim = [&]() { fresh = __ballot(mine && !((old >> (id & 31u)) & 1u)); };
+        auto claim = [&]() {
+            uint32_t was = old;
+            asm volatile("" : "+v"(was));  // keeps the test, and the wait for the atomic, here: behind the rows' loads
+            fresh = __ballot(mine && !((was >> (id & 31u)) & 1u));
+        };
         auto read_ahead = [&]() {
             if (ahead) {
                 pre_cnt = p.counts[next];
@@ -168,12 +174,10 @@ __global__ __launch_bounds__(64) void graph_search_kernel(GraphSearchParams p) {
         } else {
             using lds_ptr = __attribute__((address_space(3))) void *;
             if (kRows == kRowsSq8x16 && mine) sc = p.scales[id];
-            const uint64_t at = kRows == kRowsSq8x16
-                                    ? reinterpret_cast<uint64_t>(p.codes) + (uint64_t)id * p.padded_dim
-                                    : reinterpret_cast<uint64_t>(p.data) + (uint64_t)id * p.dim * 4u;
-            for (uint32_t c0 = 0; c0 < p.dim; c0 += o.cols) {
-                const uint32_t n = p.dim - c0 < o.cols ? p.dim - c0 : o.cols;
-                uint64_t m = c0 ? fresh : valid;
+            uint64_t at = kRows == kRowsSq8x16 ? reinterpret_cast<uint64_t>(p.codes) + (uint64_t)id * p.padded_dim
+                                               : reinterpret_cast<uint64_t>(p.data) + (uint64_t)id * p.dim * 4u;
+            asm volatile("" : "+v"(at));  // all 64 lanes have their address before the branch that reads it by lane
+            auto stage = [&](uint32_t c0, uint32_t n, uint64_t m) __attribute__((always_inline)) {
                 wave_lds_sync();
                 __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): what lies in the rows' place has been read
                 // Row j's address by two lane reads.  Nearly all rows of a
@@ -207,13 +211,12 @@ __global__ __launch_bounds__(64) void graph_search_kernel(GraphSearchParams p) {
                                                              0, 0);
                         });
                 }
-                if (c0 == 0) read_ahead();
+            };
+            auto landed = [&]() __attribute__((always_inline)) {
                 __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the rows are in LDS
                 wave_lds_sync();
-                if (c0 == 0) {
-                    claim();
-                    if (!fresh) break;
-                }
+            };
+            auto sum = [&](uint32_t c0, uint32_t n) __attribute__((always_inline)) {
                 const unsigned char *row = rows + lane * o.row_stride;
                 if constexpr (kRows == kRowsF32x4) {
                     const float4 *x4 = reinterpret_cast<const float4 *>(row);
@@ -246,6 +249,22 @@ __global__ __launch_bounds__(64) void graph_search_kernel(GraphSearchParams p) {
                         }
                     }
                     for (uint32_t t = n & ~15u; t < n; ++t) s = l2_step(s, __fmul_rn(sc, (float)c[t]), ql[c0 + t]);
+                }
+            };
+            // The first piece outside the loop: inside it, the compiler waits
+            // for the atomic ahead of the loop, and the rows' loads after it.
+            const uint32_t n0 = p.dim < o.cols ? p.dim : o.cols;
+            stage(0u, n0, valid);
+            read_ahead();
+            landed();
+            claim();
+            if (fresh) {
+                sum(0u, n0);
+                for (uint32_t c0 = o.cols; c0 < p.dim; c0 += o.cols) {
+                    const uint32_t n = p.dim - c0 < o.cols ? p.dim - c0 : o.cols;
+                    stage(c0, n, fresh);
+                    landed();
+                    sum(c0, n);
                 }
             }
         }

@@ -437,7 +437,8 @@ int launch_ks(const D0AssignParams &p, hipStream_t stream) {
     // Short lists (the builds replicate to two leaders) are ranked without a
     // branch, so the ranking can stand between the MFMAs: 64 rows per wave.  At
     // 1,000 leaders 1.08-1.3x faster over 5,000 to 400,000 rows and 50 to 1,024
-    // columns; at 40 leaders up to 4 us slower (one wave per SIMD has the rows'
+    // columns, at 129 to 480 leaders 1.02-1.6x (30,000 to 2M rows, two or three
+    // per row); at 40 leaders up to 4 us slower (one wave per SIMD has the rows'
     // load to itself for only two tiles).  2F - 1 instructions per value make
     // longer lists the slower ones that way.
     const bool wide = p.leaders > kWideLeaders;

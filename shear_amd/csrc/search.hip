@@ -80,12 +80,12 @@ __device__ __forceinline__ float l2_step(float s, float x, float q) {
     return __fadd_rn(s, __fmul_rn(t, t));
 }
 
-// Where the rows come from.
+// What the rows are.
 enum SearchRows : int {
     kRowsF32x4 = 0,   // f32, 16-byte aligned rows of dim % 4 == 0
     kRowsF32 = 1,     // f32, any
     kRowsSq8x16 = 2,  // SQ8, 16-byte aligned rows
-    kRowsDirect = 3   // read by each lane from memory: wider than kStagedMaxDim, or SQ8 unaligned
+    kRowsSq8 = 3      // SQ8, any (not staged)
 };
 
 // LDS of a query's wave: the query (dim floats, to a multiple of 4), the new
@@ -93,18 +93,22 @@ enum SearchRows : int {
 struct SearchLds {
     uint32_t keys, flags, rows, row_stride, cols, bytes;  // byte offsets; columns of a row at a time
 };
-__host__ __device__ inline SearchLds search_lds(uint32_t dim, uint32_t L, int rows, uint32_t row_bytes) {
+__host__ __device__ inline SearchLds search_lds(uint32_t dim, uint32_t L, int rows, bool staged, uint32_t row_bytes) {
     SearchLds s;
-    const uint32_t q = rows == kRowsDirect ? 0u : (dim + 3u) / 4u * 16u;
+    const uint32_t q = staged ? (dim + 3u) / 4u * 16u : 0u;
     s.keys = q;
     s.flags = s.keys + L * 8u;
     s.rows = (s.flags + L * 4u + 15u) & ~15u;
     s.cols = 0;
     s.row_stride = 0;
+    if (!staged) {
+        s.bytes = s.rows;
+        return s;
+    }
     if (rows == kRowsSq8x16) {
         s.cols = dim < row_bytes ? (dim + 15u) / 16u * 16u : row_bytes;
         s.row_stride = s.cols + 16u;
-    } else if (rows != kRowsDirect) {
+    } else {
         s.cols = dim < row_bytes / 4u ? dim : row_bytes / 4u;
         // the row lanes read different banks: 4 words past a multiple of 4, or an odd number of words
         s.row_stride = rows == kRowsF32x4 ? s.cols * 4u + 16u : (s.cols | 1u) * 4u;
@@ -113,26 +117,74 @@ __host__ __device__ inline SearchLds search_lds(uint32_t dim, uint32_t L, int ro
     return s;
 }
 
-// Per-lane distance from memory (kRowsDirect).
-__device__ __forceinline__ float direct_dist(const GraphSearchParams &p, uint32_t id, const float *q) {
-    if (p.data) {
-        const float *x = p.data + (uint64_t)id * p.dim;
-        if (p.dim % 4u == 0u && ((reinterpret_cast<uintptr_t>(p.data) | reinterpret_cast<uintptr_t>(p.queries)) & 15u) == 0u)
-            return l2_ordered<true>(x, q, p.dim);
-        return l2_ordered<false>(x, q, p.dim);
-    }
-    const int8_t *c = p.codes + (uint64_t)id * p.padded_dim;
-    const float sc = p.scales[id];
+// A lane's distance, the row read from memory (rows not staged).  64 lanes read
+// 64 rows, so what a lane has in flight is what hides the latency, and a line
+// read in several turns is gone from the L1 in between: 64 bytes of the row at a
+// time, SQ8 rows (whose conversions take longer) with the next 64 on their way.
+// The query is the wave's own and comes by scalar loads, which the rows' loads
+// do not wait for.  1,000 queries, 40,000 points, L = 64: 4,096 SQ8 columns 11.2
+// ms (32 bytes at a time and the query by vector loads 11.5, a byte at a time 4.5
+// times that); 2,049 f32 columns, rows at any float's address, 7.2 ms (a float at
+// a time 52).
+template <int kRows>
+__device__ __forceinline__ float direct_dist(const GraphSearchParams &p, uint32_t id, const float *query) {
+    const auto *q = (const __attribute__((address_space(4))) float *)(uintptr_t)query;
     float s = 0.0f;
-    for (uint32_t i = 0; i < p.dim; ++i) s = l2_step(s, __fmul_rn(sc, (float)c[i]), q[i]);
+    uint32_t i = 0;
+    if constexpr (kRows == kRowsF32) {
+        typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));
+        const float *x = p.data + (uint64_t)id * p.dim;
+        for (; i + 16u <= p.dim; i += 16u) {
+            f4 a[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a[e] = reinterpret_cast<const f4 *>(x + i)[e];
+#pragma unroll
+            for (int e = 0; e < 16; ++e) s = l2_step(s, a[e / 4][e % 4], q[i + e]);
+        }
+        for (; i < p.dim; ++i) s = l2_step(s, x[i], q[i]);
+    } else {
+        const int8_t *c = p.codes + (uint64_t)id * p.padded_dim;
+        const float sc = p.scales[id];
+        if constexpr (kRows == kRowsSq8x16) {
+            auto step = [&](const uint4 &w, uint32_t at) {
+                const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    s = l2_step(s, __fmul_rn(sc, (float)(int8_t)(ww[e / 4] >> (8 * (e % 4)))), q[at + e]);
+            };
+            const uint4 *c16 = reinterpret_cast<const uint4 *>(c);
+            const uint32_t turns = p.dim / 64u;
+            if (turns) {
+                uint4 w[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) w[e] = c16[e];
+                for (uint32_t t = 0; t < turns; ++t) {
+                    uint4 next[4];
+                    const uint32_t u = t + 1u < turns ? t + 1u : t;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) next[e] = c16[4u * u + e];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) step(w[e], 64u * t + 16u * e);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) w[e] = next[e];
+                }
+                i = turns * 64u;
+            }
+            for (; i + 16u <= p.dim; i += 16u) step(c16[i / 16u], i);
+        }
+        for (; i < p.dim; ++i) s = l2_step(s, __fmul_rn(sc, (float)c[i]), q[i]);
+    }
     return s;
 }
 
-// E: list entries per lane (entry e * 64 + lane), L <= 64 * E.
-template <int kRows, int E>
-__global__ __launch_bounds__(64) void graph_search_kernel(GraphSearchParams p) {
+// E: list entries per lane (entry e * 64 + lane), L <= 64 * E.  Rows not staged:
+// registers for the four waves per SIMD that 4,096 slots make (with 130 instead
+// of 128 registers, 20,000 queries over 768 SQ8 columns took 17.2 ms, not 14.2).
+template <int kRows, bool kStaged, int E>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kStaged ? 1 : 4))) void graph_search_kernel(
+    GraphSearchParams p) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    const SearchLds o = search_lds(p.dim, p.L, kRows, p.row_bytes);
+    const SearchLds o = search_lds(p.dim, p.L, kRows, kStaged, p.row_bytes);
     float *ql = reinterpret_cast<float *>(lds);
     uint64_t *skey = reinterpret_cast<uint64_t *>(lds + o.keys);
     uint32_t *sflag = reinterpret_cast<uint32_t *>(lds + o.flags);
@@ -167,10 +219,10 @@ __global__ __launch_bounds__(64) void graph_search_kernel(GraphSearchParams p) {
                 pre_id = load_ids(next, 0u);
             }
         };
-        if constexpr (kRows == kRowsDirect) {
+        if constexpr (!kStaged) {
             read_ahead();
             claim();
-            if ((fresh >> lane) & 1ull) s = direct_dist(p, id, q);
+            if ((fresh >> lane) & 1ull) s = direct_dist<kRows>(p, id, q);
         } else {
             using lds_ptr = __attribute__((address_space(3))) void *;
             if (kRows == kRowsSq8x16 && mine) sc = p.scales[id];
@@ -281,7 +333,7 @@ __global__ __launch_bounds__(64) void graph_search_kernel(GraphSearchParams p) {
             __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): cleared before the atomics
             wave_lds_sync();
         }
-        if constexpr (kRows != kRowsDirect) {
+        if constexpr (kStaged) {
             wave_lds_sync();
             for (uint32_t i = lane; i < p.dim; i += 64u) ql[i] = q[i];
             wave_lds_sync();
@@ -410,17 +462,17 @@ __global__ void zero_words(uint4 *v, uint64_t n) {
         v[i] = make_uint4(0u, 0u, 0u, 0u);
 }
 
-template <int kRows>
+template <int kRows, bool kStaged>
 int launch_rows(const GraphSearchParams &p, hipStream_t stream) {
-    const uint32_t bytes = search_lds(p.dim, p.L, kRows, p.row_bytes).bytes;
+    const uint32_t bytes = search_lds(p.dim, p.L, kRows, kStaged, p.row_bytes).bytes;
     auto go = [&](auto kernel) -> int {
         if (ensure_lds_limit(reinterpret_cast<const void *>(kernel), (int)bytes)) return -1;
         hipLaunchKernelGGL(kernel, dim3(p.slots), dim3(64), bytes, stream, p);
         return hipGetLastError() == hipSuccess ? 0 : -1;
     };
-    if (p.L <= 64) return go(graph_search_kernel<kRows, 1>);
-    if (p.L <= 128) return go(graph_search_kernel<kRows, 2>);
-    return go(graph_search_kernel<kRows, 4>);
+    if (p.L <= 64) return go(graph_search_kernel<kRows, kStaged, 1>);
+    if (p.L <= 128) return go(graph_search_kernel<kRows, kStaged, 2>);
+    return go(graph_search_kernel<kRows, kStaged, 4>);
 }
 
 }  // namespace
@@ -444,13 +496,15 @@ int launch_graph_search(const GraphSearchParams &params, hipStream_t stream) {
     zg = zg < 1 ? 1 : (zg > 2048 ? 2048 : zg);
     hipLaunchKernelGGL(zero_words, dim3((uint32_t)zg), dim3(256), 0, stream, reinterpret_cast<uint4 *>(p.visited), n);
     auto aligned = [](const void *x) { return (reinterpret_cast<uintptr_t>(x) & 15u) == 0u; };
-    if (p.dim > kStagedMaxDim) return launch_rows<kRowsDirect>(p, stream);
+    const bool staged = p.dim <= kStagedMaxDim;
     if (p.data) {
-        if (p.dim % 4u == 0u && aligned(p.data)) return launch_rows<kRowsF32x4>(p, stream);
-        return launch_rows<kRowsF32>(p, stream);
+        if (!staged) return launch_rows<kRowsF32, false>(p, stream);
+        return p.dim % 4u == 0u && aligned(p.data) ? launch_rows<kRowsF32x4, true>(p, stream)
+                                                   : launch_rows<kRowsF32, true>(p, stream);
     }
-    if (p.padded_dim % 16u == 0u && aligned(p.codes)) return launch_rows<kRowsSq8x16>(p, stream);
-    return launch_rows<kRowsDirect>(p, stream);
+    if (p.padded_dim % 16u == 0u && aligned(p.codes))
+        return staged ? launch_rows<kRowsSq8x16, true>(p, stream) : launch_rows<kRowsSq8x16, false>(p, stream);
+    return launch_rows<kRowsSq8, false>(p, stream);
 }
 
 }  // namespace tessa

@@ -75,7 +75,8 @@ def test_unaligned_rows(gpu, orc):
     _run(gpu, orc, x, q, t, c, 30, 10, data=flat[1:].view(500, 128))
 
 
-@pytest.mark.parametrize("dim,shift", [(16, 0), (100, 0), (512, 0), (528, 0), (1000, 0), (100, 4)])
+@pytest.mark.parametrize("dim,shift", [(16, 0), (100, 0), (512, 0), (528, 0), (1000, 0), (100, 4), (2049, 0), (2112, 0),
+                                       (2127, 0), (4096, 0), (2100, 4)])
 def test_sq8_rows(gpu, orc, dim, shift):
     rng = np.random.default_rng(dim)
     x = rng.standard_normal((400, dim)).astype(np.float32)
@@ -88,3 +89,29 @@ def test_sq8_rows(gpu, orc, dim, shift):
         m = T.Sq8Matrix(flat[shift:].view(m.codes.shape), m.scales, m.norms, m.dim)
     deq = m.codes.cpu().numpy()[:, :dim].astype(np.float32) * m.scales.cpu().numpy()[:, None]
     _run(gpu, orc, deq, q, t, c, 24, 9, data=m)
+
+
+def test_wide_sq8_rows_are_read_in_wide_loads(gpu):
+    # A quarter of the f32 rows' bytes and five instructions a code instead of three: no more than twice the f32
+    # search's time at any width.  Read a byte at a time, they took four times as long.
+    rng = np.random.default_rng(1)
+    n, dim = 4000, 2560
+    x = torch.from_numpy(rng.standard_normal((n, dim)).astype(np.float32)).to(gpu)
+    q = torch.from_numpy(rng.standard_normal((500, dim)).astype(np.float32)).to(gpu)
+    t = torch.from_numpy(rng.integers(0, n, (n, 48)).astype(np.int32)).to(gpu)
+    c = torch.full((n,), 48, dtype=torch.int32, device=gpu)
+    m = T.quantize_sq_int8_matrix(x)
+
+    def ms(f, data):
+        best = []
+        for _ in range(4):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            f(data, t, c, 3, q, 32, 5)
+            b.record()
+            b.synchronize()
+            best.append(a.elapsed_time(b))
+        return min(best)
+
+    a, b = ms(G.greedy_search_sq8, m), ms(G.greedy_search, x)
+    assert a < 2.0 * b, (a, b)

@@ -34,13 +34,11 @@
 // The kernel waits, it does not compute: one wavefront per query and a chain of
 // about L + 10 expansions, each of them neighbour ids -> visited bits -> rows ->
 // distances -> list.  What it does about that:
-//  * a chunk's rows go to LDS by LDS-DMA, whole rows by consecutive lanes and
-//    all in flight together with the visited bits' atomics (the rows of
-//    neighbours that turn out visited are read for nothing); one lane then
-//    sums one row from LDS.  Each lane reading its own row from memory, 64
-//    lines per load and a few loads in flight, took some 16 us an expansion.
-//    Waiting for the atomics ahead of the rows costs 1,000 queries of L = 64
-//    960 us instead of 792;
+//  * each lane reads its own row with 64 bytes or more in flight (direct_dist);
+//    wide rows of few queries go to LDS instead (launch_graph_search: the rule
+//    and both sides), by LDS-DMA, whole pieces by consecutive lanes and all in
+//    flight together with the visited bits' atomics (the rows of neighbours that
+//    turn out visited are read for nothing); one lane then sums one row from LDS;
 //  * the neighbour ids of the entry that is next in line so far are read
 //    meanwhile;
 //  * the list is held in registers, and a pass over the new neighbours that can
@@ -48,9 +46,10 @@
 //  * the visited set is one bit per point (25 KB per query at 200,000 points,
 //    in L2) instead of a 4-byte tag: no 0.14 ms to clear 800 MB, and 32 times
 //    the queries at a time on a set whose tags fill the scratch limit.
-// 1,000 queries, 200,000 x 128: L = 64 1,652 -> 929 us, L = 128 4,187 -> 2,380;
-// 3,000 queries, 150,000 x 200: 4,531 -> 3,075; 64 queries over SQ8 rows,
-// 100,000 x 256: 1,095 -> 961 (there the conversions bound it).
+// 40,000 points, L = 64, against tags, a list in LDS and 16 to 32 bytes of a row
+// in flight: 1,000 queries of 128 f32 columns 956 -> 530 us, of 768 4,364 -> 2,290;
+// 4,000 queries of 256 SQ8 columns 1,799 -> 1,370; 20,000 of 97 f32 columns 13.0 ->
+// 3.0 ms.
 #include "search_kernels.h"
 #include "tessa_device.h"
 #include "kernel_attr.h"
@@ -60,7 +59,6 @@ namespace tessa {
 namespace {
 
 constexpr uint64_t kNoKey = ~0ull;
-constexpr uint32_t kStagedMaxDim = 2048;    // the query lies in LDS too
 
 __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -82,38 +80,30 @@ __device__ __forceinline__ float l2_step(float s, float x, float q) {
 
 // What the rows are.
 enum SearchRows : int {
-    kRowsF32x4 = 0,   // f32, 16-byte aligned rows of dim % 4 == 0
-    kRowsF32 = 1,     // f32, any
-    kRowsSq8x16 = 2,  // SQ8, 16-byte aligned rows
-    kRowsSq8 = 3      // SQ8, any (not staged)
+    kRowsF32 = 0,     // f32; staged: 16-byte aligned rows of dim % 4 == 0
+    kRowsSq8x16 = 1,  // SQ8, 16-byte aligned rows
+    kRowsSq8 = 2      // SQ8, any (not staged)
 };
 
-// LDS of a query's wave: the query (dim floats, to a multiple of 4), the new
-// list's keys and visited flags, the rows.
+// Staged rows: columns (the query lies in LDS too), and the bytes of a row in
+// LDS at a time (handed to the kernel: as a constant in it, the loops compile to
+// something 3 % slower over f32 rows).
+constexpr uint32_t kStagedMinF32 = 128, kStagedMinSq8 = 257, kStagedMaxDim = 2048;
+constexpr uint32_t kStagedBytes = 512;
+
+// LDS of a query's wave: staged rows' query (dim floats), the new list's keys
+// and visited flags, staged rows.
 struct SearchLds {
     uint32_t keys, flags, rows, row_stride, cols, bytes;  // byte offsets; columns of a row at a time
 };
 __host__ __device__ inline SearchLds search_lds(uint32_t dim, uint32_t L, int rows, bool staged, uint32_t row_bytes) {
     SearchLds s;
-    const uint32_t q = staged ? (dim + 3u) / 4u * 16u : 0u;
-    s.keys = q;
+    s.keys = staged ? (dim + 3u) / 4u * 16u : 0u;
     s.flags = s.keys + L * 8u;
     s.rows = (s.flags + L * 4u + 15u) & ~15u;
-    s.cols = 0;
-    s.row_stride = 0;
-    if (!staged) {
-        s.bytes = s.rows;
-        return s;
-    }
-    if (rows == kRowsSq8x16) {
-        s.cols = dim < row_bytes ? (dim + 15u) / 16u * 16u : row_bytes;
-        s.row_stride = s.cols + 16u;
-    } else {
-        s.cols = dim < row_bytes / 4u ? dim : row_bytes / 4u;
-        // the row lanes read different banks: 4 words past a multiple of 4, or an odd number of words
-        s.row_stride = rows == kRowsF32x4 ? s.cols * 4u + 16u : (s.cols | 1u) * 4u;
-    }
-    s.bytes = s.rows + 64u * s.row_stride;
+    s.cols = rows == kRowsF32 ? (dim < row_bytes / 4u ? dim : row_bytes / 4u) : row_bytes;
+    s.row_stride = (rows == kRowsF32 ? s.cols * 4u : s.cols) + 16u;  // the row lanes read different banks
+    s.bytes = s.rows + (staged ? 64u * s.row_stride : 0u);
     return s;
 }
 
@@ -181,7 +171,7 @@ __device__ __forceinline__ float direct_dist(const GraphSearchParams &p, uint32_
 // registers for the four waves per SIMD that 4,096 slots make (with 130 instead
 // of 128 registers, 20,000 queries over 768 SQ8 columns took 17.2 ms, not 14.2).
 template <int kRows, bool kStaged, int E>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kStaged ? 1 : 4))) void graph_search_kernel(
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kStaged ? 0 : 4))) void graph_search_kernel(
     GraphSearchParams p) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const SearchLds o = search_lds(p.dim, p.L, kRows, kStaged, p.row_bytes);
@@ -247,22 +237,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kStaged ? 1 
                         for (; m; m &= m - 1ull) one((uint32_t)__builtin_ctzll(m));
                     }
                 };
-                if constexpr (kRows == kRowsF32) {
+                // 16 bytes per lane, a row's piece of at most 512 bytes by 32 lanes
+                const uint32_t bytes = kRows == kRowsF32 ? n * 4u : (n + 15u) & ~15u;
+                if (lane * 16u < bytes)
                     each([&](const unsigned char *src, unsigned char *dst) {
-                        for (uint32_t t = 0; t < n; t += 64u)
-                            if (t + lane < n)
-                                __builtin_amdgcn_global_load_lds(static_cast<const void *>(src + (t + lane) * 4u),
-                                                                 (lds_ptr)(dst + t * 4u), 4, 0, 0);
+                        __builtin_amdgcn_global_load_lds(static_cast<const void *>(src + lane * 16u), (lds_ptr)dst, 16, 0,
+                                                         0);
                     });
-                } else {
-                    // 16 bytes per lane, a row of at most 512 bytes by 32 lanes
-                    const uint32_t bytes = kRows == kRowsF32x4 ? n * 4u : (n + 15u) & ~15u;
-                    if (lane * 16u < bytes)
-                        each([&](const unsigned char *src, unsigned char *dst) {
-                            __builtin_amdgcn_global_load_lds(static_cast<const void *>(src + lane * 16u), (lds_ptr)dst, 16,
-                                                             0, 0);
-                        });
-                }
             };
             auto landed = [&]() __attribute__((always_inline)) {
                 __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the rows are in LDS
@@ -270,7 +251,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kStaged ? 1 
             };
             auto sum = [&](uint32_t c0, uint32_t n) __attribute__((always_inline)) {
                 const unsigned char *row = rows + lane * o.row_stride;
-                if constexpr (kRows == kRowsF32x4) {
+                if constexpr (kRows == kRowsF32) {
                     const float4 *x4 = reinterpret_cast<const float4 *>(row);
                     const float4 *q4 = reinterpret_cast<const float4 *>(ql + c0);
 #pragma unroll 4
@@ -281,10 +262,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kStaged ? 1 
                         s = l2_step(s, a.z, b.z);
                         s = l2_step(s, a.w, b.w);
                     }
-                } else if constexpr (kRows == kRowsF32) {
-                    const float *x = reinterpret_cast<const float *>(row);
-#pragma unroll 8
-                    for (uint32_t t = 0; t < n; ++t) s = l2_step(s, x[t], ql[c0 + t]);
                 } else {
                     const int8_t *c = reinterpret_cast<const int8_t *>(row);
                     const uint4 *c16 = reinterpret_cast<const uint4 *>(row);
@@ -487,23 +464,32 @@ uint32_t search_slots(uint32_t num_points, uint32_t num_queries) {
 
 int launch_graph_search(const GraphSearchParams &params, hipStream_t stream) {
     GraphSearchParams p = params;
-    // A row's bytes in LDS at a time: 512 (four waves per CU) when every
-    // query has a SIMD to itself and only its own latency counts, 256 (twice
-    // the waves) when waves must hide each other's.
-    p.row_bytes = p.num_queries <= 1024u ? 512u : 256u;
+    p.row_bytes = kStagedBytes;
     const uint64_t n = (uint64_t)p.slots * search_words(p.num_points) / 4u;
     uint64_t zg = (n + 255) / 256;
     zg = zg < 1 ? 1 : (zg > 2048 ? 2048 : zg);
     hipLaunchKernelGGL(zero_words, dim3((uint32_t)zg), dim3(256), 0, stream, reinterpret_cast<uint4 *>(p.visited), n);
     auto aligned = [](const void *x) { return (reinterpret_cast<uintptr_t>(x) & 15u) == 0u; };
-    const bool staged = p.dim <= kStagedMaxDim;
-    if (p.data) {
-        if (!staged) return launch_rows<kRowsF32, false>(p, stream);
-        return p.dim % 4u == 0u && aligned(p.data) ? launch_rows<kRowsF32x4, true>(p, stream)
-                                                   : launch_rows<kRowsF32, true>(p, stream);
-    }
+    // Rows are staged while every query has a SIMD to itself and all lie on the
+    // chip at once.  Staged over read by the lanes, 16 to 1,000 queries: f32 rows
+    // of 768 to 2,048 columns 0.83-1.08 of the time at L = 64 and 256 (1.05-1.3 at
+    // 16), of 128 to 512 columns 0.89-1.1 with 1,000 queries (0.95 on 5,000,000
+    // points) and 1.0-1.7 with few; SQ8 rows of 257 to 2,048 columns 0.84-1.16.
+    // Narrower f32 rows take 0.98-1.4, narrower SQ8 rows 1.06-1.4.  With more
+    // queries the rows of visited neighbours cost bandwidth and the LDS keeps
+    // waves off the chip: 1,100 to 20,000 queries, in pieces of 512 or 256 bytes,
+    // 0.98-1.8.  Rows at any float's address would be staged 4 bytes at a time:
+    // 2.3-6.
+    auto pays = [&](int rows) {
+        const uint32_t per_cu = 160u * 1024u / search_lds(p.dim, p.L, rows, true, p.row_bytes).bytes;
+        return p.dim >= (rows == kRowsF32 ? kStagedMinF32 : kStagedMinSq8) && p.dim <= kStagedMaxDim && p.slots <= 256u * per_cu;
+    };
+    if (p.data)
+        return p.dim % 4u == 0u && aligned(p.data) && pays(kRowsF32) ? launch_rows<kRowsF32, true>(p, stream)
+                                                                     : launch_rows<kRowsF32, false>(p, stream);
     if (p.padded_dim % 16u == 0u && aligned(p.codes))
-        return staged ? launch_rows<kRowsSq8x16, true>(p, stream) : launch_rows<kRowsSq8x16, false>(p, stream);
+        return pays(kRowsSq8x16) ? launch_rows<kRowsSq8x16, true>(p, stream)
+                                 : launch_rows<kRowsSq8x16, false>(p, stream);
     return launch_rows<kRowsSq8, false>(p, stream);
 }
 

@@ -1,7 +1,8 @@
-"""Greedy search where its row staging changes: the width of a staged piece
-(128 floats or 512 codes, half that above 1,024 queries), rows of odd widths and
-unaligned sets, list lengths at register edges, degrees around a wave, a slot's
-second query.  Bar: bit-identical to the oracle."""
+"""Greedy search where its rows' reading changes: staged in LDS by pieces of 128
+floats or 512 codes (128 to 2,048 aligned f32 columns, 257 to 2,048 SQ8 ones, up
+to four queries per CU) or read by the lanes, rows of odd widths and unaligned sets, list lengths at
+register edges, degrees around a wave, a slot's second query.  Bar: bit-identical
+to the oracle."""
 import numpy as np
 import pytest
 import torch
@@ -35,7 +36,7 @@ def _run(gpu, orc, x, q, t, c, L, K, data=None):
     assert np.array_equal(cmps.cpu().numpy().view(np.uint32), wc)
 
 
-@pytest.mark.parametrize("dim", [1, 4, 63, 64, 124, 127, 128, 129, 132, 256, 260, 513, 2048, 2052])
+@pytest.mark.parametrize("dim", [1, 4, 15, 16, 17, 63, 64, 124, 127, 128, 129, 132, 256, 260, 513, 644, 2048, 2052])
 @pytest.mark.parametrize("L,stride,nq", [(16, 65, 5), (65, 130, 5)])
 def test_row_widths(gpu, orc, dim, L, stride, nq):
     rng = np.random.default_rng(dim + L)
@@ -55,27 +56,35 @@ def test_list_lengths_and_degrees(gpu, orc, L, stride):
     _run(gpu, orc, x, q, t, c, L, min(L, 20))
 
 
-@pytest.mark.parametrize("nq", [1025, 4100])
-def test_many_queries(gpu, orc, nq):
-    # above 1,024: half-width pieces; above 4,096: a slot's wave clears its visited bits for a second query
-    rng = np.random.default_rng(nq)
-    x = rng.standard_normal((300, 132)).astype(np.float32)
-    q = rng.standard_normal((nq, 132)).astype(np.float32)
+# above 1,024: every row is read by the lanes; above 4,096: a slot's wave clears its visited bits
+# for a second query
+@pytest.mark.parametrize("nq", [1024, 1025, 4100])
+@pytest.mark.parametrize("kind,dim", [("f32", 132), ("f32", 129), ("sq8", 272), ("sq8", 400), ("f32", 516), ("sq8", 256)])
+@pytest.mark.parametrize("L", [12, 100, 200])
+def test_many_queries(gpu, orc, nq, kind, dim, L):
+    rng = np.random.default_rng(nq + dim)
+    x = rng.standard_normal((300, dim)).astype(np.float32)
+    q = rng.standard_normal((nq, dim)).astype(np.float32)
     t, c = _graph(rng, 300, 20)
-    _run(gpu, orc, x, q, t, c, 12, 5)
+    data = None
+    if kind == "sq8":
+        data = T.quantize_sq_int8_matrix(torch.from_numpy(x).to(gpu))
+        x = data.codes.cpu().numpy()[:, :dim].astype(np.float32) * data.scales.cpu().numpy()[:, None]
+    _run(gpu, orc, x, q, t, c, L, 5, data=data)
 
 
-def test_unaligned_rows(gpu, orc):
+@pytest.mark.parametrize("dim", [128, 640])
+def test_unaligned_rows(gpu, orc, dim):
     rng = np.random.default_rng(8)
-    x = rng.standard_normal((500, 128)).astype(np.float32)
-    q = rng.standard_normal((6, 128)).astype(np.float32)
+    x = rng.standard_normal((500, dim)).astype(np.float32)
+    q = rng.standard_normal((6, dim)).astype(np.float32)
     t, c = _graph(rng, 500, 40)
-    flat = torch.empty(500 * 128 + 1, device=gpu)
+    flat = torch.empty(500 * dim + 1, device=gpu)
     flat[1:] = torch.from_numpy(x.reshape(-1)).to(gpu)
-    _run(gpu, orc, x, q, t, c, 30, 10, data=flat[1:].view(500, 128))
+    _run(gpu, orc, x, q, t, c, 30, 10, data=flat[1:].view(500, dim))
 
 
-@pytest.mark.parametrize("dim,shift", [(16, 0), (100, 0), (512, 0), (528, 0), (1000, 0), (100, 4), (2049, 0), (2112, 0),
+@pytest.mark.parametrize("dim,shift", [(16, 0), (100, 0), (256, 0), (257, 0), (272, 0), (512, 0), (528, 0), (1000, 0), (100, 4), (2049, 0), (2112, 0),
                                        (2127, 0), (4096, 0), (2100, 4)])
 def test_sq8_rows(gpu, orc, dim, shift):
     rng = np.random.default_rng(dim)
@@ -91,27 +100,35 @@ def test_sq8_rows(gpu, orc, dim, shift):
     _run(gpu, orc, deq, q, t, c, 24, 9, data=m)
 
 
+def _ms(f, data, t, c, q):
+    best = []
+    for _ in range(4):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        f(data, t, c, 3, q, 32, 5)
+        b.record()
+        b.synchronize()
+        best.append(a.elapsed_time(b))
+    return min(best)
+
+
+def _timed_set(gpu, n, dim, nq):
+    rng = np.random.default_rng(1)
+    x, q = (torch.from_numpy(rng.standard_normal((m, dim)).astype(np.float32)).to(gpu) for m in (n, nq))
+    t = torch.from_numpy(rng.integers(0, n, (n, 48)).astype(np.int32)).to(gpu)
+    return x, q, t, torch.full((n,), 48, dtype=torch.int32, device=gpu)
+
+
 def test_wide_sq8_rows_are_read_in_wide_loads(gpu):
     # A quarter of the f32 rows' bytes and five instructions a code instead of three: no more than twice the f32
     # search's time at any width.  Read a byte at a time, they took four times as long.
-    rng = np.random.default_rng(1)
-    n, dim = 4000, 2560
-    x = torch.from_numpy(rng.standard_normal((n, dim)).astype(np.float32)).to(gpu)
-    q = torch.from_numpy(rng.standard_normal((500, dim)).astype(np.float32)).to(gpu)
-    t = torch.from_numpy(rng.integers(0, n, (n, 48)).astype(np.int32)).to(gpu)
-    c = torch.full((n,), 48, dtype=torch.int32, device=gpu)
-    m = T.quantize_sq_int8_matrix(x)
+    x, q, t, c = _timed_set(gpu, 4000, 2560, 500)
+    a, b = _ms(G.greedy_search_sq8, T.quantize_sq_int8_matrix(x), t, c, q), _ms(G.greedy_search, x, t, c, q)
+    assert a < 2.0 * b, (a, b)
 
-    def ms(f, data):
-        best = []
-        for _ in range(4):
-            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            a.record()
-            f(data, t, c, 3, q, 32, 5)
-            b.record()
-            b.synchronize()
-            best.append(a.elapsed_time(b))
-        return min(best)
 
-    a, b = ms(G.greedy_search_sq8, m), ms(G.greedy_search, x)
+def test_odd_widths_are_read_in_wide_loads(gpu):
+    # 129 columns take little longer than 132.  Staged a float at a time they took four times as long (and 1.1-1.3
+    # times what one float per lane and load had taken).
+    a, b = (_ms(G.greedy_search, x, t, c, q) for x, q, t, c in (_timed_set(gpu, 20000, d, 64) for d in (129, 132)))
     assert a < 2.0 * b, (a, b)

@@ -14,9 +14,10 @@
 // distinct hashes, and those are only ever replaced by better ones).  So a
 // batch of records can be merged in any order, which is what makes it a GPU
 // reduction.  Record batches:
-//   1. count records per source (atomics), exclusive scan, scatter the records
-//      grouped by source (the per-source counters return to zero);
-//   2. one wave per source with new records merges its slots with them
+//   1. count records per source (atomics), exclusive scan, list the sources that
+//      have any, scatter the records grouped by source (the per-source counters
+//      return to zero);
+//   2. one wave per listed source merges its slots with its records
 //      (hp_merge_kernel).
 // Segment batches (records left where the emitter wrote them, described by
 // per-source runs) are merged in place by the same kernel.  Between merges
@@ -56,12 +57,35 @@ __device__ __forceinline__ uint32_t wave_excl_scan(uint32_t v, uint32_t lane, ui
     return x - v;
 }
 
+// Record batches: the sources that have records, each one's first grouped
+// record and how many.  Sources of up to `few` records (0: none) are listed from
+// the end of the arrays backwards, the others from the front; count: how many
+// of each, [0] the others, [1] these.
+__host__ __device__ inline uint32_t hp_few_records(uint32_t l_max) { return l_max <= 64u ? 20u : 32u; }
+struct HpRuns {
+    uint32_t *src, *start, *len, *count;
+    uint32_t capacity, few;
+};
+HpRuns record_runs(const HashPruneState &s) {
+    uint32_t *r = s.runs;
+    return HpRuns{r,
+                  r + s.runs_capacity,
+                  r + 2 * s.runs_capacity,
+                  reinterpret_cast<uint32_t *>(s.status + 1),
+                  (uint32_t)s.runs_capacity,
+                  s.rhalf_mode != 0 ? hp_few_records(s.l_max) : 0u};
+}
+
 __global__ void hp_fill_u32(uint32_t *a, uint64_t n, uint32_t v) {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
         a[i] = v;
 }
 
-__global__ void hp_status_init(uint64_t *status) { status[0] = ~0ull; }
+// status[0]: first record with a bad source; status[1]: the lengths of a record batch's two lists.
+__global__ void hp_status_init(uint64_t *status) {
+    status[0] = ~0ull;
+    status[1] = 0ull;
+}
 
 // Lanes of a wave holding the same source as the wave's first active lane
 // share one atomic (the edge stream interleaves one row's outgoing records
@@ -138,27 +162,53 @@ __global__ __launch_bounds__(kScanThreads) void hp_scan_partials(uint32_t *sums,
     if (threadIdx.x == 0) offsets[n] = carry;
 }
 
+// Every source's first grouped record, and the lists of the sources that have
+// any: the merge takes these only (walking all points of a set of 10 M for 1,000
+// records took 2.0 ms, all of the insert with the list 0.1).  Blocks append in
+// any order.
 __global__ __launch_bounds__(kScanThreads) void hp_scan_apply(const uint32_t *bucket, uint32_t n, const uint32_t *sums,
-                                                              uint32_t *offsets) {
-    __shared__ uint32_t ws[kScanThreads / 64];
+                                                              uint32_t *offsets, HpRuns runs) {
+    __shared__ uint32_t ws[kScanThreads / 64], wa[kScanThreads / 64], at0[2];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint32_t base = blockIdx.x * kScanBlock + threadIdx.x * kScanPerThread;
-    uint32_t v[kScanPerThread], t = 0;
+    // listed: sources of more than `few` records in the low half, the others in the high one
+    static_assert(kScanBlock < 0x10000u, "a block's sources fit 16 bits");
+    uint32_t v[kScanPerThread], t = 0, listed = 0;
+    auto list_of = [&](uint32_t records) { return records == 0u ? 0u : records > runs.few ? 1u : 0x10000u; };
 #pragma unroll
     for (int e = 0; e < kScanPerThread; ++e) {
         v[e] = base + e < n ? bucket[base + e] : 0u;
         t += v[e];
+        listed += list_of(v[e]);
     }
-    uint32_t wt;
-    const uint32_t ex = wave_excl_scan(t, lane, wt);
-    if (lane == 0) ws[wave] = wt;
+    uint32_t wt, wl;
+    const uint32_t ex = wave_excl_scan(t, lane, wt), el = wave_excl_scan(listed, lane, wl);
+    if (lane == 0) {
+        ws[wave] = wt;
+        wa[wave] = wl;
+    }
     __syncthreads();
-    uint32_t before = sums[blockIdx.x];
-    for (uint32_t w = 0; w < wave; ++w) before += ws[w];
-    uint32_t run = before + ex;
+    uint32_t before = sums[blockIdx.x], ahead = 0;
+    for (uint32_t w = 0; w < wave; ++w) {
+        before += ws[w];
+        ahead += wa[w];
+    }
+    if (threadIdx.x == kScanThreads - 1u) {
+        const uint32_t all = ahead + wl;
+        at0[0] = (all & 0xffffu) ? atomicAdd(&runs.count[0], all & 0xffffu) : 0u;
+        at0[1] = (all >> 16) ? atomicAdd(&runs.count[1], all >> 16) : 0u;
+    }
+    __syncthreads();
+    uint32_t run = before + ex, many = at0[0] + ((ahead + el) & 0xffffu), few = at0[1] + ((ahead + el) >> 16);
 #pragma unroll
     for (int e = 0; e < kScanPerThread; ++e) {
         if (base + e < n) offsets[base + e] = run;
+        if (v[e] != 0u) {
+            const uint32_t at = v[e] > runs.few ? many++ : runs.capacity - 1u - few++;
+            runs.src[at] = base + e;
+            runs.start[at] = run;
+            runs.len[at] = v[e];
+        }
         run += v[e];
     }
 }
@@ -509,7 +559,7 @@ __device__ __forceinline__ void keep_best(const uint64_t (&k)[R], const uint32_t
 }
 
 // A wave's sources in the stages of its pipeline: the run (source, its sorted
-// segments [start, start + len); num_points: nothing to merge), the segments
+// segments or its records [start, start + len); num_points: nothing to merge), the segments
 // (lane s: segment s, cnt records from first), then the slots and the first
 // batch of records (the lane's record q * 64 + lane of it, q < kHpNew).  Every
 // load is unconditional, from a clamped address: a branch around a load
@@ -532,9 +582,9 @@ struct HpBatch {
 
 struct HpMergeArgs {
     const uint4 *records;   // record batches: grouped by source
-    const uint4 *sorted;    // segments by source; the runs of equal sources
+    const uint4 *sorted;    // segments by source
+    // a source's records (record batches) or its sorted segments: [start, start + len)
     const uint32_t *run_src, *run_start, *run_len, *num_runs;
-    const uint32_t *offsets;  // record batches: records [offsets[src], offsets[src + 1])
     uint32_t num_points, l_max, quota;
     uint64_t *slot_keys;
     uint16_t *slot_hash;
@@ -545,17 +595,13 @@ struct HpMergeArgs {
 __device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
 
 // Run a of na; raw loads, made a run by hp_run_ready once they have arrived.
-template <bool kGrouped>
 __device__ __forceinline__ HpRun hp_run_load(const HpMergeArgs &A, uint32_t a, uint32_t na) {
     const uint32_t i = a < na ? a : na - 1u;
-    if (kGrouped) return HpRun{i, A.offsets[i], A.offsets[i + 1u]};
     return HpRun{A.run_src[i], A.run_start[i], A.run_len[i]};
 }
-template <bool kGrouped>
 __device__ __forceinline__ HpRun hp_run_ready(const HpMergeArgs &A, const HpRun &l, uint32_t a, uint32_t na) {
     HpRun r{uniform(l.src), uniform(l.start), uniform(l.len)};
-    // past the end, a point without records, the run of empty / bad segments
-    const bool none = a >= na || r.src >= A.num_points || (kGrouped && r.len == r.start);
+    const bool none = a >= na || r.src >= A.num_points;  // past the end, the run of empty / bad segments
     if (none) r = HpRun{A.num_points, 0u, 0u};
     return r;
 }
@@ -563,7 +609,7 @@ __device__ __forceinline__ HpRun hp_run_ready(const HpMergeArgs &A, const HpRun 
 // Segments [g0, g0 + 64) of a run; the same two steps.
 template <bool kGrouped>
 __device__ __forceinline__ uint4 hp_segs_load(const HpMergeArgs &A, const HpRun &r, uint32_t g0, uint32_t lane) {
-    if (kGrouped) return make_uint4(r.src, r.start, 0u, r.len - r.start);
+    if (kGrouped) return make_uint4(r.src, r.start, 0u, r.len);
     const uint32_t s = g0 + lane;
     return A.sorted[(uint64_t)r.start + (s < r.len ? s : 0u)];
 }
@@ -773,8 +819,8 @@ __device__ __forceinline__ void wait_loads() {
     __builtin_amdgcn_sched_barrier(0);
 }
 
-// Each wave walks its sources (segment runs, or with kGrouped the points of a
-// record batch grouped by source) with the next source's first batch and
+// Each wave walks its sources (segment runs, or with kGrouped the sources of a
+// record batch) with the next source's first batch and
 // slots, and the one after's run, already in flight.  They are waited for
 // after the merge and before its stores: a wait at their first use, in the
 // next iteration, would also wait for the stores, and for the loads issued
@@ -786,16 +832,16 @@ __global__ __launch_bounds__(kHpThreads) void hp_merge_kernel(HpMergeArgs A) {
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     HpWaveLds &t = lds[wave];
     const uint32_t waves = gridDim.x * kHpWaves;
-    const uint32_t na = kGrouped ? A.num_points : *A.num_runs;
+    const uint32_t na = *A.num_runs;
     uint32_t a = blockIdx.x * kHpWaves + wave;
     if (a >= na) return;
     for (uint32_t i = lane; i < kHpBuckets; i += 64u) t.key[i] = ~0ull;
     wave_lds_order();
     const uint4 *safe = kGrouped ? A.records : A.sorted;
     // stages: slots and batch of source a, segments of the next, run of the one after
-    HpRun raw = hp_run_load<kGrouped>(A, a, na), raw1 = hp_run_load<kGrouped>(A, a + waves, na),
-          raw2 = hp_run_load<kGrouped>(A, a + 2u * waves, na);
-    HpRun run = hp_run_ready<kGrouped>(A, raw, a, na), run1 = hp_run_ready<kGrouped>(A, raw1, a + waves, na);
+    HpRun raw = hp_run_load(A, a, na), raw1 = hp_run_load(A, a + waves, na),
+          raw2 = hp_run_load(A, a + 2u * waves, na);
+    HpRun run = hp_run_ready(A, raw, a, na), run1 = hp_run_ready(A, raw1, a + waves, na);
     uint4 seg = hp_segs_load<kGrouped>(A, run, 0u, lane), seg1 = hp_segs_load<kGrouped>(A, run1, 0u, lane);
     HpSegs segs = hp_segs_ready<kGrouped>(run, seg, 0u, lane);
     HpSlots<ER> slots = hp_slots<ER>(A, run.src, lane);
@@ -804,12 +850,12 @@ __global__ __launch_bounds__(kHpThreads) void hp_merge_kernel(HpMergeArgs A) {
     wait_loads();
     for (; a < na; a += waves) {
         HpSegs segs1 = hp_segs_ready<kGrouped>(run1, seg1, 0u, lane);
-        const HpRun run2 = hp_run_ready<kGrouped>(A, raw2, a + 2u * waves, na);
+        const HpRun run2 = hp_run_ready(A, raw2, a + 2u * waves, na);
         const HpSlots<ER> slots1 = hp_slots<ER>(A, run1.src, lane);
         HpBatch batch1;
         hp_batch(batch1, A.records, safe, segs1, 0u, lane);
         seg1 = hp_segs_load<kGrouped>(A, run2, 0u, lane);
-        raw2 = hp_run_load<kGrouped>(A, a + 3u * waves, na);
+        raw2 = hp_run_load(A, a + 3u * waves, na);
         uint64_t base = 0, rk[ER], g[ER][kRhalfGroup];
         uint32_t rh[ER], c = 0;
         if (run.src < A.num_points) {
@@ -862,6 +908,175 @@ __global__ __launch_bounds__(kHpThreads) void hp_merge_kernel(HpMergeArgs A) {
         segs = segs1;
         slots = slots1;
         batch = batch1;
+    }
+}
+
+// ---- few records of a source, with groups ------------------------------------
+// A record batch's sources of up to hp_few_records records while a backfill
+// policy keeps groups: the records go in one by one, each a hash ballot and an
+// update of one lane's slot and group (a hash's best quota + 1 distinct targets
+// in order), or an append, or in a full reservoir a replacement of its worst
+// slot; only the lanes that changed are written back.  Merging a batch
+// (hp_absorb) finds the groups anew, layer by layer, some 4,000 cycles however
+// few the records.  1,000,000 sources, reservoirs of up to 30 slots, one by one
+// and merged: one record each 446 and 1,138 us, 16 records 1.38 and 1.63 ms, 20
+// 1.66 and 1.76, 24 2.02 and 1.93 (hashes drawn from 4,096); 20 records 1.67 and
+// 2.97 ms, 32 2.61 and 3.47 (from 40).  More slots make a merge dearer: with 128,
+// 32 records 3.60 and 3.65 ms (from 4,096), 3.63 and 6.68 (from 40).
+struct HpFew {
+    uint32_t src, start, len;
+};
+template <int ER>
+struct HpFewData {
+    uint64_t k[ER], g[ER][kRhalfGroup];
+    uint32_t h[ER], c;
+    uint4 rec;
+};
+
+// The run's slots, groups (of a reservoir with a free slot) and records.
+template <int ER>
+__device__ __forceinline__ void hp_few_load(HpFewData<ER> &d, const HpMergeArgs &A, const HpFew &r, uint32_t c,
+                                            uint32_t lane) {
+    const uint64_t base = (uint64_t)r.src * A.l_max;
+    d.c = c;
+    d.rec = A.records[r.start + (lane < r.len ? lane : 0u)];
+#pragma unroll
+    for (int q = 0; q < ER; ++q) {
+        const uint32_t e = (uint32_t)q * 64u + lane, at = e < c ? e : 0u;
+        d.k[q] = A.slot_keys[base + at];
+        d.h[q] = A.slot_hash[base + at];
+        const uint32_t ga = c < A.l_max ? at : 0u;
+#pragma unroll
+        for (uint32_t j = 0; j < kRhalfGroup; ++j) d.g[q][j] = A.grp_keys[(base + ga) * kRhalfGroup + j];
+    }
+}
+
+template <int ER>
+__global__ __launch_bounds__(kHpThreads) void hp_few_kernel(HpMergeArgs A, uint32_t capacity) {
+    static_assert(kRhalfGroup == 3, "a slot and three group keys");
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t waves = gridDim.x * kHpWaves;
+    const uint32_t na = A.num_runs[1];
+    uint32_t a = blockIdx.x * kHpWaves + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    if (a >= na) return;
+    // raw loads; past the end the last run's, used by nobody
+    auto run = [&](uint32_t i) {
+        const uint32_t at = capacity - 1u - (i < na ? i : na - 1u);
+        return HpFew{A.run_src[at], A.run_start[at], A.run_len[at]};
+    };
+    auto ready = [&](const HpFew &r) { return HpFew{uniform(r.src), uniform(r.start), uniform(r.len)}; };
+    // stages: data of run a, count of the next, run of the one after
+    HpFew raw2 = run(a + 2u * waves);
+    HpFew r0 = ready(run(a)), r1 = ready(run(a + waves));
+    HpFewData<ER> d0;
+    hp_few_load<ER>(d0, A, r0, uniform(A.slot_count[r0.src]), lane);
+    uint32_t c1 = A.slot_count[r1.src];
+    wait_loads();
+    for (; a < na; a += waves) {
+        HpFewData<ER> d1;
+        hp_few_load<ER>(d1, A, r1, uniform(c1), lane);
+        const HpFew r2 = ready(raw2);
+        c1 = A.slot_count[r2.src];
+        raw2 = run(a + 3u * waves);
+        const uint64_t base = (uint64_t)r0.src * A.l_max;
+        const uint64_t key = ((uint64_t)total_key(__uint_as_float(d0.rec.w)) << 32) | d0.rec.y;
+        const uint32_t hash = d0.rec.z & 0xffffu;
+        uint64_t rk[ER], g[ER][kRhalfGroup], dirty[ER];
+        uint32_t rh[ER], c = d0.c;
+#pragma unroll
+        for (int q = 0; q < ER; ++q) {
+            const bool live = (uint32_t)q * 64u + lane < c;
+            rk[q] = live ? d0.k[q] : ~0ull;
+            rh[q] = live ? d0.h[q] : 0xffffffffu;
+            dirty[q] = 0;
+#pragma unroll
+            for (uint32_t j = 0; j < kRhalfGroup; ++j) g[q][j] = live && c < A.l_max ? d0.g[q][j] : ~0ull;
+        }
+        for (uint32_t j = 0; j < r0.len; ++j) {
+            const uint64_t k = readlane64(key, j);
+            const uint32_t h = readlane32(hash, j);
+            uint64_t hit[ER], any = 0;
+#pragma unroll
+            for (int q = 0; q < ER; ++q) {
+                hit[q] = ballot64(rh[q] == h);
+                any |= hit[q];
+            }
+            if (!any) {
+                uint32_t place = c;
+                if (c == A.l_max) {
+                    // the worst slot by (distance, target, hash), if the record is better
+                    uint64_t m[ER];
+                    uint32_t worst[3];
+#pragma unroll
+                    for (int q = 0; q < ER; ++q) m[q] = lanes_below(c, q);
+#pragma unroll
+                    for (int w = 0; w < 3; ++w) {
+                        uint32_t v[ER], top = 0;
+#pragma unroll
+                        for (int q = 0; q < ER; ++q) {
+                            v[q] = w == 0 ? (uint32_t)(rk[q] >> 32) : w == 1 ? (uint32_t)rk[q] : rh[q];
+                            const uint32_t x = lane_in(m[q]) ? v[q] : 0u;
+                            top = top > x ? top : x;
+                        }
+                        worst[w] = wave_max_u32(top);
+#pragma unroll
+                        for (int q = 0; q < ER; ++q) m[q] &= ballot64(v[q] == worst[w]);
+                    }
+                    const uint64_t wk = ((uint64_t)worst[0] << 32) | worst[1];
+                    if (k > wk || (k == wk && h > worst[2])) continue;
+#pragma unroll
+                    for (int q = 0; q < ER; ++q)
+                        if (m[q]) place = (uint32_t)q * 64u + (uint32_t)__builtin_ctzll(m[q]);
+                } else {
+                    ++c;
+                }
+#pragma unroll
+                for (int q = 0; q < ER; ++q) {
+                    const uint64_t here = ballot64((uint32_t)q * 64u + lane == place);
+                    dirty[q] |= here;
+                    if (lane_in(here)) {
+                        rk[q] = k;
+                        rh[q] = h;
+#pragma unroll
+                        for (uint32_t i = 0; i < kRhalfGroup; ++i) g[q][i] = ~0ull;
+                    }
+                }
+                continue;
+            }
+#pragma unroll
+            for (int q = 0; q < ER; ++q) {
+                if (!hit[q]) continue;
+                dirty[q] |= hit[q];
+                if (!lane_in(hit[q])) continue;
+                const uint64_t e0 = rk[q], e1 = g[q][0], e2 = g[q][1], e3 = g[q][2];
+                const uint32_t t = (uint32_t)k;
+                const bool s0 = (uint32_t)e0 == t, s1 = (uint32_t)e1 == t, s2 = (uint32_t)e2 == t, s3 = (uint32_t)e3 == t;
+                if ((s0 && e0 <= k) || (s1 && e1 <= k) || (s2 && e2 <= k) || (s3 && e3 <= k)) continue;
+                // without the target's worse key, then with the new one
+                const bool p1 = s0 || s1, p2 = p1 || s2, p3 = p2 || s3;
+                const uint64_t f0 = s0 ? e1 : e0, f1 = p1 ? e2 : e1, f2 = p2 ? e3 : e2, f3 = p3 ? ~0ull : e3;
+                rk[q] = k < f0 ? k : f0;
+                g[q][0] = k < f0 ? f0 : k < f1 ? k : f1;
+                g[q][1] = A.quota < 2u ? ~0ull : k < f1 ? f1 : k < f2 ? k : f2;
+                g[q][2] = A.quota < 3u ? ~0ull : k < f2 ? f2 : k < f3 ? k : f3;
+            }
+        }
+        wait_loads();  // as in the merge: before the stores, which a wait in the next iteration would include
+#pragma unroll
+        for (int q = 0; q < ER; ++q) {
+            if (!dirty[q] || !lane_in(dirty[q])) continue;
+            const uint64_t at = base + (uint32_t)q * 64u + lane;
+            A.slot_keys[at] = rk[q];
+            A.slot_hash[at] = (uint16_t)rh[q];
+            if (c < A.l_max) {
+#pragma unroll
+                for (uint32_t j = 0; j < kRhalfGroup; ++j) A.grp_keys[at * kRhalfGroup + j] = g[q][j];
+            }
+        }
+        if (lane == 0 && c != d0.c) A.slot_count[r0.src] = c;
+        r0 = r1;
+        r1 = r2;
+        d0 = d1;
     }
 }
 
@@ -1088,6 +1303,11 @@ __global__ __launch_bounds__(kHpThreads) void hp_export_rhalf_kernel(
     }
 }
 
+template <int ER>
+void launch_few(const HpMergeArgs &A, uint32_t capacity, uint32_t grid, hipStream_t stream) {
+    hipLaunchKernelGGL(hp_few_kernel<ER>, dim3(grid), dim3(kHpThreads), 0, stream, A, capacity);
+}
+
 template <int ER, bool kGrouped>
 void launch_merge_er(const HpMergeArgs &A, bool rhalf, uint32_t grid, hipStream_t stream) {
     if (rhalf)
@@ -1129,14 +1349,24 @@ int launch_hashprune_insert(HashPruneState &s, const uint4 *records, uint64_t co
     hipLaunchKernelGGL(hp_count_kernel, dim3(grid_for(count, 256, 16384)), dim3(256), 0, stream, records, count, n,
                        s.bucket, s.status);
     const uint32_t nb = (n + kScanBlock - 1) / kScanBlock;
+    const HpRuns runs = record_runs(s);
     hipLaunchKernelGGL(hp_scan_reduce, dim3(nb), dim3(kScanThreads), 0, stream, s.bucket, n, s.block_sums);
     hipLaunchKernelGGL(hp_scan_partials, dim3(1), dim3(kScanThreads), 0, stream, s.block_sums, nb, s.offsets, n);
-    hipLaunchKernelGGL(hp_scan_apply, dim3(nb), dim3(kScanThreads), 0, stream, s.bucket, n, s.block_sums, s.offsets);
+    hipLaunchKernelGGL(hp_scan_apply, dim3(nb), dim3(kScanThreads), 0, stream, s.bucket, n, s.block_sums, s.offsets, runs);
     hipLaunchKernelGGL(hp_scatter_kernel, dim3(grid_for(count, 256, 16384)), dim3(256), 0, stream, records, count, n,
                        s.bucket, s.offsets, s.grouped);
-    const HpMergeArgs A{s.grouped, nullptr, nullptr, nullptr, nullptr, nullptr, s.offsets, n, s.l_max, s.rhalf_quota,
+    const HpMergeArgs A{s.grouped, nullptr, runs.src, runs.start, runs.len, runs.count, n, s.l_max, s.rhalf_quota,
                         s.slot_keys, s.slot_hash, s.slot_count, s.grp_keys};
-    launch_merge<true>(A, s.rhalf_mode != 0, grid_for(n, kHpWaves, kHpMergeGrid), stream);
+    const uint32_t grid = grid_for(count < n ? count : n, kHpWaves, kHpMergeGrid);
+    if (runs.few) {
+        if (s.l_max <= 64)
+            launch_few<1>(A, runs.capacity, grid, stream);
+        else if (s.l_max <= 128)
+            launch_few<2>(A, runs.capacity, grid, stream);
+        else
+            launch_few<4>(A, runs.capacity, grid, stream);
+    }
+    launch_merge<true>(A, s.rhalf_mode != 0, grid, stream);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -1168,7 +1398,7 @@ int launch_hashprune_insert_segments(HashPruneState &s, const uint4 *records, co
         return -1;
     hipLaunchKernelGGL(hp_seg_gather_kernel, dim3(grid_for(nseg, 256, 16384)), dim3(256), 0, stream, segs,
                        w.vals_out, nseg, w.sorted);
-    const HpMergeArgs A{records, w.sorted, w.run_src, w.run_start, w.run_len, w.num_runs, nullptr, n, s.l_max,
+    const HpMergeArgs A{records, w.sorted, w.run_src, w.run_start, w.run_len, w.num_runs, n, s.l_max,
                         s.rhalf_quota, s.slot_keys, s.slot_hash, s.slot_count, s.grp_keys};
     launch_merge<false>(A, s.rhalf_mode != 0, grid_for(nseg, kHpWaves, kHpMergeGrid), stream);
     return hipGetLastError() == hipSuccess ? 0 : -1;

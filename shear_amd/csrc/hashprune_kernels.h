@@ -22,7 +22,9 @@ struct HashPruneState {
     uint64_t block_sums_capacity = 0;
     uint4 *grouped = nullptr;       // the batch's records grouped by source
     uint64_t grouped_capacity = 0;
-    uint64_t *status = nullptr;     // [0] first record with src >= num_points (UINT64_MAX: none)
+    uint32_t *runs = nullptr;       // behind them: the batch's sources, first records, record counts
+    uint64_t runs_capacity = 0;     // min(grouped_capacity, num_points) of each
+    uint64_t *status = nullptr;     // [0] first record with src >= num_points (UINT64_MAX: none), [1] runs
     void *seg_ws = nullptr;          // segment mode workspace (hashprune_segment_workspace_bytes)
     uint64_t seg_ws_bytes = 0;
     // Named R-half backfill (rhalf_mode != 0): per slot the next rhalf_quota

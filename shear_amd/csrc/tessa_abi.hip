@@ -2155,6 +2155,22 @@ tessa_status resolve_backfill(const tessa_hashprune_backfill *bf, uint32_t l_max
     return ok_status();
 }
 
+// Grows the record batches' buffer: the grouped records, then the list of their sources.
+tessa_status reserve_records(tessa::HashPruneState &s, uint64_t count, hipStream_t stream) {
+    if (count <= s.grouped_capacity) return ok_status();
+    TESSA_HIP_TRY(hipStreamSynchronize(stream));
+    if (s.grouped) TESSA_HIP_TRY(hipFree(s.grouped));
+    s.grouped = nullptr;
+    s.grouped_capacity = 0;
+    const uint64_t sources = std::min<uint64_t>(count, s.num_points);
+    tessa_status st = hp_alloc((void **)&s.grouped, count * 16 + sources * 12, "hashprune grouped records");
+    if (st.code) return st;
+    s.grouped_capacity = count;
+    s.runs = reinterpret_cast<uint32_t *>(s.grouped + count);
+    s.runs_capacity = sources;
+    return ok_status();
+}
+
 // The checked shape and policy of a reducer, no memory yet.
 tessa_status hashprune_shape(uint32_t num_points, uint32_t l_max, const tessa_hashprune_backfill *bf,
                              tessa::HashPruneState &s) {
@@ -2284,15 +2300,7 @@ tessa_status tessa_hashprune_insert(tessa_hashprune *hp, const tessa_edge_record
                            (unsigned long long)count);
     auto &s = hp->st;
     hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
-    if (count > s.grouped_capacity) {
-        TESSA_HIP_TRY(hipStreamSynchronize(hs));
-        if (s.grouped) TESSA_HIP_TRY(hipFree(s.grouped));
-        s.grouped = nullptr;
-        s.grouped_capacity = 0;
-        tessa_status st = hp_alloc((void **)&s.grouped, count * 16, "hashprune grouped records");
-        if (st.code) return st;
-        s.grouped_capacity = count;
-    }
+    if (tessa_status st = reserve_records(s, count, hs); st.code) return st;
     if (tessa::launch_hashprune_insert(s, reinterpret_cast<const uint4 *>(records), count, hs) != 0)
         return make_status(TESSA_ERR_HIP, 0, "hashprune insert launch failed");
     uint64_t bad = 0;
@@ -2324,15 +2332,7 @@ tessa_status hashprune_insert_async(tessa_hashprune *hp, const tessa_edge_record
         return make_status(TESSA_ERR_UNSUPPORTED, 0, "hashprune: %llu records in one batch (limit 2^32-2)",
                            (unsigned long long)count);
     auto &s = hp->st;
-    if (count > s.grouped_capacity) {
-        TESSA_HIP_TRY(hipStreamSynchronize(hs));
-        if (s.grouped) TESSA_HIP_TRY(hipFree(s.grouped));
-        s.grouped = nullptr;
-        s.grouped_capacity = 0;
-        tessa_status st = hp_alloc((void **)&s.grouped, count * 16, "hashprune grouped records");
-        if (st.code) return st;
-        s.grouped_capacity = count;
-    }
+    if (tessa_status st = reserve_records(s, count, hs); st.code) return st;
     if (tessa::launch_hashprune_insert(s, reinterpret_cast<const uint4 *>(records), count, hs) != 0)
         return make_status(TESSA_ERR_HIP, 0, "hashprune insert launch failed");
     return ok_status();

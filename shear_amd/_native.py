@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import threading
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "libtessa_hip.so"
@@ -34,6 +35,7 @@ EXEC_EXACT = 1
 EXEC_MFMA = 2
 
 TESSA_OK = 0
+TESSA_ERR_OUT_OF_MEMORY = 5
 
 
 class TessaStatus(C.Structure):
@@ -409,6 +411,33 @@ SIGNATURES = {
 
 _lib = None
 
+# Entry points that take memory from the driver before they start their work:
+# after TESSA_ERR_OUT_OF_MEMORY they may be called again.
+_ALLOCATING = (
+    "tessa_leaf_topk", "tessa_leaf_topk_profiled", "tessa_session_upload_sq8", "tessa_session_leaf_topk",
+    "tessa_session_assign_replay", "tessa_session_run_subtree", "tessa_session_partition_roots",
+    "tessa_session_partition_small_roots", "tessa_emit_edge_records", "tessa_emit_edge_segments",
+    "tessa_emit_edge_segments_unique", "tessa_hashprune_create", "tessa_hashprune_create_backfill",
+    "tessa_hashprune_insert", "tessa_hashprune_insert_segments", "tessa_graph_pack", "tessa_graph_search",
+    "tessa_graph_search_sq8", "tessa_global_d0_assign")
+_retrying = threading.local()
+
+
+def _retry_without_cache(status, fn, args):
+    """The library's memory comes from the driver, outside torch's cache: when
+    the driver has none left, the cache's unused blocks go back to it and the
+    call is made once more."""
+    if status.code != TESSA_ERR_OUT_OF_MEMORY or getattr(_retrying, "on", False):
+        return status
+    import torch
+
+    torch.cuda.empty_cache()
+    _retrying.on = True
+    try:
+        return fn(*args)
+    finally:
+        _retrying.on = False
+
 
 class TessaError(RuntimeError):
     def __init__(self, status: TessaStatus, what: str):
@@ -434,6 +463,8 @@ def load(path: Path | str | None = None):
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
+        if name in _ALLOCATING:
+            fn.errcheck = _retry_without_cache
     if path is None:
         _lib = lib
     return lib

@@ -129,6 +129,15 @@ struct DeviceWorkspace {
 std::mutex g_ws_mutex;
 std::vector<DeviceWorkspace> g_ws;
 
+// hipMalloc; a failure leaves no error behind for the next launch's check (the
+// caller may free memory and call again).
+bool device_alloc(void **ptr, size_t bytes) {
+    if (hipMalloc(ptr, bytes) == hipSuccess) return true;
+    *ptr = nullptr;
+    (void)hipGetLastError();
+    return false;
+}
+
 template <typename T>
 tessa_status grow(T **ptr, uint64_t *cap, uint64_t need, size_t elem_bytes, const char *what) {
     if (*cap >= need) return ok_status();
@@ -139,7 +148,7 @@ tessa_status grow(T **ptr, uint64_t *cap, uint64_t need, size_t elem_bytes, cons
         *cap = 0;
     }
     const uint64_t n = need < 4096 ? 4096 : need;
-    if (hipMalloc((void **)ptr, n * elem_bytes) != hipSuccess)
+    if (!device_alloc((void **)ptr, n * elem_bytes))
         return make_status(TESSA_ERR_OUT_OF_MEMORY, TESSA_OVF_WORKSPACE_BUDGET,
                            "%s allocation of %llu entries failed overflow_flags=0x%llx "
                            "overflow_labels=WORKSPACE_BUDGET",
@@ -764,7 +773,7 @@ tessa_status ensure_scratch(tessa_session *s, size_t bytes) {
         s->scratch = nullptr;
         s->scratch_bytes = 0;
     }
-    if (hipMalloc(&s->scratch, bytes) != hipSuccess)
+    if (!device_alloc(&s->scratch, bytes))
         return make_status(TESSA_ERR_OUT_OF_MEMORY, TESSA_OVF_WORKSPACE_BUDGET,
                            "session scratch of %zu bytes failed overflow_flags=0x%llx overflow_labels=WORKSPACE_BUDGET",
                            bytes, (unsigned long long)TESSA_OVF_WORKSPACE_BUDGET);
@@ -852,9 +861,8 @@ static tessa_status tessa_session_upload_sq8_locked(tessa_session *s, const tess
     s->capture.tasks.clear();
     s->capture.rows.clear();
     const uint64_t rows = host->rows;
-    if (hipMalloc(&s->codes, rows * host->padded_dim) != hipSuccess ||
-        hipMalloc(&s->scales, rows * 4) != hipSuccess || hipMalloc(&s->norms, rows * 4) != hipSuccess ||
-        hipMalloc(&s->gids, rows * 4) != hipSuccess) {
+    if (!device_alloc((void **)&s->codes, rows * host->padded_dim) || !device_alloc((void **)&s->scales, rows * 4) ||
+        !device_alloc((void **)&s->norms, rows * 4) || !device_alloc((void **)&s->gids, rows * 4)) {
         free_sq8(s);
         return make_status(TESSA_ERR_OUT_OF_MEMORY, TESSA_OVF_WORKSPACE_BUDGET,
                            "SQ8 upload of %llu rows failed overflow_flags=0x%llx overflow_labels=WORKSPACE_BUDGET",
@@ -1229,7 +1237,7 @@ static tessa_status tessa_session_run_subtree_locked(tessa_session *s, const tes
         if (s->part) (void)hipFree(s->part);
         s->part = nullptr;
         s->part_bytes = 0;
-        if (hipMalloc(&s->part, L.bytes) != hipSuccess)
+        if (!device_alloc(&s->part, L.bytes))
             return make_status(TESSA_ERR_OUT_OF_MEMORY, TESSA_OVF_WORKSPACE_BUDGET,
                                "Failed to allocate CUDA GPU persistent subtree workspace (HIP, %zu bytes) "
                                "overflow_flags=0x%llx overflow_labels=WORKSPACE_BUDGET",
@@ -1421,7 +1429,7 @@ static tessa_status reserve_partition(tessa_session *s, size_t need) {
     if (s->part) (void)hipFree(s->part);
     s->part = nullptr;
     s->part_bytes = 0;
-    if (hipMalloc(&s->part, need) != hipSuccess)
+    if (!device_alloc(&s->part, need))
         return make_status(TESSA_ERR_OUT_OF_MEMORY, TESSA_OVF_WORKSPACE_BUDGET,
                            "Failed to allocate CUDA GPU persistent subtree workspace (HIP, %zu bytes) "
                            "overflow_flags=0x%llx overflow_labels=WORKSPACE_BUDGET",
@@ -1647,7 +1655,7 @@ tessa_status grow_device(T **p, uint64_t *cap, uint64_t need) {
     *p = nullptr;
     *cap = 0;
     const uint64_t n = need < 1024 ? 1024 : need;
-    if (hipMalloc((void **)p, n * sizeof(T)) != hipSuccess)
+    if (!device_alloc((void **)p, n * sizeof(T)))
         return make_status(TESSA_ERR_OUT_OF_MEMORY, TESSA_OVF_WORKSPACE_BUDGET,
                            "Failed to allocate CUDA GPU persistent subtree output (HIP, %llu entries) "
                            "overflow_flags=0x%llx overflow_labels=WORKSPACE_BUDGET",
@@ -2112,8 +2120,7 @@ uint64_t hashprune_state_layout(tessa::HashPruneState &s, void *base) {
 }
 
 tessa_status hp_alloc(void **ptr, uint64_t bytes, const char *what) {
-    if (hipMalloc(ptr, bytes ? bytes : 16) != hipSuccess) {
-        *ptr = nullptr;
+    if (!device_alloc(ptr, bytes ? bytes : 16)) {
         return make_status(TESSA_ERR_OUT_OF_MEMORY, TESSA_OVF_WORKSPACE_BUDGET,
                            "%s allocation of %llu bytes failed overflow_flags=0x%llx overflow_labels=WORKSPACE_BUDGET",
                            what, (unsigned long long)bytes, (unsigned long long)TESSA_OVF_WORKSPACE_BUDGET);

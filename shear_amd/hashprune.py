@@ -36,6 +36,8 @@ from .tessa import _ptr, _stream_ptr
 
 DEFAULT_L_MAX = 64  # params.rs:3346
 
+MAX_CACHED_BYTES = 8 << 30  # reservoirs of up to this size come from torch's memory (3.7 M points of 64, with groups)
+
 # PiPNNHashPruneBackfillMode names (params.rs:1935-1966) of the named R-half
 # policies, as tessa_hashprune_backfill.mode numbers them
 BACKFILL_MODES = {"off": 0, "rhalf-hash-slot-1": 1, "rhalf-distance-first-q3": 2, "rhalf-soft-tier-q3": 3,
@@ -78,16 +80,32 @@ class HashPruneReducer:
         self._state = self._seg = None
         pol = None if self.backfill is None else C.byref(self.backfill.native())
         with torch.cuda.device(self.device):
-            # the reservoirs lie in torch's memory: made and dropped once per
+            # The reservoirs lie in torch's memory: made and dropped once per
             # build, gigabytes went back to the driver and came again, which
-            # stalled for 0.1-1.4 s now and then
+            # stalled for 0.1-1.4 s now and then.  Larger ones than
+            # MAX_CACHED_BYTES, which torch's cache would keep from everybody
+            # else, and those that torch has no room for are the library's own.
             need = C.c_uint64(0)
             N.check(self._lib.tessa_hashprune_state_bytes(self.num_points, self.l_max, pol, C.byref(need)),
                     "hashprune create")
-            self._state = torch.empty(need.value, dtype=torch.uint8, device=self.device)
-            torch.cuda.current_stream().synchronize()  # what used that memory before; the reducer runs on any stream
-            N.check(self._lib.tessa_hashprune_create_in(self.num_points, self.l_max, pol, self._state.data_ptr(),
-                                                        need.value, C.byref(h)), "hashprune create")
+            self._state = self._torch_memory(need.value) if need.value <= MAX_CACHED_BYTES else None
+            if self._state is not None:
+                # what used that memory before; the reducer runs on any stream
+                torch.cuda.current_stream().synchronize()
+                st = self._lib.tessa_hashprune_create_in(self.num_points, self.l_max, pol, self._state.data_ptr(),
+                                                         need.value, C.byref(h))
+            elif pol is None:
+                st = self._lib.tessa_hashprune_create(self.num_points, self.l_max, C.byref(h))
+            else:
+                st = self._lib.tessa_hashprune_create_backfill(self.num_points, self.l_max, pol, C.byref(h))
+            N.check(st, "hashprune create")
+
+    def _torch_memory(self, nbytes: int):
+        """A block of torch's memory, or None where it has none left."""
+        try:
+            return torch.empty(nbytes, dtype=torch.uint8, device=self.device)
+        except torch.cuda.OutOfMemoryError:
+            return None
 
     def close(self) -> None:
         if self._h:
@@ -141,9 +159,10 @@ class HashPruneReducer:
             N.check(self._lib.tessa_hashprune_lend_segment_memory(self._h, None, 0), "hashprune insert segments")
             self._seg = None
             with torch.cuda.stream(stream if stream is not None else torch.cuda.current_stream(self.device)):
-                self._seg = torch.empty(need.value, dtype=torch.uint8, device=self.device)
-            N.check(self._lib.tessa_hashprune_lend_segment_memory(self._h, self._seg.data_ptr(), need.value),
-                    "hashprune insert segments")
+                self._seg = self._torch_memory(need.value)
+            if self._seg is not None:  # else the library allocates its own
+                N.check(self._lib.tessa_hashprune_lend_segment_memory(self._h, self._seg.data_ptr(), need.value),
+                        "hashprune insert segments")
         N.check(self._lib.tessa_hashprune_insert_segments(self._h, _ptr(records), _ptr(segments), n,
                                                           _stream_ptr(stream)), "hashprune insert segments")
 

@@ -278,13 +278,11 @@ def build_graph_sq8(sq8: T.Sq8Matrix, sketches: torch.Tensor, leader_rows: np.nd
     firsts = pts[fidx].cpu().numpy().view(np.uint32) if pts.numel() else np.zeros(len(osz), np.uint32)
     start = _entry_point_of(osz, firsts)
     torch.cuda.synchronize()
-    # The library allocates its workspaces itself, outside torch's cache: at
-    # most a few GB for the leaf operator and about 16 bytes per replicated row
-    # of a partition run.  Only when that much is not free does torch's cache
-    # go back to the driver (asking for it again cost 1.5 ms a build, and
-    # 0.1-1.4 s when the driver was still clearing it).
-    if torch.cuda.mem_get_info(dev)[0] < (16 << 30) + 32 * max(p.fanout_second, 1) * min(rows * max(p.fanout_top, 1),
-                                                                                    2 * p.roots_rows_per_run):
+    # The library takes its workspaces from the driver, outside torch's cache.
+    # Unless the driver can serve the whole build, the cache goes back to it
+    # first (emptying it for every build cost 1.5 ms a build, and 0.1-1.4 s when
+    # the driver was still clearing the memory).
+    if torch.cuda.mem_get_info(dev)[0] < device_bytes_bound(rows, sq8.padded_dim, osz, p, host_reducer is not None):
         torch.cuda.empty_cache()
     w1 = time.perf_counter()
     sess = S.SubtreeSession(0)
@@ -408,6 +406,31 @@ def build_graph_sq8(sq8: T.Sq8Matrix, sketches: torch.Tensor, leader_rows: np.nd
         stages["largest_task_rows"] = big
         stages["largest_task_workspace_bytes"] = int(plan.required_bytes)
     return BuiltGraph(targets, counts, start, image, w2 - w0, stages)
+
+
+def device_bytes_bound(rows: int, padded_dim: int, sizes: np.ndarray, p: GraphBuildParams, host_reducer: bool) -> int:
+    """An upper bound on the device memory the build takes after D0, from torch
+    and from the library, besides its inputs.  ``sizes``: rows of the D0
+    children."""
+    largest = int(sizes.max()) if len(sizes) else 0
+    total = int(sizes.sum())
+    famp, k = max(p.fanout_second, 1), max(p.leaf_knn, 1)
+    # rows of a partition run, replicated; leaf rows of one leaf top-k and emission batch
+    group = min(total, max(p.roots_rows_per_run, largest)) if p.multi_root else largest
+    batch = min(group * famp, p.leaf_chunk_rows + max(256, p.c_max)) if p.multi_root else group * famp
+    need = 40 * group * famp + 4 * group  # workspace (arenas, nodes, items) and outputs
+    need += 360 * batch + (2 << 30)       # leaf operator: queues, candidate sets, survivor logs
+    # two batches' top-k in flight, one's records, segments and their workspace
+    need += batch * (2 * 8 * k + 32 * k + 100)
+    if not p.multi_root:
+        need += 2 * largest * (padded_dim + 12)  # the child's own rows, here and in the session
+    if not host_reducer:
+        slot = 10 + (24 if p.hashprune_backfill is not None and p.hashprune_backfill.mode != "off" else 0)
+        need += rows * (p.l_max * slot + 16)
+    else:
+        need += 8 << 30  # TierLift's staging and its shards' reservoirs
+    need += rows * (12 * p.l_max + 40)  # tables and image
+    return need + (1 << 30)
 
 
 @dataclass

@@ -863,7 +863,11 @@ tessa_status tessa_robust_prune(const float *data, uint32_t num_points, uint32_t
  * distance evaluations after the start's (may be NULL).  L in [1, 256], K in
  * [1, L] (K > L: the reference's "Set L: .. to a value of at least K: .."),
  * start < num_points < 0xFFFFFFFF, finite data.  Device pointers; enqueued
- * on `stream`; workspace: up to 1 GiB of visited tags. */
+ * on `stream`; workspace: up to 1 GiB of visited bits, shared by the searches
+ * of a GPU: a search waits on the device for the last one, whatever streams
+ * and host threads they come from (a stream's searches have ended before it is
+ * destroyed).  Captured searches, and a search while the last one's stream is
+ * under capture, are the caller's to keep apart. */
 tessa_status tessa_graph_search(const float *data, uint32_t num_points, uint32_t dim, const uint32_t *targets,
                                 const uint32_t *counts, uint32_t row_stride, uint32_t start, const float *queries,
                                 uint32_t num_queries, uint32_t L, uint32_t K, uint32_t *out_ids, float *out_dists,

@@ -117,9 +117,13 @@ struct DeviceWorkspace {
     uint64_t graph_row_off_capacity = 0;
     uint64_t *graph_scalars = nullptr;
     uint64_t graph_scalars_capacity = 0;
-    // greedy search: visited tags, slots x points
-    uint32_t *search_tags = nullptr;
-    uint64_t search_tags_capacity = 0;
+    // greedy search: visited bits, slots x words; the stream of the last search
+    // that used them, and the event that another stream's search waits for
+    uint32_t *search_bits = nullptr;
+    uint64_t search_bits_capacity = 0;
+    hipEvent_t search_done = nullptr;  // null: no search yet
+    hipStream_t search_stream = nullptr;
+    bool search_recorded = false;
     // D0 assignment: leader ranks and their inverse, grouping scratch
     uint32_t *d0_rank = nullptr;
     uint64_t d0_rank_capacity = 0;
@@ -127,6 +131,7 @@ struct DeviceWorkspace {
     uint64_t d0_temp_capacity = 0;
 };
 std::mutex g_ws_mutex;
+std::mutex g_search_mutex;  // a search's host part
 std::vector<DeviceWorkspace> g_ws;
 
 // hipMalloc; a failure leaves no error behind for the next launch's check (the
@@ -2471,11 +2476,33 @@ static tessa_status graph_search_impl(const float *data, const int8_t *codes, co
     DeviceWorkspace *ws = nullptr;
     tessa_status st = device_workspace(&ws);
     if (st.code) return st;
+    // The visited bits are the device's: a search on another stream starts after
+    // the last one has ended.  The event is recorded when another stream comes
+    // (recording it for every search costs 5 us a call), except on the
+    // per-thread stream, whose handle means another stream in another thread.
+    // A captured search is ordered by its graph.
+    std::lock_guard<std::mutex> lock(g_search_mutex);
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    TESSA_HIP_TRY(hipStreamIsCapturing(s, &capture));
+    const bool eager = capture == hipStreamCaptureStatusNone;
     tessa::GraphSearchParams p{};
     p.slots = tessa::search_slots(num_points, num_queries);
-    st = grow(&ws->search_tags, &ws->search_tags_capacity, (uint64_t)p.slots * tessa::search_words(num_points),
+    st = grow(&ws->search_bits, &ws->search_bits_capacity, (uint64_t)p.slots * tessa::search_words(num_points),
               sizeof(uint32_t), "search visited bits");
     if (st.code) return st;
+    if (eager && !ws->search_done) {
+        TESSA_HIP_TRY(hipEventCreateWithFlags(&ws->search_done, hipEventDisableTiming));
+    } else if (eager && (s != ws->search_stream || ws->search_recorded)) {
+        hipStreamCaptureStatus last = hipStreamCaptureStatusNone;
+        if (!ws->search_recorded &&
+            (hipStreamIsCapturing(ws->search_stream, &last) != hipSuccess ||
+             (last == hipStreamCaptureStatusNone && hipEventRecord(ws->search_done, ws->search_stream) != hipSuccess))) {
+            (void)hipGetLastError();  // the last search's stream is gone
+            TESSA_HIP_TRY(hipDeviceSynchronize());
+        } else if (last == hipStreamCaptureStatusNone) {  // an event of a stream under capture would join this one to it
+            TESSA_HIP_TRY(hipStreamWaitEvent(s, ws->search_done, 0));
+        }
+    }
     p.data = data;
     p.codes = codes;
     p.scales = scales;
@@ -2493,8 +2520,13 @@ static tessa_status graph_search_impl(const float *data, const int8_t *codes, co
     p.out_ids = out_ids;
     p.out_dists = out_dists;
     p.out_cmps = out_cmps;
-    p.visited = ws->search_tags;
+    p.visited = ws->search_bits;
     if (tessa::launch_graph_search(p, s) != 0) return make_status(TESSA_ERR_HIP, 0, "graph search launch failed");
+    if (eager) {
+        ws->search_stream = s;
+        ws->search_recorded = s == hipStreamPerThread;
+        if (ws->search_recorded) TESSA_HIP_TRY(hipEventRecord(ws->search_done, s));
+    }
     return ok_status();
 }
 

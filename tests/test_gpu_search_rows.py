@@ -132,3 +132,39 @@ def test_odd_widths_are_read_in_wide_loads(gpu):
     # times what one float per lane and load had taken).
     a, b = (_ms(G.greedy_search, x, t, c, q) for x, q, t, c in (_timed_set(gpu, 20000, d, 64) for d in (129, 132)))
     assert a < 2.0 * b, (a, b)
+
+
+def test_searches_on_several_streams(gpu, orc):
+    # all searches of a GPU share its visited bits: one starts after another has ended, from two host threads too
+    import threading
+
+    rng = np.random.default_rng(12)
+    x = rng.standard_normal((3000, 32)).astype(np.float32)
+    t, c = _graph(rng, 3000, 32)
+    qs = [rng.standard_normal((n, 32)).astype(np.float32) for n in (900, 5, 4500, 300)]
+    want = [orc.greedy_search(x, t, c, 3, q, 24, 6) for q in qs]
+    xd, td, cd = (torch.from_numpy(a).to(gpu) for a in (x, t.view(np.int32), c.view(np.int32)))
+    qd = [torch.from_numpy(q).to(gpu) for q in qs]
+    torch.cuda.synchronize()
+    out = {}
+
+    def work(who):
+        streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+        for i in range(12):
+            j = (i + who) % len(qd)
+            out[who, i] = j, G.greedy_search(xd, td, cd, 3, qd[j], 24, 6, stream=streams[i % 2])
+        for s in streams:
+            s.synchronize()
+
+    threads = [threading.Thread(target=work, args=(w,)) for w in range(2)]
+    for h in threads:
+        h.start()
+    for h in threads:
+        h.join()
+    torch.cuda.synchronize()
+    assert len(out) == 24
+    for j, (ids, d, cmps) in out.values():
+        wi, wd, wc = want[j]
+        assert np.array_equal(ids.cpu().numpy().view(np.uint32), wi)
+        assert np.array_equal(d.cpu().numpy().view(np.uint32), np.asarray(wd).view(np.uint32))
+        assert np.array_equal(cmps.cpu().numpy().view(np.uint32), wc)

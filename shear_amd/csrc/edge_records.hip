@@ -634,17 +634,18 @@ int launch_emit_as(const EdgeParams &p, uint32_t grid, size_t lds, hipStream_t s
     hipLaunchKernelGGL((edge_emit_kernel<kMode, kOrder, kThreads>), dim3(grid), dim3(kThreads), lds, stream, p);
     return 0;
 }
-template <int kMode, int kThreads>
-int launch_emit_mode(const EdgeParams &p, int order, uint32_t grid, size_t lds, hipStream_t stream) {
-    if (order == kOrderReference) return launch_emit_as<kMode, kOrderReference, kThreads>(p, grid, lds, stream);
+template <int kMode>
+int launch_emit_mode(const EdgeParams &p, int order, bool wide, uint32_t grid, size_t lds, hipStream_t stream) {
+    if (order == kOrderReference)
+        return wide ? launch_emit_as<kMode, kOrderReference, kWideThreads>(p, grid, lds, stream)
+                    : launch_emit_as<kMode, kOrderReference, kThreads>(p, grid, lds, stream);
     if (order == kOrderGrouped) return launch_emit_as<kMode, kOrderGrouped, kThreads>(p, grid, lds, stream);
     return launch_emit_as<kMode, kOrderUnique, kThreads>(p, grid, lds, stream);
 }
-template <int kThreads>
-int launch_emit(const EdgeParams &p, int mode, int order, uint32_t grid, size_t lds, hipStream_t stream) {
-    if (mode == kSketchLds) return launch_emit_mode<kSketchLds, kThreads>(p, order, grid, lds, stream);
-    if (mode == kSketchGlobalV4) return launch_emit_mode<kSketchGlobalV4, kThreads>(p, order, grid, lds, stream);
-    return launch_emit_mode<kSketchGlobal, kThreads>(p, order, grid, lds, stream);
+int launch_emit(const EdgeParams &p, int mode, int order, bool wide, uint32_t grid, size_t lds, hipStream_t stream) {
+    if (mode == kSketchLds) return launch_emit_mode<kSketchLds>(p, order, wide, grid, lds, stream);
+    if (mode == kSketchGlobalV4) return launch_emit_mode<kSketchGlobalV4>(p, order, wide, grid, lds, stream);
+    return launch_emit_mode<kSketchGlobal>(p, order, wide, grid, lds, stream);
 }
 }  // namespace
 
@@ -668,11 +669,8 @@ int launch_edge_records(const EdgeParams &p, hipStream_t stream) {
     // of 8 hide its latencies (512 leaves of 2,048 rows, k 32: 433 -> 387 us,
     // 1,600 of 1,300 rows 905 -> 758).  Source-grouped, the scattered reverse
     // records bound it and more waves only spread them wider (844 -> 884 us).
-    if (order == kOrderReference && lds > kEmitLdsBudget / 2) {
-        if (launch_emit<kWideThreads>(p, mode, order, grid, lds, stream)) return -1;
-    } else {
-        if (launch_emit<kThreads>(p, mode, order, grid, lds, stream)) return -1;
-    }
+    const bool wide = order == kOrderReference && lds > kEmitLdsBudget / 2;
+    if (launch_emit(p, mode, order, wide, grid, lds, stream)) return -1;
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

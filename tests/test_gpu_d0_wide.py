@@ -2,8 +2,9 @@
 rows per wave and ranks each leader tile during the next one's products, at the
 edges of its row blocks (256), leader tiles (32) and code widths, against the
 CPU oracle's restatement of the GPU-D0 kernels
-(shear-core/src/algorithm/pipnn/compute_backend.rs:18016-18511); and against
-the kernel of the longer lists where scales and norms are not finite.
+(shear-core/src/algorithm/pipnn/compute_backend.rs:18016-18511); and, where
+scales and norms are not finite, against the distances in f32 sorted on the host
+(NaN behind every number, then by leader id) and the kernel of the longer lists.
 Bar: identical fragments, offsets and grouped points."""
 import numpy as np
 import pytest
@@ -48,3 +49,16 @@ def test_values_that_are_not_finite_rank_as_in_the_longer_lists(gpu, fanout):
     want = D.global_d0_assign(sq, gids, lead, lids, 8)[0]
     got = D.global_d0_assign(sq, gids, lead, lids, fanout)[0]
     assert torch.equal(got, want[:, :fanout])
+    rc, rs, rn, lc, ls, ln = (a.cpu().numpy() for a in (sq.codes, sq.scales, sq.norms, lead.codes, lead.scales,
+                                                        lead.norms))
+    dot = (rc.astype(np.int32) @ lc.astype(np.int32).T).astype(np.float32)
+    with np.errstate(all="ignore"):
+        d = (rn[:, None] + ln[None, :]) - ((np.float32(2) * rs)[:, None] * ls[None, :]) * dot
+    d = np.where(d <= 0, np.float32(0), d)
+    assert np.isnan(d).any() and np.isinf(d).any()
+    order = np.lexsort((np.broadcast_to(lids.cpu().numpy(), d.shape), np.nan_to_num(d, nan=0.0, posinf=np.inf),
+                        np.isnan(d)), axis=1)
+    g = got.cpu().numpy()
+    number = ~np.isnan(np.take_along_axis(d, order[:, :fanout], 1))  # of several NaN the sign decides, not the host's
+    assert np.array_equal(g[number], order[:, :fanout][number])
+    assert np.isnan(np.take_along_axis(d, g.astype(np.int64), 1)[~number]).all()

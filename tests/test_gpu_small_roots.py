@@ -1,7 +1,6 @@
 """Many small subtree roots in one run (tessa_session_partition_small_roots)
-against one tessa_session_run_subtree per root: the same leaves, rows and
-order.  The single-root run is checked against the oracle in
-test_gpu_subtree.py."""
+against the oracle's partition of each root and against one
+tessa_session_run_subtree per root: the same leaves, rows and order."""
 import numpy as np
 import pytest
 import torch
@@ -47,7 +46,7 @@ SIZES = [2, 3, 5, 33, 63, 64, 65, 127, 128, 129, 200, 255, 256, 500, 1000, 1023,
     (2, 2048, [2048, 2047, 1500, 1025], 24, 0.01, 3),  # tight clusters: many attempts
     (2, 1024, [900] * 300, 32, 0.3, 9),                # more roots than CUs
 ])
-def test_leaves_equal_single_root_runs(gpu, fanout, c_max, sizes, dim, sigma, comps):
+def test_leaves_equal_the_oracles_and_single_root_runs(gpu, orc, fanout, c_max, sizes, dim, sigma, comps):
     sq8, rows, offs = _roots(gpu, sizes, dim, len(sizes) + fanout, sigma, comps)
     params = S.PiPNNSubtreeParams(leaf_knn=8, c_max=c_max, fanout_second=fanout, max_leaders=128, max_depth=16)
     sess = S.SubtreeSession(0)
@@ -60,6 +59,7 @@ def test_leaves_equal_single_root_runs(gpu, fanout, c_max, sizes, dim, sigma, co
     got = ro.leaf_rows[: ro.leaf_rows_total].cpu().numpy()
     assert np.array_equal(starts, np.concatenate([[0], np.cumsum(lsz)[:-1]]))
     assert np.all(np.diff(roots) >= 0) and int(lsz.sum()) == ro.leaf_rows_total
+    codes, scales, norms = (a.cpu().numpy() for a in (sq8.codes, sq8.scales, sq8.norms))
     for i in range(min(len(sizes), 24)):
         sub = T.Sq8Matrix(sq8.codes[torch.from_numpy(rows[i]).to(gpu).long()],
                           sq8.scales[torch.from_numpy(rows[i]).to(gpu).long()],
@@ -72,6 +72,11 @@ def test_leaves_equal_single_root_runs(gpu, fanout, c_max, sizes, dim, sigma, co
                 for a, z in zip(one.leaf_starts[: one.leaf_count].tolist(), one.leaf_sizes[: one.leaf_count].tolist())]
         mine = [got[starts[j]:starts[j] + lsz[j]].tolist() for j in np.nonzero(roots == i)[0]]
         assert mine == want, f"root {i} of {sizes[i]} rows"
+        r = rows[i]
+        leaves, _ = orc.subtree_partition(codes[r], scales[r], norms[r], seed=_seed(sizes[i]), root_depth=1,
+                                          max_depth=16, max_leaders=128, fanout_second=fanout, leaf_min=64,
+                                          leaf_max=c_max, small_node_limit=4096)
+        assert mine == [r[leaf].tolist() for leaf in leaves], f"root {i} of {sizes[i]} rows against the oracle"
 
 
 def test_each_kind_of_root_is_refused_by_the_other_entry(gpu):

@@ -359,10 +359,10 @@ __global__ void hp_seg_gather_kernel(const uint4 *segs, const uint32_t *order, u
 // steps at four waves per SIMD): about 300 vector and 470 scalar instructions
 // and 40 LDS operations for a source with 128 records.  Inserting the
 // candidates one by one (a rank ballot, a hash ballot and a shift each) took
-// 88 SIMD cycles a record: 67 M records of 524,288 points, 2.45 ms then and
-// 0.73 ms now; with the groups of a backfill policy, 29 batches of a 1 M x 768
-// build, 13.8 ms then and 4.9 ms now.  Larger tables (fewer candidates try
-// again) or five waves per SIMD (registers spill: 0.89 ms) cost more.
+// 88 SIMD cycles a record: 67 M records of 524,288 points 2.45 ms, by batches
+// 0.73 ms.  Larger tables (fewer candidates try again) or five waves per SIMD
+// (registers spill: 0.89 ms) cost more.  With the groups of a backfill policy
+// the merges of a 1 M x 768 build take 3.5 ms in all.
 constexpr int kHpNew = 4;              // new records per lane in one batch
 constexpr uint32_t kHpBuckets = 1024;  // per wave; >= kHpMaxLMax (staging of the slots), a power of two
 
@@ -1175,11 +1175,11 @@ __global__ __launch_bounds__(kHpThreads) void hp_export_kernel(const uint64_t *s
 // candidates (a target dropped from it had quota + 1 better distinct targets
 // of the hash, whose keys only improve), so batches still merge in any
 // order.  A reservoir that has filled never frees a slot and a full row takes
-// no backups, so groups are kept only while a slot is free; nothing is
-// evicted then either, so those slots are kept unsorted (a candidate is one
-// hash ballot and an append or an in-place update).  The insert that fills
-// the reservoir sorts it in total order, the plain insert takes over, and the
-// groups are neither read nor written again.
+// no backups, so groups are kept only while a slot is free: hp_absorb merges a
+// batch with its groups (quota + 1 rounds of best_of_hash), hp_few_kernel
+// inserts a source's few records one by one.  Once the reservoir is full its
+// slots are kept as without a policy, and the groups are neither read nor
+// written again.  Slots lie in no particular order; the export ranks them.
 
 __device__ __forceinline__ uint64_t shfl_xor64(uint64_t v, int m) {
     const uint32_t lo = __shfl_xor((uint32_t)v, m);

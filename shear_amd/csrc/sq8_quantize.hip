@@ -135,9 +135,10 @@ __global__ __launch_bounds__(kQRows) void sq8_quantize_kernel(const float *x, ui
 // The two need nothing from each other.  The sums are a chain of 2 * dim
 // dependent instructions for however many lanes have a row, so they bound a
 // workgroup of few rows: one wave per 4 rows, sums, maxima and codes in turn,
-// took 1.23 ms for 1,048,576 x 768 (3.3 TB/s), now 0.85 ms (4.7 TB/s, what a copy
-// reaches); at a width that is no multiple of 4 one thread per row, rows read
-// twice and a division per element, 400,003 x 50 took 267 us, now 70.  R is the
+// took 1.23 ms for 1,048,576 x 768 (3.3 TB/s), this split takes 0.73 ms (5.5
+// TB/s); at a width that is no multiple of 4 one thread per row, rows read
+// twice and a division per element, 400,003 x 50 took 267 us, now 60 (39 in the
+// kernel).  R is the
 // largest power of two up to 32 whose rows fit kBlockLds, several workgroups
 // per CU (16 rows of 768 in 49 KB: 0.93 ms; 4 of 960: 320 us, 8: 293; 64 of
 // 128: 260 us, 32: 212), and that leave 1,024 blocks (with few rows a block's

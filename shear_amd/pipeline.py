@@ -538,14 +538,18 @@ def _run_root_group(sess, sq8, gids, pts, offs_h, sizes, group, parent_points, p
         st["leaves"] += l1 - l0
         st["leaf_rows"] += r1 - r0
 
-    pending = None
-    for l0, l1 in chunks:
-        job = launch(l0, l1)
+    try:
+        pending = None
+        for l0, l1 in chunks:
+            job = launch(l0, l1)
+            if pending is not None:
+                finish(pending)
+            pending = job
+            del job
         if pending is not None:
             finish(pending)
-        pending = job
-        del job
-    if pending is not None:
-        finish(pending)
-    main.wait_stream(side)
+    finally:
+        # also after an error: the leaf operator still reads the rows and lists of this run, whose memory the
+        # caller's stream gets back
+        main.wait_stream(side)
 

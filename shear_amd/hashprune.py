@@ -67,7 +67,12 @@ PRODUCTION_BACKFILL = HashPruneBackfill("rhalf-soft-tier-q3", None, 3, 1.02)
 
 
 class HashPruneReducer:
-    """Device-resident HashPrune reservoirs for points [0, num_points)."""
+    """Device-resident HashPrune reservoirs for points [0, num_points).
+
+    Up to MAX_CACHED_BYTES they lie in torch's memory and stay in its cache
+    after ``close`` (torch.cuda.empty_cache() gives them back to the driver);
+    larger ones, and those that torch has no room for, are the library's, and
+    running out of memory is then its TessaError."""
 
     def __init__(self, num_points: int, l_max: int = DEFAULT_L_MAX, device="cuda",
                  backfill: HashPruneBackfill | None = None):
